@@ -195,7 +195,7 @@ struct h264g_ctx {
     int dbk_schedule = H264G_DEBLOCK_BANDS;
     int intra_schedule = H264G_INTRA_BANDS;
     int intra_waves = 8;           // rows per band (waves per workgroup) of the intra band schedule
-    int dbk_waves = 8;             // MB rows per band of the deblocking band schedule (two per wave)
+    int dbk_waves = 8;             // configured MB rows per band of the deblocking band schedule (run: dbk_rows)
     std::vector<hipEvent_t> ev;    // 6 events per profiled run: inter | intra | bS | end (lane), deblock | end
     size_t ev_used = 0;            // events recorded since the last h264g_stage_times
     std::mutex mu;
@@ -210,6 +210,10 @@ extern "C" int32_t h264g_set_error(int32_t code, const char *fmt, ...) {
 }
 
 namespace {
+
+// MB rows per band that the deblocking bands are run with: the configured height, at most
+// H264G_DBK_MAX_ROWS (a wave per luma row, one to a SIMD).
+int dbk_rows(const h264g_ctx *c) { return std::min(c->dbk_waves, H264G_DBK_MAX_ROWS); }
 
 hipStream_t lane_stream(const h264g_ctx *c, int lane) { return lane ? c->aux : c->stream; }
 // The four streams: lane 0, lane 1, their deblocking streams.
@@ -851,7 +855,7 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
             uint32_t *epoch = &ctl[3].ticket;
             switch (ctx->dbk_schedule) {
             case H264G_DEBLOCK_BANDS:
-                e = h264g_launch_deblock_band(q.pics, q.dbands, q.n_dbands, &ctl[1], epoch, ctx->dbk_waves,
+                e = h264g_launch_deblock_band(q.pics, q.dbands, q.n_dbands, &ctl[1], epoch, dbk_rows(ctx),
                                               ctx->d_err, s);
                 break;
             case H264G_DEBLOCK_MB_WAVEFRONT:
@@ -1104,11 +1108,15 @@ int32_t h264g_stream_open(h264g_ctx *c, const h264g_stream_desc *d, uint32_t *id
     auto al = [](uint64_t v) { return (v + 255) & ~(uint64_t)255; };
     s.o_rowprog = al((uint64_t)s.W * s.H * 4);
     s.o_gstrip = al(s.o_rowprog + (uint64_t)s.H * 8);
-    s.o_istrip = s.o_gstrip + (uint64_t)((s.H + c->dbk_waves - 1) / c->dbk_waves) * s.W * 256;
+    s.o_istrip = s.o_gstrip + (uint64_t)((s.H + dbk_rows(c) - 1) / dbk_rows(c)) * s.W * 256;
     s.o_pair = al(s.o_istrip + (uint64_t)((s.H + c->intra_waves - 1) / c->intra_waves) * s.W * 64);
     s.set_bytes = al(s.o_pair + (s.mbaff ? (uint64_t)s.W * s.H / 2 * 4 : 0));
     const size_t dpb_bytes = s.slot_bytes * d->dpb_slots, prog_bytes = s.set_bytes * H264G_MAX_STREAM_PICS;
-    const uint64_t need = dpb_bytes + prog_bytes;
+    // The budget is charged for the strips of bands of the configured height, whatever height
+    // the bands are run with, so that admission does not depend on it.
+    const uint64_t run_bands = (uint64_t)(s.H + dbk_rows(c) - 1) / dbk_rows(c),
+                   cfg_bands = (uint64_t)(s.H + c->dbk_waves - 1) / c->dbk_waves;
+    const uint64_t need = dpb_bytes + prog_bytes - (run_bands - cfg_bands) * s.W * 256 * H264G_MAX_STREAM_PICS;
     if (c->budget && c->used + need > c->budget)
         return h264g_set_error(H264G_E_BUDGET, "DPB budget: %llu + %llu > %llu", (unsigned long long)c->used,
                                (unsigned long long)need, (unsigned long long)c->budget);
@@ -1221,7 +1229,7 @@ int enqueue_picture(h264g_ctx *c, const h264g_pic *p, bool events = true) {
     q.n_rows = p->n_rows;
     q.ibands = q.dbands = q.rows;  // band b of picture 0 is item b
     q.n_ibands = (uint32_t)((p->H + c->intra_waves - 1) / c->intra_waves);
-    q.n_dbands = (uint32_t)((p->H + c->dbk_waves - 1) / c->dbk_waves);
+    q.n_dbands = (uint32_t)((p->H + dbk_rows(c) - 1) / dbk_rows(c));
     q.dbk_off = p->desc.disable_deblocking_filter_idc == 1;
     q.scaled = p->hpic.ls != nullptr;
     if (p->mbaff) {  // items: inter MBs, intra MBs (pair t order), MB pairs (t order)
@@ -1373,7 +1381,7 @@ int build_sub(h264g_ctx *c, const std::vector<const h264g_pic *> &pics, Batch *b
     };
     std::vector<uint32_t> ibands, dbands;
     if (!intra.empty()) bands(c->intra_waves, true, ibands);
-    if (any_dbk) bands(c->dbk_waves, false, dbands);
+    if (any_dbk) bands(dbk_rows(c), false, dbands);
     if (any_dbk && c->dbk_schedule == H264G_DEBLOCK_MB_ROWS) {
         // MB rows of all pictures, row index major: the row above always comes first.
         for (int y = 0; y < maxh; y++)

@@ -1495,14 +1495,11 @@ __device__ __forceinline__ void dbk_line_edge(uint32_t (&w)[5], bool act, bool l
 // the MB and of the left / top MB.
 // cur: tile column of the MB's luma column 0 (16 or 0; chroma cur / 2); the left MB sits
 // in the other half of the tile, so a row's columns -4..-1 are at (16 - cur) + 12.
-// PAIRED: lanes 32-63 do the same for a second MB on a tile of their own (the caller's
-// per-lane wd / bsrec); act: the lane's MB is filtered in this step.
-template <int DIR, bool PAIRED = false>
+template <int DIR>
 __device__ __forceinline__ void dbk_lines(const DevPic &P, uint32_t eq, bool edge, uint32_t qq,
-                                          const uint8_t *bsrec, WaveDbk *wd, const DbkTables *tb, int cur,
-                                          bool act = true) {
-    const int lane = PAIRED ? (wave_lane() & 31) : wave_lane();
-    if (!PAIRED && lane >= 32) return;
+                                          const uint8_t *bsrec, WaveDbk *wd, const DbkTables *tb, int cur) {
+    const int lane = wave_lane();
+    if (lane >= 32) return;
     const int plane = lane < 16 ? 0 : (lane < 24 ? 1 : 2);
     const bool luma = plane == 0;
     const int k = luma ? lane : (lane & 7);
@@ -1531,7 +1528,7 @@ __device__ __forceinline__ void dbk_lines(const DevPic &P, uint32_t eq, bool edg
     const int qav = (qpe + qpq + 1) >> 1;  // internal edges: (qpq + qpq + 1) >> 1 = qpq
     const int iA0 = clip3(0, 51, qav + P.offA), iB0 = clip3(0, 51, qav + P.offB);
     const int iAi = clip3(0, 51, qpq + P.offA), iBi = clip3(0, 51, qpq + P.offB);
-    const bool t8 = dbq_t8(qq), on = act && P.dbk_idc != 1;
+    const bool t8 = dbq_t8(qq), on = P.dbk_idc != 1;
     const int seg = luma ? (k >> 2) : (k >> 1);  // 4-line luma segment of the line
     // bS of this segment's edges 0..3 (k_bs stores them [direction][segment][edge]); chroma
     // edge j lies on luma edge 2j.  All table lookups are issued before the filtering.
@@ -1713,7 +1710,6 @@ __device__ void deblock_row(const DevPic &P, int mby, Sync &sync, WaveDbk *wd, c
 }
 
 // ------------------------------------------------------------ kernels
-constexpr int DBK_WG_MAX_WAVES = 12;  // deblocking bands: up to 24 MB rows
 // The LDS working sets are per wave and the per-MB code synchronises with wave barriers,
 // so a workgroup may hold one wave (most kernels) or several (the band kernels).
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b on XCD b mod 8), each
@@ -2230,263 +2226,543 @@ __global__ __launch_bounds__(WAVE) void k_deblock_rows(const DevPic *__restrict_
     retire(ctl, gridDim.x, epoch_p, epoch);
 }
 
-// ---- deblocking over bands, two MB rows per wave
-// A band of R MB rows runs on ceil(R / 2) waves; wave w takes rows y0 + 2w (the upper
-// half: lanes 0-31) and y0 + 2w + 1 (the lower half: lanes 32-63).  The halves run the
-// per-MB step on 32 lanes each (luma lines on half-lanes 0-15, Cb 16-23, Cr 24-31), each
-// on a tile of its own, the lower half one MB behind the upper: one instruction stream
-// filters two MBs, and every lane of the wave has a line to filter.
+// ---- deblocking over bands: one luma row per wave, its four edges side by side
+// A band of R MB rows runs on two workgroups, whose chains never meet: one filters the luma
+// plane with a wave per MB row, the other Cb and Cr with a wave per two rows.  A wave walks
+// its row from left to right.  Per MB it filters the vertical edges, hands the finished MB
+// to its left down to the next row, takes the rows above its MB over from the previous row
+// and filters the horizontal edges, so a row runs about one step behind the row above it
+// and a picture takes about W + H steps.
 //
-// Row y hands the bottom 4 luma / chroma rows of each MB (the p samples of the next
-// row's top edge) to row y + 1 as a strip: inside a wave from the upper tile to the
-// lower tile, from a wave's lower row to the next wave's upper row through a ring of
-// STRIP_SLOTS LDS slots, and from a band's last row to the next band through a
-// full-width strip array in device memory (G(P.gstrip), one row of W strips per band
-// boundary).  No sample otherwise travels between rows: each sample is written to the
-// picture by exactly one half, row y storing rows 0..12 (chroma 0..4) of its MBs and row
-// y + 1 the rows 13..15 (chroma 5..7) after its top-edge filtering (the picture's last
-// row stores all).  An MB is stored, and its strip handed down, one step after its own
-// filtering, when its right neighbour's left edge has finished its columns 13..15 (the
-// row's last MB one step later as well, with nothing to filter in that step).  A lower
-// row writes strip x into ring slot x mod STRIP_SLOTS only after the next wave's upper
-// row has read strip x - STRIP_SLOTS; every wave of a band is resident, so the reader is
-// always running.
+// Bound: that chain, i.e. the instructions and LDS round trips of one step (about 0.8 us).
+// Lane 16 e + k filters edge e (samples 4 e of the direction) on line k: the edges of a line
+// do not depend on each other but for one sample (edge_pass), so the four run side by side
+// instead of one after the other.  gfx950's transposing LDS read (lds_tr) hands each lane
+// the 8 samples around its edge along a column straight from the rows, so ds_read_b64_tr_b8
+// is the whole change of direction.  What a step needs from device memory was loaded
+// DBK_AHEAD steps before, its thresholds were looked up one step before.  Measured (whole
+// launch, one picture; before: two MB rows per wave, a line's edges in order): 352x288 108 to
+// 38 us (P), 1920x1088 592 to 159 (P) / 196 us (I), 3840x2160 1152 to 309 / 391 us.  Lines
+// kept in registers with the edges in order, four rows per wave, took 330 / 369 us at
+// 1920x1088: instructions bound that step too, 8 edges of ~70 each.
+//
+// Row y hands the bottom 4 rows (chroma: 2) of each MB, the p samples of the next row's top
+// edge, to row y + 1 as a strip, as soon as the right neighbour's left edge has taken its
+// columns: inside a chroma wave through LDS, from wave to wave through a ring of STRIP_SLOTS
+// slots (a slot is written again only once the reader has taken it; every wave of a band is
+// resident, so the reader is always running), from a band to the next through tagged words
+// in device memory (StripWords), which a wave of its own brings into the next band's first
+// ring (strip_reader).  Each sample is written to the picture by one lane: rows 0..12 (chroma
+// 0..6) by their own row after the right neighbour's left edge, the others by the row below
+// after its top edge.
 constexpr int STRIP_SLOTS = 8;
-struct alignas(16) StripSlot {
-    uint32_t w[32];           // strip dword of half-lane j (see strip_word)
+constexpr int DBK_MAX_ROWS = H264G_DBK_MAX_ROWS;  // MB rows of a band, one luma wave each
+constexpr int DBK_AHEAD = 3;
+
+struct alignas(16) LumaTile {
+    uint8_t img[2][16][16];    // MB x in half x & 1: as loaded, then after its vertical edges
+    uint8_t col[16][16];       // its columns after the horizontal edges
+};
+struct alignas(16) ChromaTile {    // one of a wave's two rows; 16-byte lines: Cb in 0..7, Cr in 8..15
+    uint8_t img[2][8][16];
+    uint8_t col[8][16];
+    uint8_t strip[2][16];      // the rows above the MB
+};
+// Tables 8-16 / 8-17 as the edges read them: at[indexA][bS] = alpha' | tC0 << 16 (alpha' 0
+// for bS 0, so that nothing passes the threshold), beta[indexB] = beta' in both halves.
+struct DbkLut {
+    uint32_t at[52][8];
+    uint32_t beta[52];
 };
 struct DbkWgShared {
-    WaveDbk tiles[2 * DBK_WG_MAX_WAVES];               // tile of row y0 + r
-    StripSlot ring[DBK_WG_MAX_WAVES][STRIP_SLOTS];    // wave w's lower row -> wave w + 1's upper row
-    alignas(16) uint8_t bsrec[2 * DBK_WG_MAX_WAVES][32];
-    uint32_t prog[DBK_WG_MAX_WAVES];   // wave w's lower row: strips of MBs 0 .. prog - 1 complete
-    uint32_t cons[DBK_WG_MAX_WAVES];   // wave w's lower row: strips of MBs 0 .. cons - 1 read by wave w + 1
-    DbkTables tb;
+    union {
+        LumaTile l[DBK_MAX_ROWS];
+        ChromaTile c[DBK_MAX_ROWS];
+    };
+    // strips on their way: ring 0 from the band above to wave 0, ring w + 1 from wave w to wave
+    // w + 1 (chroma: 32 bytes of a slot)
+    alignas(16) uint8_t ring[DBK_MAX_ROWS + 1][STRIP_SLOTS][64];
+    uint32_t prog[DBK_MAX_ROWS + 1];   // strips 0 .. prog - 1 are in the ring
+    uint32_t cons[DBK_MAX_ROWS + 1];   // strips 0 .. cons - 1 have been read
+    DbkLut lut;
 };
 
-__device__ __forceinline__ void lds_release() {
-    wave_sync();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+__device__ void dbk_lut_init(DbkLut *t) {
+    for (int i = threadIdx.x; i < 52 * 8; i += blockDim.x) {
+        const int a = i >> 3, bS = i & 7;
+        t->at[a][bS] = bS < 1 || bS > 4 ? 0u : (uint32_t)c_alpha[a] | (bS < 4 ? (uint32_t)c_tc0[bS - 1][a] << 16 : 0u);
+    }
+    for (int i = threadIdx.x; i < 52; i += blockDim.x) t->beta[i] = (uint32_t)c_beta[i] * 0x10001u;
 }
-__device__ void lds_wait(const uint32_t *w, uint32_t need, uint32_t *err) {
-    for (uint32_t it = 0;; ++it) {
-        if (uniform(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) >= need) break;
+
+__device__ __forceinline__ uint32_t lds_peek(const uint32_t *w) {
+    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// Waits until *w >= need; seen: a value of *w read before.
+__device__ __forceinline__ void lds_wait(const uint32_t *w, uint32_t seen, uint32_t need, uint32_t *err) {
+    uint32_t v = uniform(seen);
+#pragma unroll 1
+    for (uint32_t it = 0; v < need; ++it) {
         if (it >= LDS_SPIN_LIMIT) {
             atomicOr(err, DEVERR_TIMEOUT);
             break;
         }
         if ((it & 1023u) == 1023u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) break;
-        __builtin_amdgcn_s_sleep(1);
+        if (it) __builtin_amdgcn_s_sleep(1);
+        v = uniform(lds_peek(w));
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    wave_sync();
 }
+// Publishes the wave's earlier LDS accesses: one wave's LDS instructions take effect in
+// order, so a counter written after them is seen after them, without a wait.
 __device__ __forceinline__ void lds_post(uint32_t *w, uint32_t v) {
-    lds_release();
+    wave_sync();
     __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-__device__ __forceinline__ int half_lane() { return threadIdx.x & 31; }
+// ds_read_b64_tr_b8: in each group of 16 lanes, lanes 2j and 2j + 1 name the two 8-byte
+// halves of row j (j < 8) of an 8 x 16 byte matrix and lane i gets its column i, byte j
+// from row j.  Every lane of the wave takes part.
+__device__ __forceinline__ uint2 lds_tr(const uint8_t *p) {
+    typedef int v2i __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) v2i lds_v2i;
+    const v2i r = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)p);
+    return make_uint2((uint32_t)r.x, (uint32_t)r.y);
+}
 
-// Body of MB (mbx, mby) and its boundary strengths for one half (prefetch registers):
-// half-lane j holds luma row j / 2, bytes 8 (j & 1) .. + 7, the chroma dword j of the
-// two 8x8 planes and, for j < 8, boundary-strength dword j.
-struct DbkPrefetch {
-    uint2 luma;
-    uint32_t chroma, bs;
+// The value of the lane 16 below (row e of 16 lanes gets row e - 1; row 0 anything).
+__device__ __forceinline__ uint32_t row_below(uint32_t v, int e) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 r = __builtin_amdgcn_permlane16_swap(v, v, false, false);      // rows 0 0 2 2 | 1 1 3 3
+    const u32x2 t = __builtin_amdgcn_permlane32_swap(r.y, r.y, false, false);  // rows 1 1 1 1
+    return e == 2 ? t.x : r.x;
+}
+
+// The edges of one direction of a MB on the lanes' samples: a = p3 p2 p1 p0 (bytes 0..3),
+// b = q0 q1 q2 q3 of the lane's line and edge; at: the DbkLut entry of (indexA, bS), beta: of
+// indexB; e: the lane's edge (0: the MB edge).  8.7.2.2 - 8.7.2.4 (Deblock.cpp:1314-1522) on
+// (p, q) pairs: the two sides are mirror images, so one packed 16-bit operation serves both.
+// Conditions are packed sign masks, and the wave skips what no lane needs.
+//
+// Luma edges side by side: with bS < 4 an edge changes p1 p0 q0 q1 and reads p2 .. q2, so the
+// only sample that edge e + 1 sees changed by edge e is its p2 (edge e's q1), and edge e's
+// q1 does not depend on its own p2.  So every lane finds its q1, passes it up as the next
+// edge's p2 and finishes.  bS 4 (s4, the MB edge only) changes up to q2, which edge 1 reads
+// as p1: where a lane needs it, it goes first.  Chroma (LUMA false): p1 .. q1 are read, p0
+// and q0 changed, and edges 8 samples apart in luma are 4 apart: nothing is shared.
+template <bool LUMA>
+__device__ __forceinline__ void edge_pass(uint32_t &a, uint32_t &b, uint32_t at, uint32_t beta, bool s4, int e) {
+    const s16x2 zero = {0, 0}, be = as_pair(beta);
+    if (any_lane(s4)) {
+        const s16x2 t = as_pair(at), al = __builtin_shufflevector(t, t, 0, 0);
+        const s16x2 P0 = as_pair(__builtin_amdgcn_perm(b, a, 0x0c040c03u)), P1 = as_pair(__builtin_amdgcn_perm(b, a, 0x0c050c02u));
+        const s16x2 X0 = pair_swap(P0), X1 = pair_swap(P1);
+        const s16x2 D0 = P0 - X0, A0 = __builtin_elementwise_max(D0, pair_swap(D0));  // |p0 - q0| in both halves
+        const s16x2 T = __builtin_elementwise_max(P1 - P0, P0 - P1) - be;
+        const s16x2 M = __builtin_elementwise_max(__builtin_elementwise_max(T, pair_swap(T)), A0 - al) >> 15;
+        const uint32_t ms = s4 ? as_bits(M) : 0u;
+        const uint32_t W0 = as_bits((P1 + P1 + P0 + X1 + (s16x2){2, 2}) >> 2);        // 2p1 + p0 + q1 + 2
+        uint32_t n0 = (W0 & ms) | (as_bits(P0) & ~ms);
+        if (LUMA) {
+            const s16x2 P2 = as_pair(__builtin_amdgcn_perm(b, a, 0x0c060c01u)), P3 = as_pair(__builtin_amdgcn_perm(b, a, 0x0c070c00u));
+            const s16x2 MA = (__builtin_elementwise_max(P2 - P0, P0 - P2) - be) >> 15;  // ap, aq < beta
+            // strong sides: |p0 - q0| < (alpha >> 2) + 2 as well
+            const uint32_t st = as_bits((A0 - ((al >> 2) + (s16x2){2, 2})) >> 15) & as_bits(MA) & ms;
+            const s16x2 sum = P1 + P0 + X0;
+            const uint32_t S0 = as_bits((sum + sum + P2 + X1 + (s16x2){4, 4}) >> 3);
+            const uint32_t S1 = as_bits((sum + P2 + (s16x2){2, 2}) >> 2);
+            const uint32_t S2 = as_bits((P3 + P3 + P2 * (s16x2){3, 3} + sum + (s16x2){4, 4}) >> 3);
+            n0 = (S0 & st) | (n0 & ~st);
+            const uint32_t n1 = (S1 & st) | (as_bits(P1) & ~st), n2 = (S2 & st) | (as_bits(P2) & ~st);
+            const uint32_t t01 = __builtin_amdgcn_perm(n1, n0, 0x06020400u);                                // np0 np1 nq0 nq1
+            const uint32_t w = __builtin_amdgcn_perm(n2, t01, 0x06040100u);                                 // np0 np1 np2 nq2
+            b = __builtin_amdgcn_perm(b, __builtin_amdgcn_perm(w, t01, 0x0c070302u), 0x07020100u);      // nq0 nq1 nq2 q3
+            a = __builtin_amdgcn_perm(w, a, 0x04050600u);                                                  // p3 np2 np1 np0
+            const uint32_t up = row_below(b, e);
+            a = e == 1 ? up : a;                                                                           // edge 1's p side
+        } else {
+            a = __builtin_amdgcn_perm(n0, a, 0x04020100u);
+            b = __builtin_amdgcn_perm(b, n0, 0x07060502u);
+        }
+    }
+    const s16x2 t = as_pair(s4 ? 0u : at), al = __builtin_shufflevector(t, t, 0, 0), tc0 = __builtin_shufflevector(t, t, 1, 1);
+    const s16x2 P0 = as_pair(__builtin_amdgcn_perm(b, a, 0x0c040c03u)), P1 = as_pair(__builtin_amdgcn_perm(b, a, 0x0c050c02u));
+    const s16x2 D0 = P0 - pair_swap(P0), A0 = __builtin_elementwise_max(D0, pair_swap(D0));
+    const s16x2 T = __builtin_elementwise_max(P1 - P0, P0 - P1) - be;
+    // all three conditions: negative in both halves
+    const s16x2 M = __builtin_elementwise_max(__builtin_elementwise_max(T, pair_swap(T)), A0 - al) >> 15;
+    const uint32_t m = as_bits(M);
+    if (!any_lane(m != 0u)) return;
+    s16x2 tc, N1 = P1;
+    if (LUMA) {
+        s16x2 P2 = as_pair(__builtin_amdgcn_perm(b, a, 0x0c060c01u));
+        // (p0 + q0 + 1) >> 1 in both halves
+        const s16x2 avg = as_pair(__builtin_amdgcn_lerp(as_bits(P0), __builtin_amdgcn_alignbit(as_bits(P0), as_bits(P0), 16), 0x01010101u));
+        const s16x2 ntc0 = zero - tc0, base = avg - (P1 + P1);
+        // p'1 = p1 + Clip3(-tC0, tC0, (p2 + avg - 2 p1) >> 1) where ap < beta, q'1 alike
+        auto side1 = [&](s16x2 &ma) {
+            ma = (__builtin_elementwise_max(P2 - P0, P0 - P2) - be) >> 15;
+            const s16x2 u = pair_clip((P2 + base) >> 1, ntc0, tc0);
+            return P1 + as_pair(as_bits(u) & as_bits(ma) & m);
+        };
+        s16x2 MA;
+        const s16x2 Q1 = side1(MA);
+        const uint32_t up = row_below(as_bits(Q1) >> 16, e);
+        P2 = e ? as_pair((as_bits(P2) & 0xFFFF0000u) | up) : P2;
+        N1 = side1(MA);
+        tc = tc0 - MA - pair_swap(MA);  // tC0 + [ap < beta] + [aq < beta]
+    } else {
+        tc = tc0 + (s16x2){1, 1};
+    }
+    // bS < 4 (8.7.2.3): delta in the low half
+    s16x2 dl = (D0 * (s16x2){-4, -4} + (P1 - pair_swap(P1)) + (s16x2){4, 4}) >> 3;
+    dl = pair_clip(dl, zero - tc, tc);
+    const s16x2 f0 = pair_clip(__builtin_shufflevector(dl, dl, 0, 0) * (s16x2){1, -1} + P0, zero, (s16x2){255, 255});
+    const uint32_t n0 = (as_bits(f0) & m) | (as_bits(P0) & ~m);
+    if (LUMA) {
+        const uint32_t t01 = __builtin_amdgcn_perm(as_bits(N1), n0, 0x06020400u);  // np0 np1 nq0 nq1
+        const uint32_t p2 = a;
+        a = __builtin_amdgcn_perm(t01, p2, 0x04050100u);                  // p3 p2 np1 np0
+        b = __builtin_amdgcn_perm(b, t01, 0x07060302u);                   // nq0 nq1 q2 q3
+    } else {
+        a = __builtin_amdgcn_perm(n0, a, 0x04020100u);                    // p3 p2 p1 np0
+        b = __builtin_amdgcn_perm(b, n0, 0x07060502u);                    // nq0 q1 q2 q3
+    }
+}
+
+// One lane's edge in one direction: its DbkLut entries and whether its bS is 4.
+struct DbkThr {
+    uint32_t at, beta;
+    bool s4;
 };
-__device__ __forceinline__ DbkPrefetch dbk_fetch(const DevPic &P, const DbkPlanes &d, int mbx, int mby, bool on) {
-    const int hl = half_lane();
-    DbkPrefetch f{make_uint2(0u, 0u), 0u, 0u};
-    if (on) {
-        f.luma = *(const uint2 *)&d.y[(uint64_t)(mby * 16 + (hl >> 1)) * d.wl + mbx * 16 + (hl & 1) * 8];
-        const uint8_t *pl = (hl >> 4) ? d.cr : d.cb;
-        f.chroma = *(const uint32_t *)&pl[(uint64_t)(mby * 8 + ((hl >> 1) & 7)) * d.wc + mbx * 8 + (hl & 1) * 4];
-        if (hl < 8) f.bs = *(const uint32_t *)&G(P.bs)[(size_t)(mby * P.W + mbx) * 32 + hl * 4];
-    }
-    return f;
-}
-__device__ __forceinline__ void dbk_place(const DbkPrefetch &f, WaveDbk *wd, uint8_t *bsrec, int cur) {
-    const int hl = half_lane();
-    *(uint2 *)&wd->L[(hl >> 1) + 4][cur + (hl & 1) * 8] = f.luma;
-    *(uint32_t *)&wd->C[hl >> 4][((hl >> 1) & 7) + 4][(cur >> 1) + (hl & 1) * 4] = f.chroma;
-    if (hl < 8) *(uint32_t *)&bsrec[hl * 4] = f.bs;
-}
-
-// Rows 0 .. ry (chroma 0 .. cy) of the MB whose column 0 sits at tile column `col` to the
-// picture: one aligned 16-byte luma row per half-lane 0..15, one 8-byte chroma row per
-// half-lane 16..31.
-__device__ __forceinline__ void dbk_store_mb(const DbkPlanes &d, int mbx, int mby, int col, int ry, int cy,
-                                             const WaveDbk *wd) {
-    const int hl = half_lane();
-    if (hl < 16) {
-        if (hl <= ry)
-            *(uint4 *)&d.y[(uint64_t)(mby * 16 + hl) * d.wl + mbx * 16] = *(const uint4 *)&wd->L[hl + 4][col];
-    } else {
-        const int k = hl - 16, c = k >> 3, r = k & 7;
-        if (r <= cy)
-            *(uint2 *)&(c ? d.cr : d.cb)[(uint64_t)(mby * 8 + r) * d.wc + mbx * 8] = *(const uint2 *)&wd->C[c][r + 4][col >> 1];
-    }
-}
-// Rows 13..15 (chroma 5..7) of the MB above the current one (tile column cur), final after
-// the current MB's top edge: half-lanes 0..2 luma, 3..8 chroma.
-__device__ __forceinline__ void dbk_store_top(const DbkPlanes &d, int mbx, int mby, const WaveDbk *wd, int cur) {
-    const int hl = half_lane();
-    if (hl < 3) {
-        *(uint4 *)&d.y[(uint64_t)(mby * 16 - 3 + hl) * d.wl + mbx * 16] = *(const uint4 *)&wd->L[hl + 1][cur];
-    } else if (hl < 9) {
-        const int k = hl - 3, c = k >= 3, r = k - 3 * c;
-        *(uint2 *)&(c ? d.cr : d.cb)[(uint64_t)(mby * 8 - 3 + r) * d.wc + mbx * 8] = *(const uint2 *)&wd->C[c][r + 1][cur >> 1];
-    }
-}
-
-// A strip is one dword per half-lane: luma row 12 + j / 4, bytes 4 (j & 3) .. + 3 for
-// j < 16; for j = 16 + k the chroma plane k / 8, row 4 + (k / 2) % 4, bytes 4 (k & 1) .. + 3.
-// Strip dword of the MB at tile column `col` (rows 12..15 / chroma 4..7).
-__device__ __forceinline__ uint32_t strip_word(const WaveDbk *wd, int col) {
-    const int hl = half_lane();
-    if (hl < 16) return *(const uint32_t *)&wd->L[16 + (hl >> 2)][col + (hl & 3) * 4];
-    const int k = hl - 16, c = k >> 3, r = (k >> 1) & 3, h = k & 1;
-    return *(const uint32_t *)&wd->C[c][8 + r][(col >> 1) + h * 4];
-}
-// A strip dword into the tile rows -4..-1 above the MB at tile column cur.
-__device__ __forceinline__ void strip_place(WaveDbk *wd, int cur, uint32_t v) {
-    const int hl = half_lane();
-    if (hl < 16) {
-        *(uint32_t *)&wd->L[hl >> 2][cur + (hl & 3) * 4] = v;
-    } else {
-        const int k = hl - 16, c = k >> 3, r = (k >> 1) & 3, h = k & 1;
-        *(uint32_t *)&wd->C[c][r][(cur >> 1) + h * 4] = v;
-    }
+// mb: the edge is the MB edge to a MB with deblocking word nb (own: or to the MB's own values).
+__device__ __forceinline__ DbkThr dbk_threshold(const DbkLut *lut, uint32_t bS, int plane, uint32_t q, uint32_t nb, bool own,
+                                                bool mb, int offA, int offB) {
+    const int qq = dbq_qp(q, plane), qn = own || !mb ? qq : dbq_qp(nb, plane), qav = (qq + qn + 1) >> 1;
+    DbkThr t;
+    t.at = lut->at[clip3(0, 51, qav + offA)][bS & 7u];
+    t.beta = lut->beta[clip3(0, 51, qav + offB)];
+    t.s4 = bS == 4u;
+    return t;
 }
 
 // Strips that cross from a band to the next (another workgroup, possibly another XCD) go
-// through device memory as 32 words of 64 bits: the strip dword of half-lane j in the low
-// half of word j, the launch epoch in the high half.  Each word is stored and loaded as
-// one agent-scope atomic, so a reader that finds the epoch in all 32 words holds the
-// whole strip; neither side needs a fence, whose L2 write-back / invalidation would also
-// hit every other kernel running on those XCDs.
+// through device memory as words of 64 bits: a strip dword in the low half, the launch
+// epoch in the high half (luma dwords 0..15, chroma 16..23).  Each word is stored and
+// loaded as one agent-scope atomic, so a reader that finds the epoch in a word holds its
+// samples; neither side needs a fence, whose L2 write-back / invalidation would also hit
+// every other kernel running on those XCDs.
 struct StripWords {
     uint64_t w[32];
 };
-__device__ __forceinline__ void strip_put_g(StripWords *sw, const WaveDbk *wd, int col, uint32_t epoch) {
-    const uint32_t v = strip_word(wd, col);
-    __hip_atomic_store(&sw->w[half_lane()], (uint64_t)epoch << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Waits (the whole wave) for the strip of this launch and puts it into the tile of the
-// lanes where `mine` holds, above the MB at tile column cur.  Bounded like the other waits.
-__device__ void strip_get_g(const StripWords *sw, WaveDbk *wd, int cur, uint32_t epoch, bool mine, uint32_t *err) {
-    uint64_t v = (uint64_t)epoch << 32;
-    for (uint32_t it = 0;; ++it) {
-        if (mine) v = __hip_atomic_load(&sw->w[half_lane()], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (!any_lane((uint32_t)(v >> 32) != epoch)) break;
-        if (it >= SPIN_LIMIT) {
-            atomicOr(err, DEVERR_TIMEOUT);
-            break;
-        }
-        if ((it & 255u) == 255u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) break;
-        __builtin_amdgcn_s_sleep(1);
-    }
-    if (mine) strip_place(wd, cur, (uint32_t)v);
-}
-
-// Wave w of the band of rows y0 .. y1 - 1 (band index b): rows y0 + 2w and, when it lies
-// in the band, y0 + 2w + 1.  Step s filters the upper row's MB s and the lower row's MB
-// s - 1, then stores (and hands down) the MBs one to the left of those.
-__device__ void deblock_pair_band(const DevPic &P, int w, int y0, int y1, int b, DbkWgShared &sh, uint32_t epoch,
-                                  uint32_t *err) {
-    const int W = P.W, H = P.H;
-    const int yu = y0 + 2 * w, yl = yu + 1;
-    const bool hasL = yl < y1, lower = wave_lane() >= 32;
-    const int y = lower ? yl : yu;
-    const DbkPlanes d = dbk_planes(P);
-    WaveDbk *const tu = &sh.tiles[2 * w], *const tl = &sh.tiles[2 * w + 1];
-    WaveDbk *const wd = lower ? tl : tu;
-    uint8_t *const bsrec = sh.bsrec[2 * w + (lower ? 1 : 0)];
-    const bool last = y == H - 1, topU = yu > 0, top = lower || topU;
-    const int ry = last ? 15 : 12, cy = last ? 7 : 4;  // rows a half stores of its own MBs
-    // the band's last row hands its strips to the next band (none after the picture's last)
-    const bool gU = !hasL && yu == y1 - 1 && yu != H - 1, gL = hasL && yl == y1 - 1 && yl != H - 1;
-    const bool ringL = hasL && yl + 1 < y1;  // the lower row hands down to wave w + 1
-    const bool from_g = topU && w == 0;      // the upper row reads the band above's strips
-    StripSlot *const ring = sh.ring[w];
-    const StripSlot *const above = w > 0 ? sh.ring[w - 1] : nullptr;
-    StripWords *const gout = (StripWords *)G(P.gstrip) + (size_t)b * W;              // this band -> next
-    const StripWords *const gin = (const StripWords *)G(P.gstrip) + (size_t)(b - 1) * W;  // previous band -> this
-    const int steps = W + (hasL ? 1 : 0);  // the lower row's last MB is stored in step W + 1
-    DbkPrefetch f = dbk_fetch(P, d, 0, yu, !lower);
-    // deblocking words of each half's MB and of the MB above it, one step ahead like the samples
-    uint32_t qq = 0u, qn = lower ? 0u : G(P.dbq)[yu * W], tn = (!lower && topU) ? G(P.dbq)[(yu - 1) * W] : 0u;
-    for (int s = 0; s <= steps; s++) {
-        const int x = lower ? s - 1 : s;  // this half's MB
-        const bool act = lower ? (hasL && s >= 1 && s <= W) : s < W;
-        const int cur = 16 * (x & 1), prev = 16 - cur;  // tile columns of MB x and MB x - 1
-        const int prevU = 16 - 16 * (s & 1);              // the upper row's MB s - 1 (= the lower's MB column)
-        const uint32_t lq = qq, tq = tn;
-        qq = qn;
-        if (act) dbk_place(f, wd, bsrec, cur);
-        {  // next step's MBs, in flight during this one
-            const bool nU = s + 1 < W, nL = hasL && s < W;
-            f = dbk_fetch(P, d, lower ? s : s + 1, y, lower ? nL : nU);
-            const uint32_t qu = nU ? G(P.dbq)[yu * W + s + 1] : 0u, ql = nL ? G(P.dbq)[yl * W + s] : 0u;
-            const uint32_t tu_ = nU && topU ? G(P.dbq)[(yu - 1) * W + s + 1] : 0u, tl_ = nL ? G(P.dbq)[yu * W + s] : 0u;
-            qn = lower ? ql : qu;
-            tn = lower ? tl_ : tu_;
-        }
-        wave_sync();
-        dbk_lines<0, true>(P, lq, x > 0, qq, bsrec, wd, &sh.tb, cur, act);  // vertical edges
-        wave_sync();
-        // MB x - 1 is final now (its columns 13..15 took MB x's left edge) except rows 13..15,
-        // which the next row's top edge filters: store it and hand its strip down before
-        // waiting for the row above, so the row below runs about one step behind
-        const bool pU = s >= 1 && s <= W, pL = hasL && s >= 2;
-        if (lower ? pL : pU) dbk_store_mb(d, x - 1, y, prev, ry, cy, wd);
-        if (hasL && pU && lower) strip_place(tl, prevU, strip_word(tu, prevU));  // upper -> lower
-        if (gU && pU && !lower) strip_put_g(&gout[s - 1], tu, prevU, epoch);
-        if (gL && pL && lower) strip_put_g(&gout[s - 2], tl, prev, epoch);
-        if (ringL && pL) {
-            const int m = s - 2;
-            if (m - STRIP_SLOTS >= 0) lds_wait(&sh.cons[w], (uint32_t)(m - STRIP_SLOTS + 1), err);  // slot read?
-            if (lower) {
-                StripSlot *sl = &ring[m % STRIP_SLOTS];
-                sl->w[half_lane()] = strip_word(tl, prev);
+// The reader wave of a band: strips (N words from word AT) of the row `sw` into ring 0, as
+// many at a time as the wave has lanes for; the rows then find every strip in LDS, whatever
+// the band above lags, and one poll's round trip serves several of them.
+template <int N, int AT>
+__device__ __forceinline__ void strip_reader(const GAS StripWords *sw, int W, DbkWgShared &sh, uint32_t epoch, uint32_t *err) {
+    constexpr int AT_ONCE = WAVE / N;
+    static_assert(AT_ONCE <= STRIP_SLOTS, "a round of strips fits the ring");
+    const int lane = wave_lane(), mine = lane / N, word = lane % N;
+    for (int x0 = 0; x0 < W; x0 += AT_ONCE) {
+        const int n = min(AT_ONCE, W - x0);
+        int have = 0;  // strips x0 .. x0 + have - 1 are in the ring
+#pragma unroll 1
+        for (uint32_t it = 0; have < n; ++it) {
+            const uint64_t r = __hip_atomic_load(&sw[x0 + min(mine, n - 1)].w[AT + word], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // the lanes whose words have arrived, up to the first strip that has not
+            const uint64_t missing = __builtin_amdgcn_ballot_w64((uint32_t)(r >> 32) != epoch);
+            const int got = missing ? min(n, (int)(__builtin_ctzll(missing) / N)) : n;
+            if (got > have) {
+                const int x = x0 + got - 1;
+                if (x >= STRIP_SLOTS) lds_wait(&sh.cons[0], 0u, (uint32_t)(x - STRIP_SLOTS + 1), err);  // slots read?
+                if (mine >= have && mine < got) *(uint32_t *)&sh.ring[0][(x0 + mine) % STRIP_SLOTS][4 * word] = (uint32_t)r;
+                lds_post(&sh.prog[0], (uint32_t)x + 1);
+                have = got;
+                continue;
             }
-            lds_post(&sh.prog[w], (uint32_t)m + 1);
-        }
-        if (topU && s < W) {  // the upper row's strip from the row above
-            if (from_g) {
-                strip_get_g(&gin[s], tu, 16 * (s & 1), epoch, !lower, err);
-            } else {
-                lds_wait(&sh.prog[w - 1], (uint32_t)s + 1, err);
-                if (!lower) strip_place(tu, 16 * (s & 1), above[s % STRIP_SLOTS].w[half_lane()]);
-                lds_post(&sh.cons[w - 1], (uint32_t)s + 1);
+            if (it >= SPIN_LIMIT) {
+                atomicOr(err, DEVERR_TIMEOUT);
+                return;
             }
+            if ((it & 255u) == 255u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) return;
+            __builtin_amdgcn_s_sleep(1);
         }
-        wave_sync();
-        dbk_lines<1, true>(P, tq, top, qq, bsrec, wd, &sh.tb, cur, act);  // horizontal edges
-        wave_sync();
-        if (act && top) dbk_store_top(d, x, y, wd, cur);
-        // the next step's tile writes (the other half of the tile) follow this barrier
-        wave_sync();
     }
 }
 
-// One workgroup per band of `rows` MB rows (rows y0 + 2w, y0 + 2w + 1 on wave w).
-__global__ __launch_bounds__(WAVE * DBK_WG_MAX_WAVES) void k_deblock_band(const DevPic *__restrict__ pics,
-                                                                          const uint32_t *__restrict__ items, uint32_t n,
-                                                                          int rows, DevCtl *ctl, uint32_t *epoch_p,
-                                                                          uint32_t *err) {
+// MB row y = y0 + w of the band of rows y0 .. y1 - 1 (band index b): the luma plane.
+__device__ __forceinline__ void deblock_luma_row(const DevPic &P, int w, int y0, int y1, int b, DbkWgShared &sh, uint32_t epoch,
+                                                 uint32_t *err) {
+    const int W = P.W, H = P.H, y = y0 + w;
+    const int lane = wave_lane(), e = lane >> 4, k = lane & 15;
+    const bool top = y > 0, last = y == H - 1;
+    const bool ring_out = y + 1 < y1, g_out = !ring_out && !last;
+    LumaTile *const tile = &sh.l[w];
+    GAS StripWords *const gout = (GAS StripWords *)G(P.gstrip) + (size_t)b * W;
+    gu8 *const slot = slot_base(P, P.dst);
+    const uint32_t pitch = (uint32_t)W * 16u, row0 = (uint32_t)(y * 16) * pitch;
+    // as loaded: lane 4 r + d takes dword d of row r; as stored: lanes 0-15 bytes 8..15 of row
+    // k, lanes 16-31 bytes 0..7
+    const uint32_t ld = row0 + (uint32_t)(lane >> 2) * pitch + (uint32_t)(lane & 3) * 4u;
+    const uint32_t so = row0 + (uint32_t)k * pitch + (e == 0 ? 8u : 0u);
+    const gu8 *const bsv = G(P.bs) + (uint32_t)((k >> 2) * 4 + e);
+    const gu8 *const dq = (const gu8 *)G(P.dbq);
+    const uint32_t mb0 = (uint32_t)(y * W), mbt = top ? (uint32_t)W * 4u : 0u;
+    const int offA = P.offA, offB = P.offB;
+    struct Ahead {
+        uint32_t px, bv, bh, q, qt;
+    };
+    // (no branches, so that the loads stay in flight: past the row's end they read its last MB)
+    auto fetch = [&](int x) {
+        const uint32_t xc = (uint32_t)min(x, W - 1), a = mb0 + xc;
+        Ahead f;
+        f.px = *(const GAS uint32_t *)(slot + (ld + xc * 16u));
+        f.bv = bsv[a * 32u];
+        f.bh = bsv[a * 32u + 16u];
+        f.q = *(const GAS uint32_t *)(dq + a * 4u);
+        f.qt = *(const GAS uint32_t *)(dq + (a * 4u - mbt));
+        return f;
+    };
+    // LDS addresses: the transposing reads (lane 2j + h of a group names half h of line j)
+    const int tj = k >> 1, th = (k & 1) * 8, tr = 4 * (e - 1) + tj;      // row tr around edge e
+    const bool tr_strip = tr < 0;
+    const uint8_t *const tr_c = &tile->col[(e == 0 ? 8 : 0) + tj][th];  // columns 8..15 for lanes 0-15, else 0..7
+    const int sr = k - 12;                                               // the lane's strip row, from row 12 on
+    Ahead f[DBK_AHEAD] = {fetch(0), fetch(1), fetch(2)};
+    ((uint32_t *)tile->img[0])[lane] = f[0].px;
+    wave_sync();
+    uint32_t bq = *(const uint32_t *)&tile->img[0][k][4 * e], ap = *(const uint32_t *)&tile->img[0][k][4 * max(e - 1, 0)];
+    DbkThr thv = dbk_threshold(&sh.lut, f[0].bv, 0, f[0].q, 0u, false, e == 0, offA, offB);
+    DbkThr thh = dbk_threshold(&sh.lut, f[0].bh, 0, f[0].q, f[0].qt, f[0].q & DBQ_OWN_TOP, e == 0, offA, offB);
+    uint2 prev = make_uint2(0u, 0u);   // MB x - 1 after its horizontal edges: row k, bytes 8..15 (lanes 0-15) or 0..7
+    // MB m = x - 1 once MB x has taken its left edge (seen: sh.cons of the row's ring, read
+    // before): final but for rows 13..15, so its strip is handed down and it is stored
+    auto finish = [&](int m, uint32_t seen) {
+        if (ring_out) {
+            if (m >= STRIP_SLOTS) lds_wait(&sh.cons[w + 1], seen, (uint32_t)(m - STRIP_SLOTS + 1), err);  // slot read?
+            if (lane < 32 && sr >= 0) *(uint2 *)&sh.ring[w + 1][m % STRIP_SLOTS][sr * 16 + (e == 0 ? 8 : 0)] = prev;
+            lds_post(&sh.prog[w + 1], (uint32_t)m + 1);
+        } else if (g_out && lane < 32 && sr >= 0) {
+            GAS uint64_t *const d = &gout[m].w[sr * 4 + (e == 0 ? 2 : 0)];
+            __hip_atomic_store(&d[0], (uint64_t)epoch << 32 | prev.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&d[1], (uint64_t)epoch << 32 | prev.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (lane < 32 && (sr < 1 || last)) *(GAS uint2 *)(slot + (so + (uint32_t)m * 16u)) = prev;
+    };
+    // MB x; cur: its register set, refilled for MB x + DBK_AHEAD; nxt: that of MB x + 1
+    auto step = [&](int x, Ahead &cur, Ahead &nxt) {
+        const uint32_t q0 = cur.q;
+        cur = fetch(x + DBK_AHEAD);
+        uint8_t *const img = &tile->img[x & 1][0][0], *const nimg = &tile->img[(x + 1) & 1][0][0];
+        ((uint32_t *)nimg)[lane] = nxt.px;
+        const uint32_t seen = lds_peek(&sh.prog[w]), seen_c = lds_peek(&sh.cons[w + 1]);
+        // ---- vertical edges: a is row k's dword before the edge, b the one after it
+        {
+            uint32_t a = e ? ap : prev.y, bb = bq;
+            edge_pass<true>(a, bb, thv.at, thv.beta, thv.s4, e);
+            *(uint32_t *)&img[k * 16 + 4 * e] = bb;
+            wave_sync();  // (the next edge's p side lies in the dword just written)
+            if (e) *(uint16_t *)&img[k * 16 + 4 * e - 2] = (uint16_t)(a >> 16);
+            else prev.y = a;
+        }
+        if (x > 0 && x <= W) finish(x - 1, seen_c);
+        // ---- the rows above the MB
+        if (top && x < W) lds_wait(&sh.prog[w], seen, (uint32_t)x + 1, err);
+        const uint8_t *const strip = sh.ring[w][x % STRIP_SLOTS];
+        wave_sync();
+        // ---- horizontal edges: a and b are rows 4 e - 4 .. 4 e + 3 of column k
+        const uint2 c = lds_tr(tr_strip ? strip + (tr + 4) * 16 + th : img + tr * 16 + th);
+        bq = *(const uint32_t *)&nimg[k * 16 + 4 * e];
+        ap = *(const uint32_t *)&nimg[k * 16 + 4 * max(e - 1, 0)];
+        // the next step's thresholds (opaque words: the compiler would narrow them as they
+        // arrive and wait for their loads steps ahead of this use)
+        asm volatile("" : "+v"(nxt.q), "+v"(nxt.qt), "+v"(nxt.bv), "+v"(nxt.bh));
+        const DbkThr nv = dbk_threshold(&sh.lut, x + 1 < W ? nxt.bv : 0u, 0, nxt.q, q0, nxt.q & DBQ_OWN_LEFT, e == 0, offA, offB);
+        const DbkThr nh = dbk_threshold(&sh.lut, nxt.bh, 0, nxt.q, nxt.qt, nxt.q & DBQ_OWN_TOP, e == 0, offA, offB);
+        lds_post(&sh.cons[w], (uint32_t)x + 1);
+        uint32_t a = c.x, bb = c.y;
+        edge_pass<true>(a, bb, thh.at, thh.beta, thh.s4, e);
+        *(uint32_t *)&tile->col[k][4 * e] = bb;
+        wave_sync();
+        if (e) {
+            *(uint16_t *)&tile->col[k][4 * e - 2] = (uint16_t)(a >> 16);
+        } else if (top && x < W) {  // the rows of the MB above that its top edge changes: column k's bytes
+            const uint32_t o = row0 - pitch + (uint32_t)(x * 16 + k);
+            slot[o] = (uint8_t)(a >> 24);
+            slot[o - pitch] = (uint8_t)(a >> 16);
+            slot[o - 2u * pitch] = (uint8_t)(a >> 8);
+        }
+        wave_sync();
+        prev = lds_tr(tr_c);
+        thv = nv;
+        thh = nh;
+    };
+    // Unrolled over the DBK_AHEAD register sets (moving a set would wait for its loads); steps
+    // past the row's end filter nothing (an exit between the steps would make the compiler
+    // wait for all stores at the loop's head).
+    for (int x = 0; x < W; x += DBK_AHEAD) {
+        step(x, f[0], f[1]);
+        step(x + 1, f[1], f[2]);
+        step(x + 2, f[2], f[0]);
+    }
+    if (W % DBK_AHEAD == 0) finish(W - 1, 0u);
+}
+
+// MB rows y0 + 2 w and y0 + 2 w + 1 (lanes 32-63, one MB behind) of the band of rows
+// y0 .. y1 - 1 (band index b): the chroma planes.  Lane 16 e + 8 p + k of a row's 32: edge e
+// of line k of plane p.
+__device__ __forceinline__ void deblock_chroma_rows(const DevPic &P, int w, int y0, int y1, int b, DbkWgShared &sh, uint32_t epoch,
+                                                    uint32_t *err) {
+    const int W = P.W, H = P.H, yw = y0 + 2 * w;
+    const bool two = yw + 1 < y1;
+    const int lane = wave_lane(), g = lane >> 5, e = (lane >> 4) & 1, pk = lane & 15, p = pk >> 3, k = pk & 7;
+    const bool rowok = g == 0 || two;
+    const int y = yw + (two ? g : 0), gl = two ? 1 : 0, yl = yw + gl;  // (an absent second row reads the first's)
+    const bool top = y > 0, last = y == H - 1;
+    const bool ring_out = yl + 1 < y1, g_out = !ring_out && yl < H - 1;
+    ChromaTile *const tile = &sh.c[2 * w + g];
+    uint8_t *const strip_dn = &sh.c[2 * w + 1].strip[0][0];
+    GAS StripWords *const gout = (GAS StripWords *)G(P.gstrip) + (size_t)b * W;
+    gu8 *const slot = slot_base(P, P.dst);
+    const uint32_t pitch = (uint32_t)W * 8u, np = (uint32_t)(W * H), row0 = (uint32_t)(y * 8) * pitch;
+    // as loaded: lane 16 p + 2 r + d of the row takes dword d of row r of plane p
+    const int lp = (lane >> 4) & 1, lr = (lane >> 1) & 7, ldw = lane & 1;
+    const uint32_t ld = np * (lp ? 320u : 256u) + row0 + (uint32_t)lr * pitch + (uint32_t)ldw * 4u;
+    const uint32_t pl = np * (p ? 320u : 256u) + row0, so = pl + (uint32_t)k * pitch;
+    const gu8 *const bsv = G(P.bs) + (uint32_t)((k >> 1) * 4 + 2 * e);  // chroma edge e lies on luma edge 2 e
+    const gu8 *const dq = (const gu8 *)G(P.dbq);
+    const uint32_t mb0 = (uint32_t)(y * W), mbt = top ? (uint32_t)W * 4u : 0u;
+    const int offA = P.offA, offB = P.offB;
+    struct Ahead {
+        uint32_t px, bv, bh, q, qt;
+    };
+    auto fetch = [&](int x) {
+        const uint32_t xc = (uint32_t)clip3(0, W - 1, x), a = mb0 + xc;
+        Ahead f;
+        f.px = *(const GAS uint32_t *)(slot + (ld + xc * 8u));
+        f.bv = bsv[a * 32u];
+        f.bh = bsv[a * 32u + 16u];
+        f.q = *(const GAS uint32_t *)(dq + a * 4u);
+        f.qt = *(const GAS uint32_t *)(dq + (a * 4u - mbt));
+        return f;
+    };
+    const int tj = pk >> 1, th = (pk & 1) * 8, tr = 4 * (e - 1) + tj;
+    const bool tr_strip = tr < 0;
+    const uint8_t *const tr_c = &tile->col[tj][th];
+    const int sr = k - 6;
+    auto active = [&](int x) { return rowok && (uint32_t)x < (uint32_t)W; };
+    Ahead f[DBK_AHEAD] = {fetch(-g), fetch(1 - g), fetch(2 - g)};
+    auto place = [&](int x, uint32_t v) {  // MB x as loaded, into its half of the tile
+        *(uint32_t *)&tile->img[x & 1][lr][lp * 8 + ldw * 4] = v;
+    };
+    place(-g, f[0].px);
+    wave_sync();
+    uint32_t bq = *(const uint32_t *)&tile->img[g & 1][k][p * 8 + 4 * e], ap = *(const uint32_t *)&tile->img[g & 1][k][p * 8];
+    DbkThr thv = dbk_threshold(&sh.lut, active(-g) ? f[0].bv : 0u, 1 + p, f[0].q, 0u, false, e == 0, offA, offB);
+    DbkThr thh = dbk_threshold(&sh.lut, active(-g) ? f[0].bh : 0u, 1 + p, f[0].q, f[0].qt, f[0].q & DBQ_OWN_TOP, e == 0, offA, offB);
+    uint2 prev = make_uint2(0u, 0u);   // MB x - 1 after its horizontal edges: row k of plane p
+    // After the vertical edges of step s: MB x - 1 is final but for row 7, so its strip is handed
+    // down and it is stored (m: the MB of the wave's last row; seen: sh.cons of its ring)
+    auto finish = [&](int s, uint32_t seen) {
+        const int x = s - g, m = s - gl - 1;
+        const bool had = rowok && x >= 1 && x <= W;
+        if (had && e == 0 && sr >= 0 && g < gl) *(uint2 *)(strip_dn + sr * 16 + p * 8) = prev;
+        if (m >= 0 && m < W) {
+            if (ring_out) {
+                if (m >= STRIP_SLOTS) lds_wait(&sh.cons[w + 1], seen, (uint32_t)(m - STRIP_SLOTS + 1), err);  // slot read?
+                if (g == gl && e == 0 && sr >= 0) *(uint2 *)&sh.ring[w + 1][m % STRIP_SLOTS][sr * 16 + p * 8] = prev;
+                lds_post(&sh.prog[w + 1], (uint32_t)m + 1);
+            } else if (g_out && g == gl && e == 0 && sr >= 0) {
+                GAS uint64_t *const d = &gout[m].w[16 + sr * 4 + p * 2];
+                __hip_atomic_store(&d[0], (uint64_t)epoch << 32 | prev.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(&d[1], (uint64_t)epoch << 32 | prev.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if (had && e == 0 && (sr < 1 || last)) *(GAS uint2 *)(slot + (so + (uint32_t)(x - 1) * 8u)) = prev;
+    };
+    auto step = [&](int s, Ahead &cur, Ahead &nxt) {
+        const int x = s - g;
+        const bool act = active(x);
+        const uint32_t q0 = cur.q;
+        cur = fetch(x + DBK_AHEAD);
+        place(x + 1, nxt.px);
+        const uint32_t seen = lds_peek(&sh.prog[w]), seen_c = lds_peek(&sh.cons[w + 1]);
+        // ---- vertical edges
+        uint8_t(*const img)[16] = tile->img[x & 1], (*const nimg)[16] = tile->img[(x + 1) & 1];
+        {
+            uint32_t a = e ? ap : prev.y, bb = bq;
+            edge_pass<false>(a, bb, thv.at, thv.beta, thv.s4, e);
+            *(uint32_t *)&img[k][p * 8 + 4 * e] = bb;
+            wave_sync();
+            if (e) img[k][p * 8 + 3] = (uint8_t)(a >> 24);
+            else prev.y = a;
+        }
+        finish(s, seen_c);
+        // ---- the rows above the MBs
+        if (y0 + 2 * w > 0 && s < W) lds_wait(&sh.prog[w], seen, (uint32_t)s + 1, err);
+        const uint8_t *const strip = g == 0 ? sh.ring[w][s % STRIP_SLOTS] : &tile->strip[0][0];
+        wave_sync();
+        // ---- horizontal edges (rows -2, -1 are the strip; rows -4, -3 are not read)
+        const uint2 c = lds_tr(tr_strip ? strip + max(tr + 2, 0) * 16 + th : &img[max(tr, 0)][th]);
+        bq = *(const uint32_t *)&nimg[k][p * 8 + 4 * e];
+        ap = *(const uint32_t *)&nimg[k][p * 8];
+        asm volatile("" : "+v"(nxt.q), "+v"(nxt.qt), "+v"(nxt.bv), "+v"(nxt.bh));
+        const DbkThr nv = dbk_threshold(&sh.lut, active(x + 1) ? nxt.bv : 0u, 1 + p, nxt.q, q0, nxt.q & DBQ_OWN_LEFT, e == 0, offA, offB);
+        const DbkThr nh = dbk_threshold(&sh.lut, active(x + 1) ? nxt.bh : 0u, 1 + p, nxt.q, nxt.qt, nxt.q & DBQ_OWN_TOP, e == 0, offA, offB);
+        lds_post(&sh.cons[w], (uint32_t)s + 1);
+        uint32_t a = c.x, bb = c.y;
+        edge_pass<false>(a, bb, thh.at, thh.beta, thh.s4, e);
+        *(uint32_t *)&tile->col[k][p * 8 + 4 * e] = bb;
+        wave_sync();
+        if (e) tile->col[k][p * 8 + 3] = (uint8_t)(a >> 24);
+        else if (act && top) slot[pl - pitch + (uint32_t)(x * 8 + k)] = (uint8_t)(a >> 24);  // row 7 of the MB above
+        wave_sync();
+        prev = lds_tr(tr_c);
+        thv = nv;
+        thh = nh;
+    };
+    const int steps = W + gl;
+    for (int s = 0; s < steps; s += DBK_AHEAD) {
+        step(s, f[0], f[1]);
+        step(s + 1, f[1], f[2]);
+        step(s + 2, f[2], f[0]);
+    }
+    if (steps % DBK_AHEAD == 0) finish(steps, 0u);  // the last row's last MB
+}
+
+// Two workgroups per band of `rows` MB rows, item 2 i for the luma plane of band i, item
+// 2 i + 1 for its chroma planes; the workgroup's last wave reads the strips of the band above.
+__global__ __launch_bounds__(WAVE *(DBK_MAX_ROWS + 1)) void k_deblock_band(const DevPic *__restrict__ pics,
+                                                                           const uint32_t *__restrict__ items, uint32_t n,
+                                                                           int rows, DevCtl *ctl, uint32_t *epoch_p,
+                                                                           uint32_t *err) {
     __shared__ DbkWgShared sh;
     __shared__ uint32_t s_ticket;
     const uint32_t epoch = launch_epoch(epoch_p);
-    const int nw = blockDim.x / WAVE, w = (int)uniform(threadIdx.x / WAVE);
-    if ((int)threadIdx.x < nw) sh.cons[threadIdx.x] = 0;
-    dbk_tables_init(&sh.tb);
-    const uint32_t t = band_ticket(ctl, &s_ticket, sh.prog, nw);
-    if (t < n) {
-        const uint32_t it = items[t];
+    const int w = (int)uniform(threadIdx.x / WAVE);
+    if ((int)threadIdx.x <= rows) sh.cons[threadIdx.x] = 0;
+    dbk_lut_init(&sh.lut);
+    const uint32_t t = band_ticket(ctl, &s_ticket, sh.prog, rows + 1);
+    if (t < 2 * n) {
+        const uint32_t it = items[t >> 1];
         const DevPic &P = pics[it >> WI_PIC_SHIFT];
         const int b = (int)(it & WI_MB_MASK), y0 = b * rows, y1 = min(P.H, y0 + rows);
-        if (P.dbk_idc != 1 && y0 + 2 * w < y1) deblock_pair_band(P, w, y0, y1, b, sh, epoch, err);
+        const GAS StripWords *const above = (const GAS StripWords *)G(P.gstrip) + (size_t)(b > 0 ? b - 1 : 0) * P.W;
+        if (P.dbk_idc != 1) {
+            if (!(t & 1u)) {
+                if (w < rows) {
+                    if (y0 + w < y1) deblock_luma_row(P, w, y0, y1, b, sh, epoch, err);
+                } else if (b > 0) {
+                    strip_reader<16, 0>(above, P.W, sh, epoch, err);
+                }
+            } else {
+                if (w < rows) {
+                    if (y0 + 2 * w < y1) deblock_chroma_rows(P, w, y0, y1, b, sh, epoch, err);
+                } else if (b > 0) {
+                    strip_reader<8, 16>(above, P.W, sh, epoch, err);
+                }
+            }
+        }
     }
     band_retire(ctl, epoch_p, epoch);
 }
@@ -2518,7 +2794,9 @@ __global__ __launch_bounds__(WAVE) void k_bs(const DevPic *__restrict__ pics, co
     // the current MB's blocks at x (or y) 15 and 0, and the current MB's qP on both sides.
     const bool own = e == 0 && other && P.dbk_idc == 0;
     const int ap = (e || own) ? addr : (dir == 0 ? addr - 1 : addr - W);
-    const bool edge = (uint32_t)addr < P.dbk_stop && (e > 0 || (has_nb && !(P.dbk_idc == 2 && other)));
+    // Nor are the internal luma edges 4 and 12 of an MB with the 8x8 transform.
+    const bool t8_skip = (e & 4) && (G(P.aux)[addr].kind & AUX_T8);
+    const bool edge = (uint32_t)addr < P.dbk_stop && !t8_skip && (e > 0 || (has_nb && !(P.dbk_idc == 2 && other)));
     if (edge) {
         MbView Qv, Pv;
         load_view(P, addr, Qv);
@@ -2622,9 +2900,9 @@ int h264g_launch_intra_band(const DevPic *pics, const uint32_t *bands, uint32_t 
 int h264g_launch_deblock_band(const DevPic *pics, const uint32_t *bands, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                               int rows, uint32_t *err, void *stream) {
     if (n == 0) return 0;
-    if (rows < 1 || rows > 2 * DBK_WG_MAX_WAVES) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_deblock_band, dim3(n), dim3(WAVE * ((rows + 1) / 2)), 0, (hipStream_t)stream, pics, bands, n,
-                       rows, ctl, epoch, err);
+    if (rows < 1 || rows > DBK_MAX_ROWS) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_deblock_band, dim3(2 * n), dim3(WAVE * (rows + 1)), 0, (hipStream_t)stream, pics, bands, n, rows, ctl,
+                       epoch, err);
     return (int)hipGetLastError();
 }
 

@@ -175,7 +175,7 @@ typedef struct h264g_config {
                                      (profiled contexts always launch directly)       */
     int32_t  deblock_schedule;    /* H264G_DEBLOCK_*                                  */
     int32_t  deblock_waves;       /* MB rows per band of H264G_DEBLOCK_BANDS, 1..24
-                                     (0 = 8); two rows per wave                      */
+                                     (0 = 8); bands run with at most 4 of them       */
     int32_t  intra_schedule;      /* H264G_INTRA_*                                    */
     int32_t  intra_waves;         /* rows per band = waves per workgroup of
                                      H264G_INTRA_BANDS, 1..8 (0 = 8)                 */
@@ -196,11 +196,11 @@ typedef struct h264g_config {
 #define H264G_INTRA_MB_WAVEFRONT 1
 
 /* Deblocking schedules (all give the raster-order result of 8.7):
- * BANDS        pictures cut into bands of `deblock_waves` MB rows, one workgroup per
- *              band and two rows per wave (the second one MB behind the first, on
- *              the wave's other 32 lanes); each MB's bottom rows go to the next row
- *              through LDS inside a band and through device memory between bands
- *              (default)
+ * BANDS        pictures cut into bands of `deblock_waves` MB rows (at most 4), two
+ *              workgroups per band, one for luma (a wave per row, the four edges of a
+ *              direction side by side on its lanes) and one for chroma (a wave per two
+ *              rows); each MB's bottom rows go to the next row through LDS inside a
+ *              band and through device memory between bands (default)
  * MB_WAVEFRONT persistent waves over single MBs ordered by t = x + 2y, progress words
  *              in device memory
  * MB_ROWS      persistent waves over MB rows of all pictures, progress in device memory */

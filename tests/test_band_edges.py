@@ -1,0 +1,31 @@
+"""The band schedules at the sizes where they can go wrong: pictures a few MBs wide or tall
+(one MB, the register sets the deblocking rows are unrolled over, the strip rings' 8 slots
+and one more, rows around the band heights, an odd second chroma row), every band height
+that changes the cut, against the C oracle, byte for byte."""
+import numpy as np
+import pytest
+
+from h264_video_decoder_demo_amd import Engine, Generator
+
+from helpers import oracle_decode
+
+SIZES = [(1, 1), (1, 9), (2, 4), (3, 5), (4, 8), (6, 3), (7, 7), (8, 2), (9, 6), (10, 13), (25, 5)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [(1, 1), (2, 3), (3, 8), (0, 0)])
+def test_band_cuts_match_oracle(rows):
+    """I, P and B pictures (4x4 and 8x8 transforms, strong and weak edges: QP 26..51)."""
+    with Engine(device=0, deblock_waves=rows[0], intra_waves=rows[1]) as eng:
+        for k, (w, h) in enumerate(SIZES):
+            gen = Generator(2, width_mbs=w, height_mbs=h, n_frames=4, seed=0xBA9D00 + 16 * k, qp_lo=26, qp_hi=51,
+                            intra_in_inter_permille=200, ipcm_permille=20)
+            sid = eng.open_stream_for(gen)
+            for i, desc, want in oracle_decode(gen):
+                p = eng.begin(sid, *gen.picture(i))
+                eng.submit(p)
+                eng.sync()
+                for got, ref, plane in zip(eng.readback(sid, desc.dst_slot), want[2], "YUV"):
+                    assert np.array_equal(got, ref), (w, h, i, plane)
+                eng.release(p)
+            eng.close_stream(sid)
