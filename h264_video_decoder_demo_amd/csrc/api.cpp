@@ -214,6 +214,8 @@ namespace {
 // MB rows per band that the deblocking bands are run with: the configured height, at most
 // H264G_DBK_MAX_ROWS (a wave per luma row, one to a SIMD).
 int dbk_rows(const h264g_ctx *c) { return std::min(c->dbk_waves, H264G_DBK_MAX_ROWS); }
+// The same for the intra bands.
+int intra_rows(const h264g_ctx *c) { return std::min(c->intra_waves, H264G_INTRA_MAX_ROWS); }
 
 hipStream_t lane_stream(const h264g_ctx *c, int lane) { return lane ? c->aux : c->stream; }
 // The four streams: lane 0, lane 1, their deblocking streams.
@@ -744,12 +746,14 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
     size_t o_bs = al(o_it + n_items * sizeof(uint32_t)), o_dbq = al(o_bs + (size_t)n_mbs * 32);
     size_t o_ires = al(o_dbq + (size_t)n_mbs * 4), o_bsref = al(o_ires + (size_t)pic->n_intra * 768);
     size_t o_ls = al(o_bsref + bsref.size()), o_pic = al(o_ls + lsv.size() * sizeof(uint16_t));
-    size_t total = al(o_pic + sizeof(DevPic));
+    size_t counted = al(o_pic + sizeof(DevPic));
+    // IMETA entries, which a fixed block holds beyond its counted bytes (H264G_SCRATCH_IMETA)
+    size_t o_imeta = counted, total = al(o_imeta + (mbaff ? 0 : (size_t)pic->n_intra * 16));
     void *dm = fixed;
     if (fixed) {
-        if (total > fixed_cap)
+        if (counted > fixed_cap)
             return h264g_set_error(H264G_E_ARG, "picture needs %zu bytes of device staging, the fixed block holds %zu",
-                                   total, fixed_cap);
+                                   counted, fixed_cap);
     } else {
         std::lock_guard<std::mutex> lk(ctx->mu);  // the rest of the staging runs unlocked
         dm = pool_get(ctx, total);
@@ -780,6 +784,7 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
     P.mbs = pic->d_mbs; P.aux = pic->d_aux; P.levels = pic->d_levels; P.wt = pic->d_wt;
     P.dpb = st.dpb; P.slot_bytes = st.slot_bytes; P.bs = d_bs; P.dbq = d_dbq; P.dst = d.dst_slot;
     P.ires = (int16_t *)(base + o_ires);
+    P.imeta = (uint32_t *)(base + o_imeta);
     P.irow = pic->d_items + irow_at; P.n_intra = pic->n_intra;
     P.W = W; P.H = H; P.offA = d.filter_offset_a; P.offB = d.filter_offset_b;
     P.mbaff = mbaff ? 1 : 0;
@@ -834,7 +839,7 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
         if (ev) HIPCHK(hipEventRecord(ev[1], s));
         if (q.n_intra)
             e = ctx->intra_schedule == H264G_INTRA_BANDS
-                    ? h264g_launch_intra_band(q.pics, q.ibands, q.n_ibands, &ctl[0], &ctl[2].ticket, ctx->intra_waves,
+                    ? h264g_launch_intra_band(q.pics, q.ibands, q.n_ibands, &ctl[0], &ctl[2].ticket, intra_rows(ctx),
                                               ctx->d_err, s)
                     : h264g_launch_intra(q.pics, q.intra, q.n_intra, &ctl[0], &ctl[2].ticket, ctx->d_err, ctx->waves, 0,
                                          s);
@@ -1106,17 +1111,20 @@ int32_t h264g_stream_open(h264g_ctx *c, const h264g_stream_desc *d, uint32_t *id
     // the strips between row bands (deblocking: 256 B per MB column and band; intra: 64 B)
     // and the MB pair progress words of MBAFF streams
     auto al = [](uint64_t v) { return (v + 255) & ~(uint64_t)255; };
-    s.o_rowprog = al((uint64_t)s.W * s.H * 4);
-    s.o_gstrip = al(s.o_rowprog + (uint64_t)s.H * 8);
-    s.o_istrip = s.o_gstrip + (uint64_t)((s.H + dbk_rows(c) - 1) / dbk_rows(c)) * s.W * 256;
-    s.o_pair = al(s.o_istrip + (uint64_t)((s.H + c->intra_waves - 1) / c->intra_waves) * s.W * 64);
-    s.set_bytes = al(s.o_pair + (s.mbaff ? (uint64_t)s.W * s.H / 2 * 4 : 0));
+    auto bands_of = [&](int rows) { return (uint64_t)((s.H + rows - 1) / rows); };
+    auto set_layout = [&](int drows, int irows) {  // with strips for bands of these heights
+        s.o_rowprog = al((uint64_t)s.W * s.H * 4);
+        s.o_gstrip = al(s.o_rowprog + (uint64_t)s.H * 8);
+        s.o_istrip = s.o_gstrip + bands_of(drows) * s.W * 256;
+        s.o_pair = al(s.o_istrip + bands_of(irows) * s.W * 64);
+        return al(s.o_pair + (s.mbaff ? (uint64_t)s.W * s.H / 2 * 4 : 0));
+    };
+    // The budget is charged for the strips of bands of the configured heights, whatever heights
+    // the bands are run with, so that admission does not depend on those.
+    const uint64_t charged_set = set_layout(c->dbk_waves, c->intra_waves);
+    s.set_bytes = set_layout(dbk_rows(c), intra_rows(c));
     const size_t dpb_bytes = s.slot_bytes * d->dpb_slots, prog_bytes = s.set_bytes * H264G_MAX_STREAM_PICS;
-    // The budget is charged for the strips of bands of the configured height, whatever height
-    // the bands are run with, so that admission does not depend on it.
-    const uint64_t run_bands = (uint64_t)(s.H + dbk_rows(c) - 1) / dbk_rows(c),
-                   cfg_bands = (uint64_t)(s.H + c->dbk_waves - 1) / c->dbk_waves;
-    const uint64_t need = dpb_bytes + prog_bytes - (run_bands - cfg_bands) * s.W * 256 * H264G_MAX_STREAM_PICS;
+    const uint64_t need = dpb_bytes + charged_set * H264G_MAX_STREAM_PICS;
     if (c->budget && c->used + need > c->budget)
         return h264g_set_error(H264G_E_BUDGET, "DPB budget: %llu + %llu > %llu", (unsigned long long)c->used,
                                (unsigned long long)need, (unsigned long long)c->budget);
@@ -1228,7 +1236,7 @@ int enqueue_picture(h264g_ctx *c, const h264g_pic *p, bool events = true) {
     q.rows = q.all + p->n_mbs;
     q.n_rows = p->n_rows;
     q.ibands = q.dbands = q.rows;  // band b of picture 0 is item b
-    q.n_ibands = (uint32_t)((p->H + c->intra_waves - 1) / c->intra_waves);
+    q.n_ibands = (uint32_t)((p->H + intra_rows(c) - 1) / intra_rows(c));
     q.n_dbands = (uint32_t)((p->H + dbk_rows(c) - 1) / dbk_rows(c));
     q.dbk_off = p->desc.disable_deblocking_filter_idc == 1;
     q.scaled = p->hpic.ls != nullptr;
@@ -1380,7 +1388,7 @@ int build_sub(h264g_ctx *c, const std::vector<const h264g_pic *> &pics, Batch *b
             }
     };
     std::vector<uint32_t> ibands, dbands;
-    if (!intra.empty()) bands(c->intra_waves, true, ibands);
+    if (!intra.empty()) bands(intra_rows(c), true, ibands);
     if (any_dbk) bands(dbk_rows(c), false, dbands);
     if (any_dbk && c->dbk_schedule == H264G_DEBLOCK_MB_ROWS) {
         // MB rows of all pictures, row index major: the row above always comes first.

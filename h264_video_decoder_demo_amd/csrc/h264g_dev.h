@@ -40,6 +40,12 @@ static_assert(sizeof(DevAux) == 28, "DevAux layout");
 #define ICOL_AV_SHIFT  11
 #define ICOL_DEP_SHIFT 15
 #define ICOL_RES       (1u << 19)
+// DevPic::imeta, one uint4 per intra MB at its index in DevPic::ires: its ICOL entry with its
+// type (0 I4x4, 1 I8x8, 2 I16x16) and the Intra16x16 / chroma prediction modes, the
+// Intra4x4 / Intra8x8 modes as nibbles in the next two words.
+#define IMETA_TYPE_SHIFT   20
+#define IMETA_I16_SHIFT    22
+#define IMETA_CHROMA_SHIFT 24
 
 // Resolved weighted-prediction parameters of one (refIdxL0, refIdxL1) combination.
 struct DevWeight {
@@ -73,6 +79,8 @@ struct DevPic {
     uint32_t *dbq;            // per-MB deblocking word, written by k_bs
     int16_t  *ires;           // residual of each intra MB with levels (DevAux::ires): luma
                               // 16x16 then Cb, Cr 8x8, raster; written by the inter stage
+    uint32_t *imeta;          // frame pictures: IMETA entries of the intra MBs, written by the
+                              // inter stage, read by the intra band schedule
     int32_t  mbaff;           // MbaffFrameFlag: MB address 2 p + b is the top / bottom MB of
                               // pair p, pairs in raster order
     const int8_t *bsref;      // MBAFF frames: per MB [list][quadrant] the picture identity
@@ -90,6 +98,8 @@ struct DevPic {
 #define LS8_AT   192          // first 8x8 entry
 #define LS8_LIST 384          // entries per 8x8 list (6 x 64)
 #define LS_ENTRIES 960
+
+static_assert(sizeof(DevPic) <= 256, "DevPic fits the 256 bytes that staging counts for it");
 
 // Work item: picture index in the batch and macroblock address.
 #define WI_PIC_SHIFT 20u
@@ -119,9 +129,11 @@ int h264g_launch_deblock(const DevPic *pics, const uint32_t *items, uint32_t n, 
                          uint32_t *err, int waves, void *stream);
 int h264g_launch_deblock_rows(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                               uint32_t *err, int waves, void *stream);
-// One workgroup of `waves` waves per picture (pics[0..n_pics)); pictures of up to 1024 MB rows.
+// Two workgroups (luma, chroma) of rows + 1 waves per band of `rows` MB rows, rows at most
+// H264G_INTRA_MAX_ROWS (one row to a SIMD, as for deblocking).
+#define H264G_INTRA_MAX_ROWS 4
 int h264g_launch_intra_band(const DevPic *pics, const uint32_t *bands, uint32_t n, DevCtl *ctl, uint32_t *epoch,
-                            int waves, uint32_t *err, void *stream);
+                            int rows, uint32_t *err, void *stream);
 // Two workgroups (luma, chroma) of rows + 1 waves per band of `rows` MB rows, rows at most
 // H264G_DBK_MAX_ROWS: with 4 each SIMD of the CU has one luma row to itself, and more rows
 // share its issue slots (a 1920x1088 I / P picture: 196 / 159 us with bands of 4 rows, 237 /
@@ -137,7 +149,11 @@ int h264g_launch_deblock_mbaff(const DevPic *pics, const uint32_t *items, uint32
 int h264g_launch_bgr24(const uint8_t *yuv, int wl, int hl, uint8_t *bgr, uint32_t stride, int flip, void *stream);
 int h264g_launch_copy(const uint8_t *src, uint8_t *dst, uint64_t bytes, void *stream);
 }
-// Device address of the static scratch array (H264G_STATIC_SCRATCH_BYTES) on `device`,
+// Bytes of the static scratch array beyond H264G_STATIC_SCRATCH_BYTES, for the IMETA entries: an
+// intra MB counts at least 768 + 172 + 28 bytes of the array and has 16 here.
+#define H264G_SCRATCH_IMETA (2u << 20)
+static_assert(H264G_STATIC_SCRATCH_BYTES / 968u * 16u + 256u <= H264G_SCRATCH_IMETA, "every intra MB has its entry");
+// Device address of the static scratch array on `device`,
 // which must be the current device; looked up on the first call per device.  Returns a
 // hipError_t.
 int h264g_scratch_address(int device, void **out);

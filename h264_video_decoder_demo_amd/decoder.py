@@ -135,13 +135,17 @@ class _Prefetch:
             yield x
 
     def close(self):
+        """Stops the producer: empties the queue until a blocked put has gone through and the
+        thread has ended (joined in short steps: a blocking get on the drained queue would
+        sit out its whole timeout while the thread ends)."""
         self._stop.set()
         while self._t.is_alive():
             try:
-                self._q.get(timeout=0.05)
+                while True:
+                    self._q.get_nowait()
             except queue.Empty:
                 pass
-        self._t.join()
+            self._t.join(0.0005)
 
 
 class H264VideoDecoder:

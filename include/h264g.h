@@ -177,8 +177,8 @@ typedef struct h264g_config {
     int32_t  deblock_waves;       /* MB rows per band of H264G_DEBLOCK_BANDS, 1..24
                                      (0 = 8); bands run with at most 4 of them       */
     int32_t  intra_schedule;      /* H264G_INTRA_*                                    */
-    int32_t  intra_waves;         /* rows per band = waves per workgroup of
-                                     H264G_INTRA_BANDS, 1..8 (0 = 8)                 */
+    int32_t  intra_waves;         /* MB rows per band of H264G_INTRA_BANDS, 1..8
+                                     (0 = 8); bands run with at most 4 of them       */
     int32_t  lane_split_mbs;      /* streams of at least this many MBs per picture run
                                      on a second lane, so their long intra /
                                      deblocking chains overlap the other pictures'
@@ -187,9 +187,10 @@ typedef struct h264g_config {
                                      (no deblocking overlap either)                   */
 } h264g_config;
 
-/* Intra schedules: BANDS = pictures cut into bands of `intra_waves` MB rows, one
- * workgroup per band and one wave per row walking the row's intra MBs, LDS row progress
- * inside a band and device-memory progress between bands (default); MB_WAVEFRONT =
+/* Intra schedules: BANDS = pictures cut into bands of `intra_waves` MB rows (at most 4),
+ * one workgroup per band for luma and one for chroma, one wave per row walking the row's
+ * intra MBs, LDS rings between the rows of a band and tagged words in device memory
+ * between bands (default); MB_WAVEFRONT =
  * persistent waves over the intra MBs of all pictures ordered by t = x + 2y, progress
  * words in device memory. */
 #define H264G_INTRA_BANDS        0

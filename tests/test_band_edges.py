@@ -29,3 +29,23 @@ def test_band_cuts_match_oracle(rows):
                     assert np.array_equal(got, ref), (w, h, i, plane)
                 eng.release(p)
             eng.close_stream(sid)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("permille", [4, 60, 700])
+def test_sparse_and_dense_intra_rows_match_oracle(permille):
+    """Intra MBs few and far between, and many, in P and B pictures wider than the intra rows'
+    rings (64 columns): rows that wait far ahead of, or behind, the row above."""
+    with Engine(device=0) as eng:
+        for k, (w, h) in enumerate([(66, 9), (131, 6), (200, 3)]):
+            gen = Generator(2, width_mbs=w, height_mbs=h, n_frames=3, b_frames=1, seed=0xBA9E00 + 16 * k,
+                            intra_in_inter_permille=permille)
+            sid = eng.open_stream_for(gen)
+            for i, desc, want in oracle_decode(gen):
+                p = eng.begin(sid, *gen.picture(i))
+                eng.submit(p)
+                eng.sync()
+                for got, ref, plane in zip(eng.readback(sid, desc.dst_slot), want[2], "YUV"):
+                    assert np.array_equal(got, ref), (w, h, i, plane)
+                eng.release(p)
+            eng.close_stream(sid)
