@@ -56,9 +56,9 @@ struct Stream {
     uint64_t slot_bytes = 0;
     // H264G_MAX_STREAM_PICS progress sets, one for each picture of the stream in one
     // launch, each: per-MB progress words | per-row progress words | deblocking strips
-    // between row bands | intra strips | MBAFF streams: deblocking progress per MB pair
+    // between row bands | intra strips
     uint8_t *prog = nullptr;
-    uint64_t set_bytes = 0, o_rowprog = 0, o_gstrip = 0, o_istrip = 0, o_pair = 0;
+    uint64_t set_bytes = 0, o_rowprog = 0, o_gstrip = 0, o_istrip = 0;
     bool mbaff = false;            // MBAFF frames (pairs of field / frame MBs)
     int strip_dbk_rows = 0, strip_intra_rows = 0;  // strips sized for bands of at least these many rows
     uint64_t bytes = 0;
@@ -76,7 +76,6 @@ void use_set(const Stream &s, int k, DevPic &P) {
     P.rowprog = (uint64_t *)(b + s.o_rowprog);
     P.gstrip = b + s.o_gstrip;
     P.istrip = (uint64_t *)(b + s.o_istrip);
-    P.pairprog = s.mbaff ? (uint32_t *)(b + s.o_pair) : nullptr;
 }
 
 struct Batch;
@@ -841,15 +840,14 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
             e = ctx->intra_schedule == H264G_INTRA_BANDS
                     ? h264g_launch_intra_band(q.pics, q.ibands, q.n_ibands, &ctl[0], &ctl[2].ticket, intra_rows(ctx),
                                               ctx->d_err, s)
-                    : h264g_launch_intra(q.pics, q.intra, q.n_intra, &ctl[0], &ctl[2].ticket, ctx->d_err, ctx->waves, 0,
-                                         s);
+                    : h264g_launch_intra(q.pics, q.intra, q.n_intra, &ctl[0], &ctl[2].ticket, ctx->d_err, ctx->waves, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "intra launch: %s", hipGetErrorString((hipError_t)e));
-        if (q.n_mintra)
-            e = h264g_launch_intra(q.pics, q.mintra, q.n_mintra, &ctl[0], &ctl[2].ticket, ctx->d_err, ctx->waves, 1, s);
+        if (q.n_mintra) e = h264g_launch_intra_mbaff(q.pics, q.n_pics, ctx->d_err, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "intra launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         if (ev) HIPCHK(hipEventRecord(ev[2], s));
         if (!q.dbk_off) {
             e = h264g_launch_bs(q.pics, q.all, q.n_all, s);
+            if (!e) e = h264g_launch_bs_mbaff(q.pics, q.mpairs, q.n_mpairs, s);
             if (e) return h264g_set_error(H264G_E_DEVICE, "bS launch: %s", hipGetErrorString((hipError_t)e));
         }
         if (ev) HIPCHK(hipEventRecord(ev[3], s));
@@ -870,7 +868,7 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
                 e = h264g_launch_deblock_rows(q.pics, q.rows, q.n_rows, &ctl[1], epoch, ctx->d_err, ctx->waves, s);
             }
             if (e) return h264g_set_error(H264G_E_DEVICE, "deblock launch: %s", hipGetErrorString((hipError_t)e));
-            e = h264g_launch_deblock_mbaff(q.pics, q.mpairs, q.n_mpairs, &ctl[1], epoch, ctx->d_err, ctx->waves, s);
+            if (q.n_mpairs) e = h264g_launch_deblock_mbaff(q.pics, q.n_pics, ctx->d_err, s);
             if (e) return h264g_set_error(H264G_E_DEVICE, "deblock launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         }
         if (ev) HIPCHK(hipEventRecord(ev[5], s));
@@ -1109,19 +1107,18 @@ int32_t h264g_stream_open(h264g_ctx *c, const h264g_stream_desc *d, uint32_t *id
     s.lane = c->split_mbs > 0 && s.W * s.H >= c->split_mbs ? 1 : 0;
     // DPB slots, and the progress sets: per-MB progress words, per-row progress words,
     // the strips between row bands (deblocking: 256 B per MB column and band; intra: 64 B)
-    // and the MB pair progress words of MBAFF streams
     auto al = [](uint64_t v) { return (v + 255) & ~(uint64_t)255; };
     auto bands_of = [&](int rows) { return (uint64_t)((s.H + rows - 1) / rows); };
     auto set_layout = [&](int drows, int irows) {  // with strips for bands of these heights
         s.o_rowprog = al((uint64_t)s.W * s.H * 4);
         s.o_gstrip = al(s.o_rowprog + (uint64_t)s.H * 8);
         s.o_istrip = s.o_gstrip + bands_of(drows) * s.W * 256;
-        s.o_pair = al(s.o_istrip + bands_of(irows) * s.W * 64);
-        return al(s.o_pair + (s.mbaff ? (uint64_t)s.W * s.H / 2 * 4 : 0));
+        return al(s.o_istrip + bands_of(irows) * s.W * 64);
     };
     // The budget is charged for the strips of bands of the configured heights, whatever heights
-    // the bands are run with, so that admission does not depend on those.
-    const uint64_t charged_set = set_layout(c->dbk_waves, c->intra_waves);
+    // the bands are run with, and for a word per MB pair of MBAFF streams, so that admission
+    // does not depend on the schedule.
+    const uint64_t charged_set = al(set_layout(c->dbk_waves, c->intra_waves) + (s.mbaff ? (uint64_t)s.W * s.H / 2 * 4 : 0));
     s.set_bytes = set_layout(dbk_rows(c), intra_rows(c));
     const size_t dpb_bytes = s.slot_bytes * d->dpb_slots, prog_bytes = s.set_bytes * H264G_MAX_STREAM_PICS;
     const uint64_t need = dpb_bytes + charged_set * H264G_MAX_STREAM_PICS;

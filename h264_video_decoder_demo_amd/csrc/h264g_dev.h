@@ -66,7 +66,8 @@ struct DevPic {
     uint32_t *flags;          // per-MB wavefront progress words of the stream
     uint64_t *rowprog;        // per-MB-row progress of row-pipelined deblocking:
                               // epoch << 32 | MBs of the row finished
-    uint8_t  *bs;             // boundary strengths, 32 per MB: [dir][4-line segment][edge]
+    uint8_t  *bs;             // boundary strengths, 32 bytes per MB: [dir][4-line segment][edge]
+                              // (MBAFF frames: nibbles, see k_bs_mbaff)
     const uint32_t *irow;     // intra MBs per row: H + 1 offsets, then one ICOL entry per intra MB
     uint32_t n_intra;         // intra-predicted MBs of the picture
     int32_t  dst;             // destination slot
@@ -76,7 +77,7 @@ struct DevPic {
     int32_t  cip;             // constrained_intra_pred_flag
     uint8_t  *gstrip;         // deblocking strips between bands of the stream: W x 256 B per band
     uint64_t *istrip;         // intra strips between bands of the stream: W x 8 words per band
-    uint32_t *dbq;            // per-MB deblocking word, written by k_bs
+    uint32_t *dbq;            // per-MB deblocking word, written with the strengths
     int16_t  *ires;           // residual of each intra MB with levels (DevAux::ires): luma
                               // 16x16 then Cb, Cr 8x8, raster; written by the inter stage
     uint32_t *imeta;          // frame pictures: IMETA entries of the intra MBs, written by the
@@ -85,7 +86,6 @@ struct DevPic {
                               // pair p, pairs in raster order
     const int8_t *bsref;      // MBAFF frames: per MB [list][quadrant] the picture identity
                               // the bS derivation compares, RefPicListX[RefIdxLX] (-1: none)
-    uint32_t *pairprog;       // MBAFF streams: per-MB-pair deblocking progress words
     uint32_t dbk_stop;        // MBs from this address on filter none of their edges (the
                               // first MB of no slice; W * H when every MB has one)
     int32_t  multi_slice;     // the MBs carry more than one slice number (MBs of no slice
@@ -124,7 +124,9 @@ int h264g_launch_inter(const DevPic *pics, const uint32_t *items, uint32_t n, co
 // `epoch` points at the device word shared by all wavefront launches of a context
 // (initially 1; each launch's last wave advances it).
 int h264g_launch_intra(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
-                       uint32_t *err, int waves, int mbaff, void *stream);
+                       uint32_t *err, int waves, void *stream);
+// Intra MBs of the MBAFF frames among the launch's pictures, one workgroup per picture.
+int h264g_launch_intra_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *err, void *stream);
 int h264g_launch_deblock(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                          uint32_t *err, int waves, void *stream);
 int h264g_launch_deblock_rows(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
@@ -142,10 +144,10 @@ int h264g_launch_intra_band(const DevPic *pics, const uint32_t *bands, uint32_t 
 int h264g_launch_deblock_band(const DevPic *pics, const uint32_t *bands, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                               int rows, uint32_t *err, void *stream);
 int h264g_launch_bs(const DevPic *pics, const uint32_t *items, uint32_t n, void *stream);
-// Deblocking of MBAFF frames: persistent waves over MB pairs (items: picture index << 20 |
-// pair index, ordered by t = x + 2 y of the pair), one pair per wave at a time.
-int h264g_launch_deblock_mbaff(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
-                               uint32_t *err, int waves, void *stream);
+// Boundary strengths of the MBAFF frames (pairs: picture index << 20 | pair index), then their
+// deblocking, one workgroup per picture.
+int h264g_launch_bs_mbaff(const DevPic *pics, const uint32_t *pairs, uint32_t n, void *stream);
+int h264g_launch_deblock_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *err, void *stream);
 int h264g_launch_bgr24(const uint8_t *yuv, int wl, int hl, uint8_t *bgr, uint32_t stride, int flip, void *stream);
 int h264g_launch_copy(const uint8_t *src, uint8_t *dst, uint64_t bytes, void *stream);
 }

@@ -49,3 +49,26 @@ def test_sparse_and_dense_intra_rows_match_oracle(permille):
                     assert np.array_equal(got, ref), (w, h, i, plane)
                 eng.release(p)
             eng.close_stream(sid)
+
+
+@pytest.mark.gpu
+def test_mbaff_and_frame_pictures_in_one_batch():
+    """MBAFF frames of 1 to 20 pair rows (one workgroup walks them in rounds of 16) beside
+    frame pictures and a picture without deblocking in the same batches."""
+    with Engine(device=0) as eng:
+        gens = [Generator(3, width_mbs=w, height_mbs=h, n_frames=3, seed=0xBA9F00 + h, intra_in_inter_permille=200,
+                          disable_deblocking_filter_idc=idc) for w, h, idc in [(1, 2, 0), (5, 34, 0), (9, 40, 0), (4, 6, 1)]]
+        gens.append(Generator(2, width_mbs=9, height_mbs=5, n_frames=3, seed=0xBA9F99))
+        sids = [eng.open_stream_for(g) for g in gens]
+        for wants in zip(*(oracle_decode(g) for g in gens)):
+            pics = [eng.begin(s, *g.picture(w[0])) for s, g, w in zip(sids, gens, wants)]
+            b = eng.batch_create(pics)
+            for _ in range(2):
+                eng.batch_run(b)
+            eng.sync()
+            for k, (s, (i, desc, want)) in enumerate(zip(sids, wants)):
+                for got, ref, plane in zip(eng.readback(s, desc.dst_slot), want[2], "YUV"):
+                    assert np.array_equal(got, ref), (k, i, plane)
+            eng.batch_destroy(b)
+            for p in pics:
+                eng.release(p)
