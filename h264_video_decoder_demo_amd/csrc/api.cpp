@@ -119,17 +119,15 @@ struct h264g_pic {
     DevAux *d_aux = nullptr;
     int16_t *d_levels = nullptr;
     DevWeight *d_wt = nullptr;
-    uint32_t *d_items = nullptr;   // inter | intra | deblock (per MB) | deblock (rows) queues
+    uint32_t *d_items = nullptr;   // t-ordered intra MBs | all MBs | MB rows (those that the context's
+                                   // schedules take lists of) | intra MBs per row
     DevPic *d_pic = nullptr;
-    uint32_t n_inter = 0, n_intra = 0, n_mbs = 0, n_rows = 0;
+    uint32_t n_intra = 0;
     DevPic hpic;                   // host copy (batches re-pack it)
-    std::vector<uint32_t> intra_t, all_t;  // host copies of the t-ordered queues (MB addresses;
-                                           // MBAFF frames: intra MBs in pair t order, and
-                                           // all_t holds MB pair indices)
-    std::vector<uint32_t> inter_list;
-    bool mbaff = false;            // an MBAFF frame: intra on the per-MB wavefront, deblocking
-                                   // over MB pairs (the band schedules take frame MBs only)
-    uint32_t n_pairs = 0;
+    std::vector<uint32_t> intra_t, all_t;  // host copies of the t-ordered queues (MB addresses), for
+                                           // the schedules that walk them
+    bool mbaff = false;            // an MBAFF frame: one workgroup walks its MB pairs (the band
+                                   // schedules take frame MBs only)
     uint64_t alg[3] = {0, 0, 0};
 };
 
@@ -140,12 +138,11 @@ struct Batch {
     size_t dbytes = 0;
     DevPic *d_pics = nullptr;
     uint32_t n_pics = 0;
-    uint32_t *d_inter = nullptr, *d_intra = nullptr, *d_all = nullptr, *d_rows = nullptr;
+    uint32_t *d_chunks = nullptr, *d_mchunks = nullptr;  // runs of MBs of the frame pictures / MBAFF frames
+    uint32_t *d_intra = nullptr, *d_all = nullptr, *d_rows = nullptr;
     uint32_t *d_ibands = nullptr, *d_dbands = nullptr;   // (picture, band) items, band-major
-    uint32_t n_inter = 0, n_intra = 0, n_all = 0, n_rows = 0, n_ibands = 0, n_dbands = 0;
-    // MBAFF frames: inter MBs (after the frame pictures' in d_inter), intra MBs, MB pairs
-    uint32_t *d_minter = nullptr, *d_mintra = nullptr, *d_mpairs = nullptr;
-    uint32_t n_minter = 0, n_mintra = 0, n_mpairs = 0;
+    uint32_t n_chunks = 0, n_mchunks = 0, n_all = 0, n_rows = 0, n_ibands = 0, n_dbands = 0;
+    uint32_t n_intra = 0, n_mintra = 0;  // intra MBs of the frame pictures / MBAFF frames
     bool dbk_off = false;            // no picture of the batch is deblocked
     bool scaled = false;             // a picture of the batch has scaling matrices
     hipGraphExec_t graph = nullptr;  // the captured stage sequence (kernel nodes only)
@@ -658,43 +655,28 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
         }
         alg_inter += 384 + 2 * (uint64_t)(nmask + nvals) + 8;
     }
-    // ---- queues
-    pic->inter_list.clear();
+    // ---- queues ordered by t = x + 2 y, for the schedules that walk one
     pic->intra_t.clear();
     pic->all_t.clear();
-    for (uint32_t a = 0; a < n_mbs; a++)
-        if (aux[a].kind & (AUX_INTER | AUX_PCM)) pic->inter_list.push_back(a);
     pic->mbaff = mbaff;
-    if (mbaff) {  // pairs by t = x + 2 y, the top MB before the bottom one
-        const int HP = H / 2;
-        for (int t = 0; t <= (W - 1) + 2 * (HP - 1); t++)
-            for (int y = 0; y < HP; y++) {
-                const int xx = t - 2 * y;
-                if (xx < 0) break;
-                if (xx >= W) continue;
-                const uint32_t pair = (uint32_t)(y * W + xx);
-                pic->all_t.push_back(pair);
-                for (uint32_t a = 2 * pair; a < 2 * pair + 2; a++)
-                    if (aux[a].kind & AUX_INTRA) {
-                        aux[a].ires |= (uint32_t)pic->intra_t.size();  // residual slot
-                        pic->intra_t.push_back(a);
-                    }
-            }
-        pic->n_pairs = (uint32_t)pic->all_t.size();
-    } else {
+    pic->n_intra = 0;
+    for (uint32_t a = 0; a < n_mbs; a++)
+        if (aux[a].kind & AUX_INTRA) {
+            if (mbaff) aux[a].ires |= pic->n_intra;  // residual slot (frame pictures: below)
+            pic->n_intra++;
+        }
+    const bool want_intra_t = !mbaff && ctx->intra_schedule != H264G_INTRA_BANDS,
+               want_all_t = !mbaff && ctx->dbk_schedule == H264G_DEBLOCK_MB_WAVEFRONT;
+    if (want_intra_t || want_all_t)
         for (int t = 0; t <= (W - 1) + 2 * (H - 1); t++)
             for (int y = 0; y < H; y++) {
                 int xx = t - 2 * y;
                 if (xx < 0) break;
                 if (xx >= W) continue;
                 uint32_t a = (uint32_t)(y * W + xx);
-                pic->all_t.push_back(a);
-                if (aux[a].kind & AUX_INTRA) pic->intra_t.push_back(a);
+                if (want_all_t) pic->all_t.push_back(a);
+                if (want_intra_t && (aux[a].kind & AUX_INTRA)) pic->intra_t.push_back(a);
             }
-    }
-    pic->n_inter = (uint32_t)pic->inter_list.size();
-    pic->n_intra = (uint32_t)pic->intra_t.size();
-    pic->n_mbs = mbaff ? pic->n_pairs : n_mbs;  // entries of all_t
     pic->alg[0] = alg_inter;
     pic->alg[1] = alg_intra;
     // deblocking: one read and one write of the picture, the bS inputs (motion records,
@@ -704,7 +686,6 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     size_t o_mbs = 0, o_aux = al(o_mbs + n_mbs * sizeof(h264g_mb)), o_lv = al(o_aux + n_mbs * sizeof(DevAux));
     size_t o_wt = al(o_lv + n_levels * sizeof(int16_t) + 16), o_it = al(o_wt + wt.size() * sizeof(DevWeight));
-    pic->n_rows = mbaff ? 0u : (uint32_t)H;
     // intra MBs per row: offsets, then one entry per intra MB (the per-picture intra band
     // schedule; an MB's residual sits at its entry's index in P.ires).  The entry carries
     // what the band kernel would otherwise load from the neighbours' records before its
@@ -741,7 +722,10 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
         }
     }
     irow[H] = (uint32_t)icol.size();
-    size_t n_items = pic->n_inter + pic->n_intra + pic->all_t.size() + pic->n_rows + irow.size() + icol.size();
+    const uint32_t n_rows = !mbaff && ctx->dbk_schedule == H264G_DEBLOCK_MB_ROWS ? (uint32_t)H : 0u;
+    // (the bytes counted against a fixed block are those of full lists: inter and intra MBs, all
+    // MBs or MB pairs, rows, intra MBs per row)
+    size_t n_items = (size_t)n_mbs + (mbaff ? n_mbs / 2 : n_mbs + (uint32_t)H) + irow.size() + icol.size();
     size_t o_bs = al(o_it + n_items * sizeof(uint32_t)), o_dbq = al(o_bs + (size_t)n_mbs * 32);
     size_t o_ires = al(o_dbq + (size_t)n_mbs * 4), o_bsref = al(o_ires + (size_t)pic->n_intra * 768);
     size_t o_ls = al(o_bsref + bsref.size()), o_pic = al(o_ls + lsv.size() * sizeof(uint16_t));
@@ -771,10 +755,9 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
     uint32_t *d_dbq = (uint32_t *)(base + o_dbq);
     std::vector<uint32_t> items;
     items.reserve(n_items);
-    items.insert(items.end(), pic->inter_list.begin(), pic->inter_list.end());
     items.insert(items.end(), pic->intra_t.begin(), pic->intra_t.end());
     items.insert(items.end(), pic->all_t.begin(), pic->all_t.end());
-    for (uint32_t y = 0; y < pic->n_rows; y++) items.push_back(y);
+    for (uint32_t y = 0; y < n_rows; y++) items.push_back(y);
     const size_t irow_at = items.size();
     items.insert(items.end(), irow.begin(), irow.end());
     items.insert(items.end(), icol.begin(), icol.end());
@@ -804,20 +787,18 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
     return 0;
 }
 
-// The launches of one picture or batch.  all = every MB (t order: it serves the bS
-// pre-pass and the per-MB deblocking wavefront); rows = MB rows (row index major) for
-// the cross-CU row schedule.
+// The launches of one picture or batch.  chunks / mchunks: runs of MBs of the frame pictures and
+// of the MBAFF frames (null: all of picture 0); intra, all: MBs in t order for the per-MB
+// wavefronts; rows: MB rows (row index major) for the cross-CU row schedule; ibands, dbands:
+// bands (null: those of picture 0).
 struct StageSet {
     const DevPic *pics;
     uint32_t n_pics;
-    const uint32_t *inter, *intra, *all, *rows, *ibands, *dbands;
-    uint32_t n_inter, n_intra, n_all, n_rows, n_ibands, n_dbands;
-    bool dbk_off;
+    const uint32_t *chunks = nullptr, *mchunks = nullptr, *intra = nullptr, *all = nullptr, *rows = nullptr,
+                   *ibands = nullptr, *dbands = nullptr;
+    uint32_t n_chunks = 0, n_mchunks = 0, n_intra = 0, n_mintra = 0, n_all = 0, n_rows = 0, n_ibands = 0, n_dbands = 0;
+    bool dbk_off = false;
     bool scaled = false;  // a picture has scaling matrices: the inter stage takes the kernel that reads them
-    // MBAFF frames: inter MBs, intra MBs for the per-MB wavefront, MB pairs for their
-    // deblocking
-    const uint32_t *minter = nullptr, *mintra = nullptr, *mpairs = nullptr;
-    uint32_t n_minter = 0, n_mintra = 0, n_mpairs = 0;
 };
 
 // Parts of a stage set: inter / intra / bS, and deblocking.
@@ -830,10 +811,9 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
     int e = 0;
     if (parts & kFront) {
         if (ev) HIPCHK(hipEventRecord(ev[0], s));
-        e = h264g_launch_inter(q.pics, q.inter, q.n_inter, q.intra, q.n_intra, 0, q.scaled ? 1 : 0, ctx->d_err, s);
+        e = h264g_launch_inter(q.pics, q.chunks, q.n_chunks, 0, q.scaled ? 1 : 0, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "inter launch: %s", hipGetErrorString((hipError_t)e));
-        // MBAFF frames: inter MBs and the residuals of their intra MBs (lists of their own)
-        e = h264g_launch_inter(q.pics, q.minter, q.n_minter, q.mintra, q.n_mintra, 1, 0, ctx->d_err, s);
+        e = h264g_launch_inter(q.pics, q.mchunks, q.n_mchunks, 1, 0, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "inter launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         if (ev) HIPCHK(hipEventRecord(ev[1], s));
         if (q.n_intra)
@@ -846,8 +826,8 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
         if (e) return h264g_set_error(H264G_E_DEVICE, "intra launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         if (ev) HIPCHK(hipEventRecord(ev[2], s));
         if (!q.dbk_off) {
-            e = h264g_launch_bs(q.pics, q.all, q.n_all, s);
-            if (!e) e = h264g_launch_bs_mbaff(q.pics, q.mpairs, q.n_mpairs, s);
+            e = h264g_launch_bs(q.pics, q.chunks, q.n_chunks, 0, s);
+            if (!e) e = h264g_launch_bs(q.pics, q.mchunks, q.n_mchunks, 1, s);
             if (e) return h264g_set_error(H264G_E_DEVICE, "bS launch: %s", hipGetErrorString((hipError_t)e));
         }
         if (ev) HIPCHK(hipEventRecord(ev[3], s));
@@ -868,7 +848,7 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
                 e = h264g_launch_deblock_rows(q.pics, q.rows, q.n_rows, &ctl[1], epoch, ctx->d_err, ctx->waves, s);
             }
             if (e) return h264g_set_error(H264G_E_DEVICE, "deblock launch: %s", hipGetErrorString((hipError_t)e));
-            if (q.n_mpairs) e = h264g_launch_deblock_mbaff(q.pics, q.n_pics, ctx->d_err, s);
+            if (q.n_mchunks) e = h264g_launch_deblock_mbaff(q.pics, q.n_pics, ctx->d_err, s);
             if (e) return h264g_set_error(H264G_E_DEVICE, "deblock launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         }
         if (ev) HIPCHK(hipEventRecord(ev[5], s));
@@ -1220,32 +1200,25 @@ namespace {
 // The launches of one staged picture (caller holds ctx->mu).  events: profiling contexts
 // record stage events (created on demand).
 int enqueue_picture(h264g_ctx *c, const h264g_pic *p, bool events = true) {
-    const uint32_t *it = p->d_items;
     StageSet q;
     q.pics = p->d_pic;
     q.n_pics = 1;
-    q.inter = it;
-    q.n_inter = p->n_inter;
-    q.intra = it + p->n_inter;
-    q.n_intra = p->n_intra;
-    q.all = q.intra + p->n_intra;
-    q.n_all = p->n_mbs;
-    q.rows = q.all + p->n_mbs;
-    q.n_rows = p->n_rows;
-    q.ibands = q.dbands = q.rows;  // band b of picture 0 is item b
-    q.n_ibands = (uint32_t)((p->H + intra_rows(c) - 1) / intra_rows(c));
-    q.n_dbands = (uint32_t)((p->H + dbk_rows(c) - 1) / dbk_rows(c));
     q.dbk_off = p->desc.disable_deblocking_filter_idc == 1;
     q.scaled = p->hpic.ls != nullptr;
-    if (p->mbaff) {  // items: inter MBs, intra MBs (pair t order), MB pairs (t order)
-        q.minter = q.inter;
-        q.n_minter = q.n_inter;
-        q.n_inter = 0;
-        q.mintra = q.intra;
+    const uint32_t n_chunks = ((uint32_t)(p->W * p->H) + MB_CHUNK - 1) / MB_CHUNK;
+    if (p->mbaff) {
+        q.n_mchunks = n_chunks;
         q.n_mintra = p->n_intra;
-        q.mpairs = q.all;
-        q.n_mpairs = q.dbk_off ? 0u : p->n_pairs;
-        q.n_intra = q.n_all = q.n_rows = q.n_ibands = q.n_dbands = 0;
+    } else {
+        q.n_chunks = n_chunks;
+        q.n_intra = p->n_intra;
+        q.intra = p->d_items;
+        q.all = q.intra + p->intra_t.size();
+        q.n_all = (uint32_t)p->all_t.size();
+        q.rows = q.all + p->all_t.size();
+        q.n_rows = (uint32_t)p->H;
+        q.n_ibands = (uint32_t)((p->H + intra_rows(c) - 1) / intra_rows(c));
+        q.n_dbands = (uint32_t)((p->H + dbk_rows(c) - 1) / dbk_rows(c));
     }
     return enqueue(c, q, c->streams[p->stream].lane, {slot_use(p->stream, p->desc)}, nullptr, events);
 }
@@ -1328,8 +1301,9 @@ namespace {
 int build_sub(h264g_ctx *c, const std::vector<const h264g_pic *> &pics, Batch *b) {
     const uint32_t n = (uint32_t)pics.size();
     std::vector<DevPic> hp(n);
-    std::vector<uint32_t> inter, intra, dbk, minter;
+    std::vector<uint32_t> chunks, mchunks, intra, all, rows;
     int maxt = 0;
+    bool any_dbk = false, any_mdbk = false;
     b->uses.clear();
     b->streams.clear();
     for (uint32_t i = 0; i < n; i++) {
@@ -1342,37 +1316,27 @@ int build_sub(h264g_ctx *c, const std::vector<const h264g_pic *> &pics, Batch *b
         use_set(c->streams[p->stream], k, hp[i]);
         b->uses.push_back(slot_use(p->stream, p->desc));
         b->streams.push_back({p->stream, p->stream_gen});
-        for (uint32_t a : p->inter_list) (p->mbaff ? minter : inter).push_back((i << WI_PIC_SHIFT) | a);
+        std::vector<uint32_t> &ch = p->mbaff ? mchunks : chunks;
+        for (uint32_t a = 0; a < (uint32_t)(p->W * p->H); a += MB_CHUNK) ch.push_back((i << WI_PIC_SHIFT) | a);
+        (p->mbaff ? b->n_mintra : b->n_intra) += p->n_intra;
+        (p->mbaff ? any_mdbk : any_dbk) |= p->desc.disable_deblocking_filter_idc != 1;
         maxt = std::max(maxt, (p->W - 1) + 2 * (p->H - 1));
     }
-    // the frame pictures' inter MBs, then the MBAFF frames' (each set is one launch)
-    const uint32_t n_frame_inter = (uint32_t)inter.size();
-    inter.insert(inter.end(), minter.begin(), minter.end());
-    // Wavefront queues of all pictures merged by t = x + 2y (counting sort): every
-    // dependency of an entry has a smaller t and therefore an earlier ticket.  MBAFF frames
-    // (mbaff = true) go by the t of their MB pairs, the top MB before the bottom one.
-    auto merge = [&](bool intra_only, bool mbaff, std::vector<uint32_t> &outq) {
+    // Wavefront queues of all frame pictures merged by t = x + 2y (counting sort), for the per-MB
+    // wavefront schedules: every dependency of an entry has a smaller t and therefore an
+    // earlier ticket.
+    auto merge = [&](bool intra_only, std::vector<uint32_t> &outq) {
         std::vector<std::vector<uint32_t>> byt(maxt + 1);
         for (uint32_t i = 0; i < n; i++) {
             const h264g_pic *p = pics[i];
-            if (p->mbaff != mbaff || (!intra_only && p->desc.disable_deblocking_filter_idc == 1)) continue;
-            const std::vector<uint32_t> &q = intra_only ? p->intra_t : p->all_t;
-            for (uint32_t a : q) {
-                const uint32_t xy = mbaff && intra_only ? a >> 1 : a;  // MB pairs: all_t holds pairs
-                int t = (int)(xy % p->W) + 2 * (int)(xy / p->W);
-                byt[t].push_back((i << WI_PIC_SHIFT) | a);
-            }
+            if (!intra_only && p->desc.disable_deblocking_filter_idc == 1) continue;
+            for (uint32_t a : intra_only ? p->intra_t : p->all_t)
+                byt[(int)(a % p->W) + 2 * (int)(a / p->W)].push_back((i << WI_PIC_SHIFT) | a);
         }
         for (auto &v : byt) outq.insert(outq.end(), v.begin(), v.end());
     };
-    merge(true, false, intra);
-    std::vector<uint32_t> mintra, mpairs;
-    merge(true, true, mintra);
-    merge(false, true, mpairs);
-    bool any_dbk = false;
-    for (uint32_t i = 0; i < n; i++) any_dbk |= !pics[i]->mbaff && pics[i]->desc.disable_deblocking_filter_idc != 1;
-    std::vector<uint32_t> all, rows;
-    if (any_dbk) merge(false, false, all);
+    if (c->intra_schedule != H264G_INTRA_BANDS) merge(true, intra);
+    if (c->dbk_schedule == H264G_DEBLOCK_MB_WAVEFRONT && any_dbk) merge(false, all);
     int maxh = 0;
     for (uint32_t i = 0; i < n; i++) maxh = std::max(maxh, pics[i]->H);
     // bands of R rows of all pictures, band index major: the band above always comes first
@@ -1385,7 +1349,7 @@ int build_sub(h264g_ctx *c, const std::vector<const h264g_pic *> &pics, Batch *b
             }
     };
     std::vector<uint32_t> ibands, dbands;
-    if (!intra.empty()) bands(intra_rows(c), true, ibands);
+    if (b->n_intra) bands(intra_rows(c), true, ibands);
     if (any_dbk) bands(dbk_rows(c), false, dbands);
     if (any_dbk && c->dbk_schedule == H264G_DEBLOCK_MB_ROWS) {
         // MB rows of all pictures, row index major: the row above always comes first.
@@ -1394,45 +1358,42 @@ int build_sub(h264g_ctx *c, const std::vector<const h264g_pic *> &pics, Batch *b
                 if (!pics[i]->mbaff && y < pics[i]->H) rows.push_back((i << WI_PIC_SHIFT) | (uint32_t)y);
     }
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    size_t o_p = 0, o_i = al(n * sizeof(DevPic)), o_a = al(o_i + inter.size() * 4), o_l = al(o_a + intra.size() * 4);
-    size_t o_r = al(o_l + all.size() * 4), o_ib = al(o_r + rows.size() * 4), o_db = al(o_ib + ibands.size() * 4);
-    size_t o_mi = al(o_db + dbands.size() * 4), o_mp = al(o_mi + mintra.size() * 4);
-    size_t total = al(o_mp + mpairs.size() * 4 + 4);
+    // one block: the descriptors, then the lists, uploaded in one copy
+    const size_t o_p = 0, o_c = al(n * sizeof(DevPic)), o_m = al(o_c + chunks.size() * 4), o_i = al(o_m + mchunks.size() * 4);
+    const size_t o_l = al(o_i + intra.size() * 4), o_r = al(o_l + all.size() * 4), o_ib = al(o_r + rows.size() * 4);
+    const size_t o_db = al(o_ib + ibands.size() * 4), total = al(o_db + dbands.size() * 4 + 4);
     b->dmem = pool_get(c, total);
     b->dbytes = total;
     if (!b->dmem) return h264g_set_error(H264G_E_NOMEM, "batch device memory");
     char *base = (char *)b->dmem;
     b->d_pics = (DevPic *)(base + o_p);
     b->n_pics = n;
-    b->d_inter = (uint32_t *)(base + o_i);
-    b->d_intra = (uint32_t *)(base + o_a);
+    b->d_chunks = (uint32_t *)(base + o_c);
+    b->d_mchunks = (uint32_t *)(base + o_m);
+    b->d_intra = (uint32_t *)(base + o_i);
     b->d_all = (uint32_t *)(base + o_l);
     b->d_rows = (uint32_t *)(base + o_r);
     b->d_ibands = (uint32_t *)(base + o_ib);
     b->d_dbands = (uint32_t *)(base + o_db);
-    b->n_inter = n_frame_inter;
-    b->d_minter = b->d_inter + n_frame_inter;
-    b->n_minter = (uint32_t)minter.size();
-    b->n_intra = (uint32_t)intra.size();
+    b->n_chunks = (uint32_t)chunks.size();
+    b->n_mchunks = (uint32_t)mchunks.size();
     b->n_all = (uint32_t)all.size();
     b->n_rows = (uint32_t)rows.size();
     b->n_ibands = (uint32_t)ibands.size();
     b->n_dbands = (uint32_t)dbands.size();
-    b->d_mintra = (uint32_t *)(base + o_mi);
-    b->d_mpairs = (uint32_t *)(base + o_mp);
-    b->n_mintra = (uint32_t)mintra.size();
-    b->n_mpairs = (uint32_t)mpairs.size();
-    b->dbk_off = !any_dbk && mpairs.empty();
+    b->dbk_off = !any_dbk && !any_mdbk;
+    std::vector<char> blob(total, 0);
+    auto put = [&](size_t at, const void *v, size_t bytes) { if (bytes) std::memcpy(&blob[at], v, bytes); };
+    put(o_p, hp.data(), n * sizeof(DevPic));
+    put(o_c, chunks.data(), chunks.size() * 4);
+    put(o_m, mchunks.data(), mchunks.size() * 4);
+    put(o_i, intra.data(), intra.size() * 4);
+    put(o_l, all.data(), all.size() * 4);
+    put(o_r, rows.data(), rows.size() * 4);
+    put(o_ib, ibands.data(), ibands.size() * 4);
+    put(o_db, dbands.data(), dbands.size() * 4);
     for (uint32_t i = 0; i < n; i++) b->scaled |= hp[i].ls != nullptr;
-    if (hipMemcpy(b->d_pics, hp.data(), n * sizeof(DevPic), hipMemcpyHostToDevice) != hipSuccess ||
-        (!inter.empty() && hipMemcpy(b->d_inter, inter.data(), inter.size() * 4, hipMemcpyHostToDevice) != hipSuccess) ||
-        (!intra.empty() && hipMemcpy(b->d_intra, intra.data(), intra.size() * 4, hipMemcpyHostToDevice) != hipSuccess) ||
-        (!all.empty() && hipMemcpy(b->d_all, all.data(), all.size() * 4, hipMemcpyHostToDevice) != hipSuccess) ||
-        (!rows.empty() && hipMemcpy(b->d_rows, rows.data(), rows.size() * 4, hipMemcpyHostToDevice) != hipSuccess) ||
-        (!ibands.empty() && hipMemcpy(b->d_ibands, ibands.data(), ibands.size() * 4, hipMemcpyHostToDevice) != hipSuccess) ||
-        (!dbands.empty() && hipMemcpy(b->d_dbands, dbands.data(), dbands.size() * 4, hipMemcpyHostToDevice) != hipSuccess) ||
-        (!mintra.empty() && hipMemcpy(b->d_mintra, mintra.data(), mintra.size() * 4, hipMemcpyHostToDevice) != hipSuccess) ||
-        (!mpairs.empty() && hipMemcpy(b->d_mpairs, mpairs.data(), mpairs.size() * 4, hipMemcpyHostToDevice) != hipSuccess))
+    if (hipMemcpy(base, blob.data(), total, hipMemcpyHostToDevice) != hipSuccess)
         return h264g_set_error(H264G_E_DEVICE, "batch upload");
     return H264G_OK;
 }
@@ -1487,10 +1448,13 @@ StageSet batch_stages(const Batch *b) {
     StageSet q;
     q.pics = b->d_pics;
     q.n_pics = b->n_pics;
-    q.inter = b->d_inter;
-    q.n_inter = b->n_inter;
+    q.chunks = b->d_chunks;
+    q.n_chunks = b->n_chunks;
+    q.mchunks = b->d_mchunks;
+    q.n_mchunks = b->n_mchunks;
     q.intra = b->d_intra;
     q.n_intra = b->n_intra;
+    q.n_mintra = b->n_mintra;
     q.all = b->d_all;
     q.n_all = b->n_all;
     q.rows = b->d_rows;
@@ -1501,12 +1465,6 @@ StageSet batch_stages(const Batch *b) {
     q.n_dbands = b->n_dbands;
     q.dbk_off = b->dbk_off;
     q.scaled = b->scaled;
-    q.minter = b->d_minter;
-    q.n_minter = b->n_minter;
-    q.mintra = b->d_mintra;
-    q.n_mintra = b->n_mintra;
-    q.mpairs = b->d_mpairs;
-    q.n_mpairs = b->n_mpairs;
     return q;
 }
 }  // namespace

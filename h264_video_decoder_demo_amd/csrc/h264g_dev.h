@@ -117,10 +117,14 @@ struct DevCtl {
 
 extern "C" {
 // Kernel launchers (kernels.hip); all enqueue on `stream` and return a hipError_t.
+// Launches over MBs take them in runs of MB_CHUNK of one picture: chunks[0 .. n) (picture index
+// << 20 | first MB), or null with n runs of picture 0.
+#define MB_CHUNK 64u
 // mbaff: every picture of the launch is an MBAFF frame (else none is).
 // scaled: some picture of the launch has scaling matrices (DevPic::ls).
-int h264g_launch_inter(const DevPic *pics, const uint32_t *items, uint32_t n, const uint32_t *intra_items, uint32_t n_intra,
-                       int mbaff, int scaled, uint32_t *err, void *stream);
+int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, void *stream);
+// Boundary strengths, of pictures that are deblocked.
+int h264g_launch_bs(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, void *stream);
 // `epoch` points at the device word shared by all wavefront launches of a context
 // (initially 1; each launch's last wave advances it).
 int h264g_launch_intra(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
@@ -132,7 +136,8 @@ int h264g_launch_deblock(const DevPic *pics, const uint32_t *items, uint32_t n, 
 int h264g_launch_deblock_rows(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                               uint32_t *err, int waves, void *stream);
 // Two workgroups (luma, chroma) of rows + 1 waves per band of `rows` MB rows, rows at most
-// H264G_INTRA_MAX_ROWS (one row to a SIMD, as for deblocking).
+// H264G_INTRA_MAX_ROWS (one row to a SIMD, as for deblocking).  bands: picture index << 20 |
+// band, or null for n bands of picture 0; so for the deblocking bands.
 #define H264G_INTRA_MAX_ROWS 4
 int h264g_launch_intra_band(const DevPic *pics, const uint32_t *bands, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                             int rows, uint32_t *err, void *stream);
@@ -143,10 +148,7 @@ int h264g_launch_intra_band(const DevPic *pics, const uint32_t *bands, uint32_t 
 #define H264G_DBK_MAX_ROWS 4
 int h264g_launch_deblock_band(const DevPic *pics, const uint32_t *bands, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                               int rows, uint32_t *err, void *stream);
-int h264g_launch_bs(const DevPic *pics, const uint32_t *items, uint32_t n, void *stream);
-// Boundary strengths of the MBAFF frames (pairs: picture index << 20 | pair index), then their
-// deblocking, one workgroup per picture.
-int h264g_launch_bs_mbaff(const DevPic *pics, const uint32_t *pairs, uint32_t n, void *stream);
+// Deblocking of the MBAFF frames among the launch's pictures, one workgroup per picture.
 int h264g_launch_deblock_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *err, void *stream);
 int h264g_launch_bgr24(const uint8_t *yuv, int wl, int hl, uint8_t *bgr, uint32_t stride, int flip, void *stream);
 int h264g_launch_copy(const uint8_t *src, uint8_t *dst, uint64_t bytes, void *stream);

@@ -1706,22 +1706,31 @@ __device__ __forceinline__ uint32_t xcd_item(uint32_t b, uint32_t n) {
     return x * q + min(x, r) + b / N_XCD;
 }
 
-// Workgroups 0 .. n - 1 reconstruct the inter (and I_PCM) MBs of `items`, the following
-// ni build the residuals of the intra MBs of `iitems`.
+// The MBs of a launch's pictures in runs of MB_CHUNK of one picture: run i starts at MB
+// chunks[i] (picture index << 20 | address), or, without a list, at MB i * MB_CHUNK of picture 0.
+// Slot s of the launch is MB s mod MB_CHUNK of run s / MB_CHUNK; a picture's last run may go
+// past its last MB.
+struct MbSlot {
+    uint32_t pic;
+    int addr;
+};
+__device__ __forceinline__ MbSlot mb_slot(const uint32_t *chunks, uint32_t s) {
+    const uint32_t c = s / MB_CHUNK, it = chunks ? chunks[c] : c * MB_CHUNK;
+    return {it >> WI_PIC_SHIFT, (int)((it & WI_MB_MASK) + s % MB_CHUNK)};
+}
+
+// One wave per MB: inter (and I_PCM) MBs are reconstructed, intra MBs get their residual and
+// their entry built for the intra stage.
 // MBAFF: the instance for MBAFF frames (field MBs: geometry, field scans, field references);
 // frame pictures run the instance without any of it.
 template <bool MBAFF, bool SCALED>
-__global__ __launch_bounds__(WAVE) void k_inter(const DevPic *__restrict__ pics, const uint32_t *__restrict__ items, uint32_t n,
-                                                const uint32_t *__restrict__ iitems, uint32_t ni, uint32_t *err) {
+__global__ __launch_bounds__(WAVE) void k_inter(const DevPic *__restrict__ pics, const uint32_t *__restrict__ chunks) {
     __shared__ WaveRes lds;
-    const uint32_t total = n + ni;
-    if (blockIdx.x >= total) return;
-    const uint32_t i = xcd_item(blockIdx.x, total);
-    const uint32_t it = i < n ? items[i] : iitems[i - n];
-    const DevPic &P = pics[it >> WI_PIC_SHIFT];
-    if (i < n) inter_mb<MBAFF, SCALED>(P, (int)(it & WI_MB_MASK), &lds);
-    else intra_res_build<MBAFF, SCALED>(P, (int)(it & WI_MB_MASK), &lds);
-    (void)err;
+    const MbSlot m = mb_slot(chunks, xcd_item(blockIdx.x, gridDim.x));
+    const DevPic &P = pics[m.pic];
+    if (m.addr >= P.W * P.H) return;
+    if (!(uniform(G(P.aux)[m.addr].kind) & AUX_INTRA)) inter_mb<MBAFF, SCALED>(P, m.addr, &lds);
+    else intra_res_build<MBAFF, SCALED>(P, m.addr, &lds);
 }
 
 // Neighbour availability of an intra MB for intra prediction (6.4.11, with
@@ -2387,7 +2396,7 @@ __global__ __launch_bounds__(WAVE *(H264G_INTRA_MAX_ROWS + 1)) void k_intra_band
         __syncthreads();
     }
     if (t < 2 * n) {
-        const uint32_t it = items[t >> 1];
+        const uint32_t it = items ? items[t >> 1] : t >> 1;
         const DevPic &P = pics[it >> WI_PIC_SHIFT];
         const int band = (int)(it & WI_MB_MASK), y0 = band * rows, y = y0 + w, y1 = min(P.H, y0 + rows);
         if (P.n_intra != 0) {
@@ -2550,12 +2559,11 @@ __device__ __forceinline__ MbaffNb mbaff_nb(int W, int addr, bool field, bool lf
 // k_bs, with its field flag.
 constexpr int MBS_LEFT = 0, MBS_LEFT_C = 16, MBS_V = 24, MBS_TOP = 36, MBS_TOP_C = 40, MBS_TOP2 = 44, MBS_TOP2_C = 48, MBS_H = 52;
 constexpr uint32_t DBQ_FIELD = 1u << 27;
-__global__ __launch_bounds__(WAVE) void k_bs_mbaff(const DevPic *__restrict__ pics, const uint32_t *__restrict__ items, uint32_t n) {
-    const uint32_t i = blockIdx.x >> 1;
-    if (i >= n) return;
-    const uint32_t it = items[i];
-    const DevPic &P = pics[it >> WI_PIC_SHIFT];
-    const int pair = (int)(it & WI_MB_MASK), addr = 2 * pair + (int)(blockIdx.x & 1u), W = P.W, px = pair % W, py = pair / W;
+__global__ __launch_bounds__(WAVE) void k_bs_mbaff(const DevPic *__restrict__ pics, const uint32_t *__restrict__ chunks) {
+    const MbSlot m = mb_slot(chunks, xcd_item(blockIdx.x, gridDim.x));
+    const DevPic &P = pics[m.pic];
+    const int addr = m.addr, pair = addr >> 1, W = P.W, px = pair % W, py = pair / W;
+    if (addr >= W * P.H || P.dbk_idc == 1) return;
     const int l = wave_lane();
     const DevAux &ax = G(P.aux)[addr];
     const MbaffNb nb = mbaff_nb(W, addr, (G(P.mbs)[addr].flags & H264G_MBF_FIELD) != 0,
@@ -3313,7 +3321,7 @@ __global__ __launch_bounds__(WAVE *(DBK_MAX_ROWS + 1)) void k_deblock_band(const
     dbk_lut_init(&sh.lut);
     const uint32_t t = band_ticket(ctl, &s_ticket, sh.prog, rows + 1);
     if (t < 2 * n) {
-        const uint32_t it = items[t >> 1];
+        const uint32_t it = items ? items[t >> 1] : t >> 1;
         const DevPic &P = pics[it >> WI_PIC_SHIFT];
         const int b = (int)(it & WI_MB_MASK), y0 = b * rows, y1 = min(P.H, y0 + rows);
         const GAS StripWords *const above = (const GAS StripWords *)G(P.gstrip) + (size_t)(b > 0 ? b - 1 : 0) * P.W;
@@ -3341,14 +3349,14 @@ __global__ __launch_bounds__(WAVE *(DBK_MAX_ROWS + 1)) void k_deblock_band(const
 // as one dword, and each MB's deblocking word (G(P.dbq): qP of luma / Cb edges / Cr edges in
 // bytes 0..2, transform_size_8x8_flag in bit 24, the own-qP flags of its MB edges in bits
 // 25 / 26); fully parallel: they depend on syntax
-// only, not on samples.  Half a wave per MB; lane j = 16 * dir + 4 * edge + segment.
-__global__ __launch_bounds__(WAVE) void k_bs(const DevPic *__restrict__ pics, const uint32_t *__restrict__ items, uint32_t n) {
+// only, not on samples.  Half a wave per MB (neighbouring MBs, so that an XCD's L2 serves the
+// records two MBs share); lane j = 16 * dir + 4 * edge + segment.
+__global__ __launch_bounds__(WAVE) void k_bs(const DevPic *__restrict__ pics, const uint32_t *__restrict__ chunks) {
     const int lane = wave_lane();
-    const uint32_t i = blockIdx.x * 2 + (lane >> 5);
-    if (i >= n) return;
-    const uint32_t it = items[i];
-    const DevPic &P = pics[it >> WI_PIC_SHIFT];
-    const int addr = (int)(it & WI_MB_MASK), W = P.W, mbx = addr % W, mby = addr / W;
+    const MbSlot m = mb_slot(chunks, 2 * xcd_item(blockIdx.x, gridDim.x));
+    const DevPic &P = pics[m.pic];
+    const int addr = m.addr + (lane >> 5), W = P.W, mbx = addr % W, mby = addr / W;
+    if (addr >= W * P.H || P.dbk_idc == 1) return;
     const int j = lane & 31, dir = j >> 4, e = ((j >> 2) & 3) * 4, k = (j & 3) * 4;
     int bS = 0;
     const bool has_nb = dir == 0 ? mbx > 0 : mby > 0;
@@ -3416,18 +3424,15 @@ __global__ void k_copy(const uint4 *src, uint4 *dst, uint64_t n16) {
 
 extern "C" {
 
-int h264g_launch_inter(const DevPic *pics, const uint32_t *items, uint32_t n, const uint32_t *intra_items, uint32_t n_intra,
-                       int mbaff, int scaled, uint32_t *err, void *stream) {
-    if (n + n_intra == 0) return 0;
+int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, void *stream) {
+    if (n == 0) return 0;
+    const dim3 grid(n * MB_CHUNK), block(WAVE);
     if (mbaff)  // (scaling matrices are refused in MBAFF frames)
-        hipLaunchKernelGGL((k_inter<true, false>), dim3(n + n_intra), dim3(WAVE), 0, (hipStream_t)stream, pics, items, n,
-                           intra_items, n_intra, err);
+        hipLaunchKernelGGL((k_inter<true, false>), grid, block, 0, (hipStream_t)stream, pics, chunks);
     else if (scaled)
-        hipLaunchKernelGGL((k_inter<false, true>), dim3(n + n_intra), dim3(WAVE), 0, (hipStream_t)stream, pics, items, n,
-                           intra_items, n_intra, err);
+        hipLaunchKernelGGL((k_inter<false, true>), grid, block, 0, (hipStream_t)stream, pics, chunks);
     else
-        hipLaunchKernelGGL((k_inter<false, false>), dim3(n + n_intra), dim3(WAVE), 0, (hipStream_t)stream, pics, items, n,
-                           intra_items, n_intra, err);
+        hipLaunchKernelGGL((k_inter<false, false>), grid, block, 0, (hipStream_t)stream, pics, chunks);
     return (int)hipGetLastError();
 }
 
@@ -3485,15 +3490,10 @@ int h264g_launch_deblock_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *er
     return (int)hipGetLastError();
 }
 
-int h264g_launch_bs_mbaff(const DevPic *pics, const uint32_t *pairs, uint32_t n, void *stream) {
+int h264g_launch_bs(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, void *stream) {
     if (n == 0) return 0;
-    hipLaunchKernelGGL(k_bs_mbaff, dim3(2 * n), dim3(WAVE), 0, (hipStream_t)stream, pics, pairs, n);
-    return (int)hipGetLastError();
-}
-
-int h264g_launch_bs(const DevPic *pics, const uint32_t *items, uint32_t n, void *stream) {
-    if (n == 0) return 0;
-    hipLaunchKernelGGL(k_bs, dim3((n + 1) / 2), dim3(WAVE), 0, (hipStream_t)stream, pics, items, n);
+    if (mbaff) hipLaunchKernelGGL(k_bs_mbaff, dim3(n * MB_CHUNK), dim3(WAVE), 0, (hipStream_t)stream, pics, chunks);
+    else hipLaunchKernelGGL(k_bs, dim3(n * (MB_CHUNK / 2)), dim3(WAVE), 0, (hipStream_t)stream, pics, chunks);
     return (int)hipGetLastError();
 }
 
