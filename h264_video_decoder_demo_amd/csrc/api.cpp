@@ -192,6 +192,13 @@ struct h264g_ctx {
     int intra_schedule = H264G_INTRA_BANDS;
     int intra_waves = 8;           // rows per band (waves per workgroup) of the intra band schedule
     int dbk_waves = 8;             // configured MB rows per band of the deblocking band schedule (run: dbk_rows)
+    // One staging call at a time uses a slot: a stream and pinned memory for its small uploads
+    // and its result.  Slots are made when all are in use (one with the context) and kept.
+    struct StageSlot {
+        hipStream_t s = nullptr;
+        uint8_t *pin = nullptr;
+    };
+    std::vector<StageSlot> slots;  // free ones
     std::vector<hipEvent_t> ev;    // 6 events per profiled run: inter | intra | bS | end (lane), deblock | end
     size_t ev_used = 0;            // events recorded since the last h264g_stage_times
     std::mutex mu;
@@ -403,6 +410,219 @@ int partitions(const h264g_mb &m, int out[16][4]) {
     return n;
 }
 
+// Where the parts of a picture's device block lie: records | levels | weights | LevelScale
+// tables | descriptor (and StageResult) | lists (what is uploaded, together) | DevAux | bS |
+// deblocking words | intra residuals | MBAFF picture identities | IMETA entries.
+struct StageLayout {
+    size_t o_mbs, o_lv, o_wt, o_ls, o_pic, o_it, o_aux, o_bs, o_dbq, o_ires, o_bsref, o_imeta;
+    size_t counted;  // the bytes that count against a fixed block, which holds the IMETA entries
+                     // beyond them (H264G_SCRATCH_IMETA); lists count in full: inter and intra
+                     // MBs, all MBs or MB pairs, rows, intra MBs per row
+    size_t total;
+};
+StageLayout stage_layout(uint32_t n_mbs, int H, uint64_t n_levels, size_t n_wt, uint32_t n_intra, bool mbaff, size_t ls_entries) {
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    StageLayout l;
+    const size_t n_items = (size_t)n_mbs + (mbaff ? n_mbs / 2 : n_mbs + (uint32_t)H) + (size_t)H + 1 + (mbaff ? 0 : n_intra);
+    l.o_mbs = 0;
+    l.o_lv = al(n_mbs * sizeof(h264g_mb));
+    l.o_wt = al(l.o_lv + n_levels * sizeof(int16_t) + 16);
+    l.o_ls = al(l.o_wt + n_wt * sizeof(DevWeight));
+    l.o_pic = al(l.o_ls + ls_entries * sizeof(uint16_t));
+    l.o_it = al(l.o_pic + sizeof(DevPic));
+    l.o_aux = al(l.o_it + n_items * sizeof(uint32_t));
+    l.o_bs = al(l.o_aux + n_mbs * sizeof(DevAux));
+    l.o_dbq = al(l.o_bs + (size_t)n_mbs * 32);
+    l.o_ires = al(l.o_dbq + (size_t)n_mbs * 4);
+    l.o_bsref = al(l.o_ires + (size_t)n_intra * 768);
+    l.counted = al(l.o_bsref + (mbaff ? (size_t)n_mbs * 8 : 0));
+    l.o_imeta = l.counted;
+    l.total = al(l.o_imeta + (mbaff ? 0 : (size_t)n_intra * 16));
+    return l;
+}
+
+// The descriptor of a picture staged at `base` (all but the slice fields, the lists' place and
+// the MBAFF parts).
+void fill_devpic(const Stream &st, const h264g_pic_desc &d, char *base, const StageLayout &l, uint32_t n_intra, bool ls, h264g_pic *pic) {
+    pic->d_mbs = (h264g_mb *)(base + l.o_mbs);
+    pic->d_aux = (DevAux *)(base + l.o_aux);
+    pic->d_levels = (int16_t *)(base + l.o_lv);
+    pic->d_wt = (DevWeight *)(base + l.o_wt);
+    pic->d_items = (uint32_t *)(base + l.o_it);
+    pic->d_pic = (DevPic *)(base + l.o_pic);
+    DevPic &P = pic->hpic;
+    std::memset(&P, 0, sizeof(P));
+    P.mbs = pic->d_mbs; P.aux = pic->d_aux; P.levels = pic->d_levels; P.wt = pic->d_wt;
+    P.dpb = st.dpb; P.slot_bytes = st.slot_bytes; P.dst = d.dst_slot;
+    P.bs = (uint8_t *)(base + l.o_bs); P.dbq = (uint32_t *)(base + l.o_dbq);
+    P.ires = (int16_t *)(base + l.o_ires);
+    P.imeta = (uint32_t *)(base + l.o_imeta);
+    P.n_intra = n_intra;
+    P.W = st.W; P.H = st.H; P.offA = d.filter_offset_a; P.offB = d.filter_offset_b;
+    use_set(st, 0, P);
+    P.dbk_idc = d.disable_deblocking_filter_idc; P.cip = d.constrained_intra_pred_flag;
+    P.ls = ls ? (const uint16_t *)(base + l.o_ls) : nullptr;
+}
+
+constexpr size_t kSlotPin = 1 << 20;            // pinned bytes of a staging slot
+constexpr size_t kSlotResult = kSlotPin - 256;  // where the result comes back
+
+bool make_slot(h264g_ctx::StageSlot &sl) {
+    return hipStreamCreateWithFlags(&sl.s, hipStreamNonBlocking) == hipSuccess &&
+           hipHostMalloc((void **)&sl.pin, kSlotPin, hipHostMallocDefault) == hipSuccess;
+}
+void free_slot(h264g_ctx::StageSlot &sl) {
+    if (sl.s) {
+        (void)hipStreamSynchronize(sl.s);
+        (void)hipStreamDestroy(sl.s);
+    }
+    if (sl.pin) (void)hipHostFree(sl.pin);
+    sl = h264g_ctx::StageSlot();
+}
+
+// Staging of a frame picture on the device: records and levels go up as they are, k_stage
+// validates them and derives the DevAux and ICOL entries; the host only counts the intra MBs
+// of each row.  Returns 0 when the picture is staged, 1 when the host has to stage it: a
+// schedule that walks lists of MBs, more weight entries than a byte names, a block at the
+// limit of a fixed one, or a record that breaks a rule (the host's pass names it).  The
+// calls for a CIF and a 1920x1088 B picture took 245 and 1760 us on the host, 50 and 185 us
+// this way (most of it the copies).
+int stage_on_device(h264g_ctx *ctx, const Stream &st, const h264g_pic_desc &d, const h264g_mb *mbs, uint32_t n_mbs,
+                    const int16_t *levels, uint64_t n_levels, const std::vector<uint16_t> &lsv, h264g_pic *pic, void *fixed,
+                    size_t fixed_cap) {
+    if (ctx->intra_schedule != H264G_INTRA_BANDS || ctx->dbk_schedule != H264G_DEBLOCK_BANDS) return 1;
+    const int W = st.W, H = st.H;
+    const int n0 = d.slice_type == H264G_SLICE_I ? 0 : d.num_ref_idx_active[0], n1 = d.slice_type == H264G_SLICE_B ? d.num_ref_idx_active[1] : 0;
+    const size_t n_wt = (size_t)(n0 + 1) * (n1 + 1);
+    if (n_wt > 255) return 1;
+    // ---- every weight entry a record could name
+    StageIn in;
+    std::memset(&in, 0, sizeof(in));
+    std::vector<DevWeight> wt(n_wt);
+    std::memset(wt.data(), 0, n_wt * sizeof(DevWeight));
+    for (int r0 = -1; r0 < n0; r0++)
+        for (int r1 = -1; r1 < n1; r1++) {
+            const size_t e = (size_t)(r0 + 1) * (n1 + 1) + (size_t)(r1 + 1);
+            if (e && derive_weight(d, r0, r1, wt[e])) in.bad_weight[e >> 5] |= 1u << (e & 31);
+        }
+    // ---- intra MBs before each row, slice of the first MB that has one
+    std::vector<uint32_t> irow(H + 1);
+    uint32_t n_intra = 0;
+    for (int y = 0; y < H; y++) {
+        irow[y] = n_intra;
+        const h264g_mb *const row = mbs + (size_t)y * W;
+        uint32_t k = 0;
+        for (int x = 0; x < W; x++) k += cls_intra(row[x].mb_type);
+        n_intra += k;
+    }
+    irow[H] = n_intra;
+    in.first_sn = H264G_SLICE_NONE;
+    for (uint32_t a = 0; a < n_mbs && in.first_sn == H264G_SLICE_NONE; a++) in.first_sn = mbs[a].slice_num;
+    const StageLayout l = stage_layout(n_mbs, H, n_levels, n_wt, n_intra, false, lsv.size());
+    // Weights, tables, descriptor and row offsets are put together in the slot's pinned memory
+    // and go up in one copy; so do the records and levels of a picture that fits there (a CIF
+    // picture: one copy instead of three from pageable memory).
+    const size_t up_end = l.o_it + irow.size() * sizeof(uint32_t);
+    const bool whole = up_end <= kSlotResult;
+    const size_t up_at = whole ? 0 : l.o_wt;
+    if (up_end - up_at > kSlotResult) return 1;
+    char *base = (char *)fixed;
+    h264g_ctx::StageSlot sl;
+    {
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        if (!fixed) {
+            base = (char *)pool_get(ctx, l.total);
+            if (!base) return h264g_set_error(H264G_E_NOMEM, "picture device memory (%zu bytes)", l.total);
+            pic->dmem = base;
+            pic->dbytes = l.total;
+        } else if (l.counted > fixed_cap) {
+            return 1;
+        }
+        if (!ctx->slots.empty()) {
+            sl = ctx->slots.back();
+            ctx->slots.pop_back();
+        } else if (fixed) {
+            return 1;  // a fixed block is staged without allocating
+        }
+    }
+    if (!sl.s && !make_slot(sl)) {
+        free_slot(sl);
+        return h264g_set_error(H264G_E_DEVICE, "staging stream");
+    }
+    fill_devpic(st, d, base, l, n_intra, !lsv.empty(), pic);
+    DevPic &P = pic->hpic;
+    P.irow = pic->d_items;
+    P.dbk_stop = n_mbs;
+    in.mbs = pic->d_mbs;
+    in.levels = pic->d_levels;
+    in.n_levels = n_levels;
+    in.aux = pic->d_aux;
+    in.irow = pic->d_items;
+    in.icol = pic->d_items + H + 1;
+    in.res = (StageResult *)(base + l.o_pic + STAGE_RESULT_AT);
+    in.W = W;
+    in.H = H;
+    in.slice_type = d.slice_type;
+    in.cip = d.constrained_intra_pred_flag ? 1 : 0;
+    in.cqo[0] = d.chroma_qp_index_offset;
+    in.cqo[1] = d.second_chroma_qp_index_offset;
+    in.n1 = n1 + 1;
+    for (int k = 0; k < 2; k++) {
+        in.nref[k] = d.num_ref_idx_active[k];
+        for (int r = 0; r < 32; r++) in.ref_slot[k][r] = (int8_t)(r < d.num_ref_idx_active[k] ? d.ref_slot[k][r] : -1);
+    }
+    const auto up = [&](size_t o) { return sl.pin + (o - up_at); };  // what goes to base + o
+    std::memset(up(l.o_wt), 0, up_end - l.o_wt);
+    std::memcpy(up(l.o_wt), wt.data(), n_wt * sizeof(DevWeight));
+    if (!lsv.empty()) std::memcpy(up(l.o_ls), lsv.data(), lsv.size() * sizeof(uint16_t));
+    std::memcpy(up(l.o_pic), &P, sizeof(P));
+    StageResult res{~0u, n_mbs, 0u, 0u, {0, 0, 0}};
+    std::memcpy(up(l.o_pic) + STAGE_RESULT_AT, &res, sizeof(res));
+    std::memcpy(up(l.o_it), irow.data(), irow.size() * sizeof(uint32_t));
+    if (whole) {
+        std::memcpy(up(l.o_mbs), mbs, n_mbs * sizeof(h264g_mb));
+        if (n_levels) std::memcpy(up(l.o_lv), levels, n_levels * sizeof(int16_t));
+    }
+    auto run = [&]() -> int {
+        if (!whole) {
+            HIPCHK(hipMemcpyAsync(pic->d_mbs, mbs, n_mbs * sizeof(h264g_mb), hipMemcpyHostToDevice, sl.s));
+            if (n_levels) HIPCHK(hipMemcpyAsync(pic->d_levels, levels, n_levels * sizeof(int16_t), hipMemcpyHostToDevice, sl.s));
+        }
+        HIPCHK(hipMemcpyAsync(base + up_at, up(up_at), up_end - up_at, hipMemcpyHostToDevice, sl.s));
+        if (int e = h264g_launch_stage(&in, sl.s)) return h264g_set_error(H264G_E_DEVICE, "staging launch: %s", hipGetErrorString((hipError_t)e));
+        HIPCHK(hipMemcpyAsync(sl.pin + kSlotResult, in.res, sizeof(StageResult), hipMemcpyDeviceToHost, sl.s));
+        HIPCHK(hipStreamSynchronize(sl.s));
+        std::memcpy(&res, sl.pin + kSlotResult, sizeof(res));
+        if (res.err_mb != ~0u) return 1;
+        P.dbk_stop = res.dbk_stop;
+        P.multi_slice = res.multi_slice ? 1 : 0;
+        if (res.dbk_stop != n_mbs || res.multi_slice) {  // k_stage's findings into the descriptor
+            std::memcpy(up(l.o_pic), &P, sizeof(P));
+            HIPCHK(hipMemcpyAsync(pic->d_pic, up(l.o_pic), sizeof(P), hipMemcpyHostToDevice, sl.s));
+            HIPCHK(hipStreamSynchronize(sl.s));
+        }
+        return 0;
+    };
+    const int rc = run();
+    if (rc) (void)hipStreamSynchronize(sl.s);  // nothing reads the caller's arrays or the block any more
+    {
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        ctx->slots.push_back(sl);
+        if (rc > 0 && !fixed) {
+            pool_put(ctx, pic->dmem, pic->dbytes);
+            pic->dmem = nullptr;
+            pic->dbytes = 0;
+        }
+    }
+    if (rc) return rc;
+    pic->mbaff = false;
+    pic->n_intra = n_intra;
+    pic->alg[0] = res.alg[0];
+    pic->alg[1] = res.alg[1];
+    pic->alg[2] = 2ull * 384 * n_mbs + 8ull * n_mbs + 5 * res.alg[2] + 4ull * n_mbs;
+    return 0;
+}
+
 // Validates and stages one picture.  Its device block comes from the context's pool, or,
 // when `fixed` is given, is the caller's block of `fixed_cap` bytes (pictures that need
 // more are refused).
@@ -434,23 +654,6 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
     if (d.disable_deblocking_filter_idc < 0 || d.disable_deblocking_filter_idc > 2 || d.filter_offset_a < -12 || d.filter_offset_a > 12 ||
         d.filter_offset_b < -12 || d.filter_offset_b > 12)
         return h264g_set_error(H264G_E_ARG, "deblocking parameters");
-    // Slices.  Deblocking stops at the first MB of no slice (H264G_SLICE_NONE), where the
-    // reference's bS derivation fails on the MB's reset type and the failure is ignored
-    // (H264InterPrediction.cpp:3182-3186, H264PictureBase.cpp:707-708).  MBAFF frames take
-    // one slice.
-    uint32_t dbk_stop = n_mbs, first_sn = H264G_SLICE_NONE;
-    bool multi_slice = false;
-    for (uint32_t a = 0; a < n_mbs; a++) {
-        const uint32_t sn = mbs[a].slice_num;
-        if (sn == H264G_SLICE_NONE) {
-            if (mbaff) return h264g_set_error(H264G_E_ARG, "mb %u: MBs of no slice in an MBAFF frame", a);
-            if (dbk_stop == n_mbs) dbk_stop = a;
-            continue;
-        }
-        if (first_sn == H264G_SLICE_NONE) first_sn = sn;
-        if (sn != first_sn && mbaff) return h264g_set_error(H264G_E_ARG, "mb %u: several slices in an MBAFF frame", a);
-        multi_slice |= sn != first_sn;
-    }
     // Scaling matrices: LevelScale4x4 / 8x8 (8-315 / 8-318) of the two luma lists the
     // reference dequantises with (chroma takes the MB's luma list, quirk Q13).
     std::vector<uint16_t> lsv;
@@ -475,6 +678,27 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
                     lsv[LS8_AT + l * LS8_LIST + m * 64 + k] = (uint16_t)(d.weight_scale8x8[l][k] * v8[m][c]);
                 }
             }
+    }
+    if (!mbaff) {
+        const int rc = stage_on_device(ctx, st, d, mbs, n_mbs, levels, n_levels, lsv, pic, fixed, fixed_cap);
+        if (rc <= 0) return rc;
+    }
+    // Slices.  Deblocking stops at the first MB of no slice (H264G_SLICE_NONE), where the
+    // reference's bS derivation fails on the MB's reset type and the failure is ignored
+    // (H264InterPrediction.cpp:3182-3186, H264PictureBase.cpp:707-708).  MBAFF frames take
+    // one slice.
+    uint32_t dbk_stop = n_mbs, first_sn = H264G_SLICE_NONE;
+    bool multi_slice = false;
+    for (uint32_t a = 0; a < n_mbs; a++) {
+        const uint32_t sn = mbs[a].slice_num;
+        if (sn == H264G_SLICE_NONE) {
+            if (mbaff) return h264g_set_error(H264G_E_ARG, "mb %u: MBs of no slice in an MBAFF frame", a);
+            if (dbk_stop == n_mbs) dbk_stop = a;
+            continue;
+        }
+        if (first_sn == H264G_SLICE_NONE) first_sn = sn;
+        if (sn != first_sn && mbaff) return h264g_set_error(H264G_E_ARG, "mb %u: several slices in an MBAFF frame", a);
+        multi_slice |= sn != first_sn;
     }
     std::vector<DevAux> aux(n_mbs);
     std::vector<int8_t> bsref(mbaff ? (size_t)n_mbs * 8 : 0, (int8_t)-1);
@@ -682,10 +906,6 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
     // deblocking: one read and one write of the picture, the bS inputs (motion records,
     // 8 bytes per MB and 5 per partition-list) and 4 bytes of non-zero / QP bits per MB
     pic->alg[2] = 2ull * 384 * n_mbs + 8ull * n_mbs + 5 * n_part_lists + 4ull * n_mbs;
-    // ---- device block: mbs | aux | levels | weights | items | pic
-    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    size_t o_mbs = 0, o_aux = al(o_mbs + n_mbs * sizeof(h264g_mb)), o_lv = al(o_aux + n_mbs * sizeof(DevAux));
-    size_t o_wt = al(o_lv + n_levels * sizeof(int16_t) + 16), o_it = al(o_wt + wt.size() * sizeof(DevWeight));
     // intra MBs per row: offsets, then one entry per intra MB (the per-picture intra band
     // schedule; an MB's residual sits at its entry's index in P.ires).  The entry carries
     // what the band kernel would otherwise load from the neighbours' records before its
@@ -723,66 +943,41 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
     }
     irow[H] = (uint32_t)icol.size();
     const uint32_t n_rows = !mbaff && ctx->dbk_schedule == H264G_DEBLOCK_MB_ROWS ? (uint32_t)H : 0u;
-    // (the bytes counted against a fixed block are those of full lists: inter and intra MBs, all
-    // MBs or MB pairs, rows, intra MBs per row)
-    size_t n_items = (size_t)n_mbs + (mbaff ? n_mbs / 2 : n_mbs + (uint32_t)H) + irow.size() + icol.size();
-    size_t o_bs = al(o_it + n_items * sizeof(uint32_t)), o_dbq = al(o_bs + (size_t)n_mbs * 32);
-    size_t o_ires = al(o_dbq + (size_t)n_mbs * 4), o_bsref = al(o_ires + (size_t)pic->n_intra * 768);
-    size_t o_ls = al(o_bsref + bsref.size()), o_pic = al(o_ls + lsv.size() * sizeof(uint16_t));
-    size_t counted = al(o_pic + sizeof(DevPic));
-    // IMETA entries, which a fixed block holds beyond its counted bytes (H264G_SCRATCH_IMETA)
-    size_t o_imeta = counted, total = al(o_imeta + (mbaff ? 0 : (size_t)pic->n_intra * 16));
+    const StageLayout l = stage_layout(n_mbs, H, n_levels, wt.size(), pic->n_intra, mbaff, lsv.size());
     void *dm = fixed;
     if (fixed) {
-        if (counted > fixed_cap)
+        if (l.counted > fixed_cap)
             return h264g_set_error(H264G_E_ARG, "picture needs %zu bytes of device staging, the fixed block holds %zu",
-                                   counted, fixed_cap);
+                                   l.counted, fixed_cap);
     } else {
         std::lock_guard<std::mutex> lk(ctx->mu);  // the rest of the staging runs unlocked
-        dm = pool_get(ctx, total);
-        if (!dm) return h264g_set_error(H264G_E_NOMEM, "picture device memory (%zu bytes)", total);
+        dm = pool_get(ctx, l.total);
+        if (!dm) return h264g_set_error(H264G_E_NOMEM, "picture device memory (%zu bytes)", l.total);
         pic->dmem = dm;
-        pic->dbytes = total;
+        pic->dbytes = l.total;
     }
     char *base = (char *)dm;
-    pic->d_mbs = (h264g_mb *)(base + o_mbs);
-    pic->d_aux = (DevAux *)(base + o_aux);
-    pic->d_levels = (int16_t *)(base + o_lv);
-    pic->d_wt = (DevWeight *)(base + o_wt);
-    pic->d_items = (uint32_t *)(base + o_it);
-    pic->d_pic = (DevPic *)(base + o_pic);
-    uint8_t *d_bs = (uint8_t *)(base + o_bs);
-    uint32_t *d_dbq = (uint32_t *)(base + o_dbq);
     std::vector<uint32_t> items;
-    items.reserve(n_items);
     items.insert(items.end(), pic->intra_t.begin(), pic->intra_t.end());
     items.insert(items.end(), pic->all_t.begin(), pic->all_t.end());
     for (uint32_t y = 0; y < n_rows; y++) items.push_back(y);
     const size_t irow_at = items.size();
     items.insert(items.end(), irow.begin(), irow.end());
     items.insert(items.end(), icol.begin(), icol.end());
+    fill_devpic(st, d, base, l, pic->n_intra, !lsv.empty(), pic);
     DevPic &P = pic->hpic;
-    std::memset(&P, 0, sizeof(P));
-    P.mbs = pic->d_mbs; P.aux = pic->d_aux; P.levels = pic->d_levels; P.wt = pic->d_wt;
-    P.dpb = st.dpb; P.slot_bytes = st.slot_bytes; P.bs = d_bs; P.dbq = d_dbq; P.dst = d.dst_slot;
-    P.ires = (int16_t *)(base + o_ires);
-    P.imeta = (uint32_t *)(base + o_imeta);
-    P.irow = pic->d_items + irow_at; P.n_intra = pic->n_intra;
-    P.W = W; P.H = H; P.offA = d.filter_offset_a; P.offB = d.filter_offset_b;
+    P.irow = pic->d_items + irow_at;
     P.mbaff = mbaff ? 1 : 0;
-    P.bsref = mbaff ? (const int8_t *)(base + o_bsref) : nullptr;
-    use_set(st, 0, P);
-    P.dbk_idc = d.disable_deblocking_filter_idc; P.cip = d.constrained_intra_pred_flag;
+    P.bsref = mbaff ? (const int8_t *)(base + l.o_bsref) : nullptr;
     P.dbk_stop = dbk_stop;
     P.multi_slice = multi_slice ? 1 : 0;
-    P.ls = lsv.empty() ? nullptr : (const uint16_t *)(base + o_ls);
     HIPCHK(hipMemcpy(pic->d_mbs, mbs, n_mbs * sizeof(h264g_mb), hipMemcpyHostToDevice));
-    if (!lsv.empty()) HIPCHK(hipMemcpy(base + o_ls, lsv.data(), lsv.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+    if (!lsv.empty()) HIPCHK(hipMemcpy(base + l.o_ls, lsv.data(), lsv.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(pic->d_aux, aux.data(), n_mbs * sizeof(DevAux), hipMemcpyHostToDevice));
     if (n_levels) HIPCHK(hipMemcpy(pic->d_levels, levels, n_levels * sizeof(int16_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(pic->d_wt, wt.data(), wt.size() * sizeof(DevWeight), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(pic->d_items, items.data(), items.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-    if (mbaff) HIPCHK(hipMemcpy(base + o_bsref, bsref.data(), bsref.size(), hipMemcpyHostToDevice));
+    if (mbaff) HIPCHK(hipMemcpy(base + l.o_bsref, bsref.data(), bsref.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(pic->d_pic, &P, sizeof(DevPic), hipMemcpyHostToDevice));
     return 0;
 }
@@ -1025,6 +1220,13 @@ int32_t h264g_create(const h264g_config *cfg, h264g_ctx **out) {
         h264g_destroy(c);
         return h264g_set_error(H264G_E_DEVICE, "context allocation failed");
     }
+    h264g_ctx::StageSlot sl;
+    const bool have_slot = make_slot(sl);
+    c->slots.push_back(sl);
+    if (!have_slot) {
+        h264g_destroy(c);
+        return h264g_set_error(H264G_E_DEVICE, "staging stream");
+    }
     // events of the deblocking history, so that enqueuing creates none
     for (auto &lane : c->hist)
         for (auto &r : lane)
@@ -1041,6 +1243,7 @@ int32_t h264g_destroy(h264g_ctx *c) {
     (void)hipSetDevice(c->device);
     for (int i = 0; i < 4; i++)
         if (any_stream(c, i)) (void)hipStreamSynchronize(any_stream(c, i));
+    for (auto &sl : c->slots) free_slot(sl);
     for (auto &b : c->pool) {
         for (auto ev : b.ready) (void)hipEventDestroy(ev);
         (void)hipFree(b.ptr);

@@ -99,7 +99,37 @@ struct DevPic {
 #define LS8_LIST 384          // entries per 8x8 list (6 x 64)
 #define LS_ENTRIES 960
 
-static_assert(sizeof(DevPic) <= 256, "DevPic fits the 256 bytes that staging counts for it");
+// What k_stage finds about a picture besides its DevAux records; initialised by the host.
+struct StageResult {
+    uint32_t err_mb;          // the first MB that breaks a rule of staging (~0: none)
+    uint32_t dbk_stop;        // the first MB of no slice (initially W * H)
+    uint32_t multi_slice;     // some MB's slice differs from StageIn::first_sn
+    uint32_t pad;
+    unsigned long long alg[3];  // algorithmic bytes: inter, intra, (partition, list) pairs
+};
+// A picture's DevPic and StageResult stand in the 256 bytes that staging counts for it.
+constexpr size_t STAGE_RESULT_AT = 200;
+static_assert(sizeof(DevPic) <= STAGE_RESULT_AT && STAGE_RESULT_AT + sizeof(StageResult) <= 256, "descriptor and result");
+
+// Arguments of k_stage: a frame picture's records and levels in device memory, and what its
+// descriptor says about them.
+struct StageIn {
+    const h264g_mb *mbs;
+    const int16_t *levels;
+    uint64_t n_levels;
+    DevAux *aux;
+    const uint32_t *irow;     // intra MBs before each row
+    uint32_t *icol;           // their ICOL entries, from irow[y] on
+    StageResult *res;
+    int32_t W, H;
+    int32_t slice_type, cip;
+    int32_t cqo[2];           // chroma_qp_index_offset, second_chroma_qp_index_offset
+    int32_t nref[2];          // num_ref_idx_active
+    int32_t n1;               // weight entry of (refIdxL0, refIdxL1): (r0 + 1) * n1 + r1 + 1
+    uint32_t first_sn;        // slice of the first MB that has one
+    int8_t ref_slot[2][32];
+    uint32_t bad_weight[8];   // entries whose weights the reference rejects
+};
 
 // Work item: picture index in the batch and macroblock address.
 #define WI_PIC_SHIFT 20u
@@ -117,6 +147,8 @@ struct DevCtl {
 
 extern "C" {
 // Kernel launchers (kernels.hip); all enqueue on `stream` and return a hipError_t.
+// Validates a frame picture's records and derives their DevAux and ICOL entries.
+int h264g_launch_stage(const StageIn *in, void *stream);
 // Launches over MBs take them in runs of MB_CHUNK of one picture: chunks[0 .. n) (picture index
 // << 20 | first MB), or null with n runs of picture 0.
 #define MB_CHUNK 64u

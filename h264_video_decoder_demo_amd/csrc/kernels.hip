@@ -3391,6 +3391,255 @@ __global__ __launch_bounds__(WAVE) void k_bs(const DevPic *__restrict__ pics, co
     }
 }
 
+// ------------------------------------------------------------ staging
+// Validation of a frame picture's syntax records and the per-MB values the other kernels read
+// (DevAux, ICOL), a lane per MB, 64 MBs of a row per wave.  The rules are those of the host's
+// staging (stage_picture in api.cpp), which decides what an error is called: this kernel only
+// names the first MB that breaks one.  Bound: one pass over the records and masks, latency of
+// a few dependent loads (record, masks, neighbours' records); the host's pass took 1.6 ms for
+// a 1920x1088 B picture.
+__constant__ uint8_t c_cqp[22] = {29, 30, 31, 32, 32, 33, 34, 34, 35, 35, 36, 36, 37, 37, 37, 38, 38, 38, 39, 39, 39, 39};
+__device__ __forceinline__ uint32_t stage_chroma_qp(int qp, int off) {  // 8.5.8, Table 8-15
+    const int q = clip3(0, 51, qp + off);
+    return q < 30 ? (uint32_t)q : c_cqp[q - 30];
+}
+// Intra4x4 / Intra8x8 mode with neighbouring samples left, above, above left (nxn_mode_ok).
+__device__ __forceinline__ bool stage_mode_ok(int mode, bool left, bool top, bool tl) {
+    // samples a mode reads (1 left, 2 above, 4 above left), 8 for what is no mode
+    const uint32_t need = mode > 8 ? 8u : mode == 2 ? 0u : mode == 0 || mode == 3 || mode == 7 ? 2u : mode == 1 || mode == 8 ? 1u : 7u;
+    const uint32_t have = (left ? 1u : 0u) | (top ? 2u : 0u) | (tl ? 4u : 0u);
+    return (need & ~have) == 0u;
+}
+struct StageSums {
+    uint32_t inter, intra, lists;
+};
+// One MB; false when it breaks a rule.  ax is complete but for the residual index of an intra MB.
+__device__ __forceinline__ bool stage_mb(const StageIn &S, int x, int y, DevAux &ax, StageSums &sum) {
+    const int W = S.W, a = y * W + x;
+    const GAS h264g_mb *const mbs = G(S.mbs);
+    const GAS h264g_mb &m = mbs[a];
+    const int cls = m.mb_type, cbp = m.cbp, qp = m.qp_y;
+    const bool i16 = cls == H264G_MB_I16x16, t8 = m.flags & H264G_MBF_T8x8;
+    const uint64_t off = m.level_offset;
+    if (cls > H264G_MB_B || qp > 51 || off > S.n_levels || (cbp >> 4) > 2) return false;
+    if (i16 && (cbp & 15) != 0 && (cbp & 15) != 15) return false;
+    if (cls == H264G_MB_P_SKIP && cbp) return false;
+    if (cls == H264G_MB_I8x8 && !t8) return false;
+    if ((cls == H264G_MB_I4x4 || i16) && t8) return false;
+    const uint32_t sub = *(const GAS uint32_t *)m.sub_part_shape;
+    if (cls_inter(cls) && t8 && ((cbp & 15) == 0 || (m.part_shape == H264G_PART_8x8 && sub != 0u))) return false;
+    if (m.flags & H264G_MBF_FIELD) return false;
+    if (S.slice_type == H264G_SLICE_I && cls_inter(cls)) return false;
+    if (S.slice_type != H264G_SLICE_B && cls == H264G_MB_B) return false;
+    if (S.slice_type != H264G_SLICE_P && (cls == H264G_MB_P || cls == H264G_MB_P_SKIP)) return false;
+    const int qd = cls == H264G_MB_IPCM ? 0 : qp;
+    ax.qdb[0] = (uint8_t)qd;
+    ax.qdb[1] = (uint8_t)stage_chroma_qp(qd, S.cqo[1]);
+    ax.qdb[2] = (uint8_t)stage_chroma_qp(qd, S.cqo[0]);
+    ax.qpc[0] = (uint8_t)stage_chroma_qp(qp, S.cqo[0]);
+    ax.qpc[1] = (uint8_t)stage_chroma_qp(qp, S.cqo[1]);
+    if (cls == H264G_MB_IPCM) {
+        if (off + 384 > S.n_levels) return false;
+        ax.kind = AUX_PCM;
+#pragma unroll
+        for (int l = 0; l < 2; l++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) ax.refid[l][q] = S.nref[l] > 0 ? S.ref_slot[l][0] : (int8_t)-1;
+        sum.inter += 384 + 384 * 2 + 16;
+        return true;
+    }
+    const bool intra = cls_intra(cls);
+    uint32_t kind = (intra ? AUX_INTRA : AUX_INTER) | (t8 ? AUX_T8 : 0u);
+    // ---- levels: masks -> non-zero bits
+    const int lm = cbp & 15, cc = cbp >> 4, nl = 4 * __popc((uint32_t)lm);
+    const int nmask = (i16 ? 1 : 0) + nl + (cc >= 1 ? 2 : 0) + (cc == 2 ? 8 : 0);
+    if (off + (uint64_t)nmask > S.n_levels) return false;
+    const GAS uint16_t *const lv = (const GAS uint16_t *)G(S.levels) + off;
+    uint32_t nvals = 0, nz4 = 0, nz8 = 0, stray = 0;
+    int i = 0;
+    if (i16) nvals += __popc((uint32_t)lv[i++]);
+    const uint32_t lbits = i16 ? 0xFFFEu : 0xFFFFu;
+    for (int q = 0; q < 4; q++)
+        if ((lm >> q) & 1)
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const uint32_t mk = lv[i++];
+                nvals += __popc(mk);
+                stray |= mk & ~lbits;
+                if (mk && t8) nz8 |= 1u << q;
+                if (mk && !t8) nz4 |= 1u << (4 * q + b);
+            }
+    if (cc >= 1)
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const uint32_t mk = lv[i++];
+            nvals += __popc(mk);
+            stray |= mk & ~0x000Fu;
+        }
+    if (cc == 2)
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const uint32_t mk = lv[i++];
+            nvals += __popc(mk);
+            stray |= mk & ~0xFFFEu;
+        }
+    if (stray & 0xFFFFu) return false;
+    if (off + (uint64_t)nmask + nvals > S.n_levels) return false;
+    if (nmask) kind |= AUX_RESID;
+    ax.kind = (uint8_t)kind;
+    ax.nmask = (uint8_t)nmask;
+    ax.nz4 = (uint16_t)nz4;
+    ax.nz8 = (uint8_t)nz8;
+    ax.ires = nvals << AUX_NVALS_SHIFT;
+    // ---- intra modes vs neighbour availability
+    if (intra) {
+        auto avail = [&](int dx, int dy) -> bool {
+            const int nx = x + dx, ny = y + dy;
+            if (nx < 0 || ny < 0 || nx >= W) return false;
+            const GAS h264g_mb &n = mbs[ny * W + nx];
+            if (n.slice_num != m.slice_num) return false;
+            return !(S.cip && (n.mb_type == H264G_MB_P_SKIP || ((n.mb_type == H264G_MB_P || n.mb_type == H264G_MB_B) &&
+                                                               n.part_shape != H264G_PART_8x8)));
+        };
+        const bool A = avail(-1, 0), B = avail(0, -1), D = avail(-1, -1);
+        if (!i16) {
+            const int n = cls == H264G_MB_I4x4 ? 4 : 2;
+            for (int by = 0; by < n; by++)
+                for (int bx = 0; bx < n; bx++) {
+                    const bool left = bx > 0 || A, top = by > 0 || B;
+                    const bool tl = bx > 0 ? (by > 0 || B) : (by > 0 ? A : D);
+                    const int blk = n == 4 ? 8 * (by >> 1) + 4 * (bx >> 1) + 2 * (by & 1) + (bx & 1) : by * 2 + bx;
+                    if (!stage_mode_ok(m.intra_pred_modes[blk], left, top, tl)) return false;
+                }
+        } else {
+            const int md = m.intra16x16_pred_mode;
+            if (md > 3 || (md == 0 && !B) || (md == 1 && !A) || (md == 3 && !(A && B && D))) return false;
+        }
+        const int cm = m.intra_chroma_pred_mode;
+        if (cm > 3 || (cm == 1 && !A) || (cm == 2 && !B) || (cm == 3 && !(A && B && D))) return false;
+        sum.intra += 384 + 2 * ((uint32_t)nmask + nvals) + 16 * 2 + 48;
+        return true;
+    }
+    // ---- inter: reference slots, prediction flags, weight entries
+    const int shape = m.part_shape;
+    if (shape > 3) return false;
+    if (shape == H264G_PART_8x8 && (sub & 0xFCFCFCFCu)) return false;
+    uint32_t pf = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int r0 = m.ref_idx[0][q], r1 = m.ref_idx[1][q];
+        if (r0 < 0 && r1 < 0) return false;
+        if (cls != H264G_MB_B && r1 >= 0) return false;
+        if (r0 < -1 || r0 >= S.nref[0] || r1 < -1 || r1 >= S.nref[1]) return false;
+        if (r0 >= 0) {
+            ax.refid[0][q] = S.ref_slot[0][r0];
+            pf |= 1u << q;
+        }
+        if (r1 >= 0) {
+            ax.refid[1][q] = S.ref_slot[1][r1];
+            pf |= 16u << q;
+        }
+        const uint32_t e = (uint32_t)((r0 + 1) * S.n1 + r1 + 1);
+        if ((S.bad_weight[e >> 5] >> (e & 31u)) & 1u) return false;
+        ax.wp[q] = (uint8_t)e;
+    }
+    ax.pf = (uint8_t)pf;
+    // ---- algorithmic bytes: per partition and list used (stage_picture)
+    const int ps = cls == H264G_MB_P_SKIP ? H264G_PART_16x16 : shape;
+    uint32_t bytes = 0, lists = 0;
+    for (int b = 0; b < 16; b++) {
+        const int bx = b & 3, by = b >> 2, q = (by >> 1) * 2 + (bx >> 1);
+        int w, h;
+        if (ps != H264G_PART_8x8) {
+            w = ps == H264G_PART_8x16 ? 2 : 4;
+            h = ps == H264G_PART_16x8 ? 2 : 4;
+        } else {
+            const uint32_t ss = (sub >> (8 * q)) & 3u;
+            w = ss == H264G_SUB_8x8 || ss == H264G_SUB_8x4 ? 2 : 1;
+            h = ss == H264G_SUB_8x8 || ss == H264G_SUB_4x8 ? 2 : 1;
+        }
+        if (bx % w || by % h) continue;
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+            if (!((pf >> (4 * l + q)) & 1u)) continue;
+            const int mx = m.mv[l][b][0], my = m.mv[l][b][1];
+            bytes += (uint32_t)((4 * w + 5 * ((mx & 3) != 0)) * (4 * h + 5 * ((my & 3) != 0)) +
+                                2 * (2 * w + ((mx & 7) != 0)) * (2 * h + ((my & 7) != 0)) + 5);
+            lists++;
+        }
+    }
+    sum.inter += bytes + 384 + 2 * ((uint32_t)nmask + nvals) + 8;
+    sum.lists += lists;
+    return true;
+}
+__global__ __launch_bounds__(WAVE) void k_stage(StageIn S) {
+    const int lane = wave_lane(), W = S.W, per = (W + WAVE - 1) / WAVE;
+    const int y = (int)(blockIdx.x / (uint32_t)per), x0 = (int)(blockIdx.x % (uint32_t)per) * WAVE, x = x0 + lane;
+    const GAS h264g_mb *const mbs = G(S.mbs);
+    const bool in = x < W;
+    const int a = y * W + (in ? x : W - 1);
+    DevAux ax;
+    {
+        uint32_t *const w = (uint32_t *)&ax;
+#pragma unroll
+        for (int k = 0; k < (int)(sizeof(DevAux) / 4); k++) w[k] = k < 2 ? 0xFFFFFFFFu : 0u;  // refid -1, the rest 0
+    }
+    StageSums sum{0u, 0u, 0u};
+    const bool ok = !in || stage_mb(S, x, y, ax, sum);
+    const GAS h264g_mb &m = mbs[a];
+    const uint32_t sn = m.slice_num;
+    const bool intra = in && cls_intra(m.mb_type);
+    // residual index: the row's intra MBs before this one
+    uint32_t before = G(S.irow)[y];
+    for (int c = 0; c < x0; c += WAVE) before += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(cls_intra(mbs[y * W + c + lane].mb_type)));
+    const uint64_t im = __builtin_amdgcn_ballot_w64(intra);
+    const uint32_t idx = before + __builtin_amdgcn_mbcnt_hi((uint32_t)(im >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)im, 0u));
+    if (intra) {
+        ax.ires |= idx;
+        uint32_t av = (x > 0 ? 1u : 0u) | (y > 0 ? 2u : 0u) | (y > 0 && x < W - 1 ? 4u : 0u) | (x > 0 && y > 0 ? 8u : 0u), dep = 0;
+        const int nb[4] = {a - 1, a - W, a - W + 1, a - W - 1};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (!(av & (1u << k))) continue;
+            const GAS h264g_mb &n = mbs[nb[k]];
+            if (n.slice_num != sn) {
+                av &= ~(1u << k);
+                continue;
+            }
+            const int c = n.mb_type;
+            if (S.cip && (c == H264G_MB_P_SKIP || ((c == H264G_MB_P || c == H264G_MB_B) && n.part_shape != H264G_PART_8x8))) av &= ~(1u << k);
+            if (cls_intra(c)) dep |= 1u << k;
+        }
+        if (!(m.mb_type == H264G_MB_I8x8 || (m.mb_type == H264G_MB_I4x4 && (m.intra_pred_modes[5] == 3 || m.intra_pred_modes[5] == 7))))
+            dep &= ~4u;
+        G(S.icol)[idx] = (uint32_t)x | av << ICOL_AV_SHIFT | dep << ICOL_DEP_SHIFT | ((ax.kind & AUX_RESID) ? ICOL_RES : 0u);
+    }
+    if (in) {
+        GAS uint32_t *const o = (GAS uint32_t *)G(S.aux + a);
+        const uint32_t *const w = (const uint32_t *)&ax;
+#pragma unroll
+        for (int k = 0; k < (int)(sizeof(DevAux) / 4); k++) o[k] = w[k];
+    }
+    GAS StageResult *const r = G(S.res);
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(!ok), none = __builtin_amdgcn_ballot_w64(in && sn == H264G_SLICE_NONE),
+                   other = __builtin_amdgcn_ballot_w64(in && sn != H264G_SLICE_NONE && sn != S.first_sn);
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        sum.inter += __shfl_xor(sum.inter, d);
+        sum.intra += __shfl_xor(sum.intra, d);
+        sum.lists += __shfl_xor(sum.lists, d);
+    }
+    if (lane == 0) {
+        const uint32_t base = (uint32_t)(y * W + x0);
+        if (bad) atomicMin((uint32_t *)&r->err_mb, base + (uint32_t)__builtin_ctzll(bad));
+        if (none) atomicMin((uint32_t *)&r->dbk_stop, base + (uint32_t)__builtin_ctzll(none));
+        if (other) atomicOr((uint32_t *)&r->multi_slice, 1u);
+        atomicAdd((unsigned long long *)&r->alg[0], (unsigned long long)sum.inter);
+        atomicAdd((unsigned long long *)&r->alg[1], (unsigned long long)sum.intra);
+        atomicAdd((unsigned long long *)&r->alg[2], (unsigned long long)sum.lists);
+    }
+}
+
 // YUV420P -> BGR24 of one DPB slot (CH264PictureBase::convertYuv420pToBgr24,
 // H264PictureBase.cpp:440-495): one thread per 2x2 luma block (one chroma sample);
 // BT.601 integer coefficients over 1000 with C division (toward zero), clipped.
@@ -3423,6 +3672,12 @@ __global__ void k_copy(const uint4 *src, uint4 *dst, uint64_t n16) {
 }  // namespace
 
 extern "C" {
+
+int h264g_launch_stage(const StageIn *in, void *stream) {
+    if (in->W <= 0 || in->H <= 0) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_stage, dim3((uint32_t)in->H * (uint32_t)((in->W + WAVE - 1) / WAVE)), dim3(WAVE), 0, (hipStream_t)stream, *in);
+    return (int)hipGetLastError();
+}
 
 int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, void *stream) {
     if (n == 0) return 0;
