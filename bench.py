@@ -288,7 +288,7 @@ def main():
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-plain", action="store_true")
     ap.add_argument("--waves", type=int, default=0)
-    ap.add_argument("--no-graphs", action="store_true", help="launch batch stages directly instead of hipGraph replay")
+    ap.add_argument("--no-graphs", action="store_true", help="no effect: batch stages are launched directly")
     ap.add_argument("--deblock", choices=["bands", "mb_wavefront", "mb_rows"], default="bands",
                     help="deblocking schedule")
     ap.add_argument("--deblock-waves", type=int, default=0, help="MB rows per band of the bands schedule (0 = 8)")
@@ -378,7 +378,7 @@ def main():
     log(f"staged {sum(len(r) for r in pics)} pictures ({mpix_step:.1f} Mpix per step) in "
         f"{time.perf_counter() - t:.1f} s")
 
-    # ---- batched: warmup (captures each batch's stage graph), then K timed passes
+    # ---- batched: warmup (untimed), then K timed passes
     for _ in range(max(1, args.warmup)):
         for b in batches:
             eng.batch_run(b)

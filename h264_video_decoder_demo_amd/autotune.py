@@ -98,7 +98,7 @@ def autotune(gens, n_frames: int = 0, reps: int = 2, deblock_rows=DEBLOCK_ROWS, 
             eng.set_bands(d, i)
             batches = [eng.batch_create([r[f] for f in run for r in rows]) for run in independent_runs(rows)]
             try:
-                for b in batches:  # graph capture
+                for b in batches:  # first pass untimed
                     eng.batch_run(b)
                 eng.sync()
                 t0 = _clock()

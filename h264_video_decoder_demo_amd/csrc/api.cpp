@@ -145,8 +145,6 @@ struct Batch {
     uint32_t n_intra = 0, n_mintra = 0;  // intra MBs of the frame pictures / MBAFF frames
     bool dbk_off = false;            // no picture of the batch is deblocked
     bool scaled = false;             // a picture of the batch has scaling matrices
-    hipGraphExec_t graph = nullptr;  // the captured stage sequence (kernel nodes only)
-    hipGraphExec_t graph_dbk = nullptr;  // its deblocking, when that runs on the lane's deblocking stream
     std::vector<SlotUse> uses;       // DPB slots the pictures write and read
     std::vector<std::pair<uint32_t, uint64_t>> streams;  // (stream id, Stream::gen) of its pictures
 };
@@ -171,6 +169,8 @@ struct h264g_ctx {
     // a B picture not used for reference).
     hipStream_t dstream[2] = {nullptr, nullptr};
     hipEvent_t front[2] = {nullptr, nullptr};  // end of a lane's last pre-deblocking stages
+    bool front_on_ds[2] = {false, false};      // those ran on its deblocking stream
+    bool joined[2] = {true, true};             // the deblocking stream is ordered after all of the lane's work
     DbkRec hist[2][kDbkHist];
     int hist_next[2] = {0, 0};
     int split_mbs = 16384;         // 0: one lane
@@ -187,7 +187,6 @@ struct h264g_ctx {
     std::vector<PoolBlock> pool;
     size_t pool_bytes = 0;
     bool profile = false;
-    bool no_graphs = false;
     int dbk_schedule = H264G_DEBLOCK_BANDS;
     int intra_schedule = H264G_INTRA_BANDS;
     int intra_waves = 8;           // rows per band (waves per workgroup) of the intra band schedule
@@ -1071,63 +1070,49 @@ bool conflicts(const DbkRec &r, const std::vector<SlotUse> &uses) {
     return false;
 }
 
-// Stages of `q` (pictures `uses`) on `lane`.  sb: the batch whose captured graphs to replay
-// (captured on first use), or null for direct launches.  Order: the lane waits for the
-// newest deblocking launch in flight that writes a slot these pictures write or read
-// (deblocking launches on the lane's deblocking stream complete in order, so that one
-// covers the older ones); inter / intra / bS on the lane; deblocking on the deblocking
-// stream after them, with the band schedule in a two-lane context (the other schedules
-// share per-MB progress words with the intra stage, and a one-lane context is the
-// strictly sequential shape: there deblocking stays on the lane).
-int enqueue(h264g_ctx *c, const StageSet &q, int lane, const std::vector<SlotUse> &uses, Batch *sb,
-            bool events = true) {
+// Stages of `q` (pictures `uses`) on `lane`, three to eight launches, which cost the host less
+// than replaying them as a captured graph (12 us a batch against 45; sixteen dependent CIF
+// pictures took 943 us directly, 1168 as graphs).  Order: deblocking goes to the lane's
+// deblocking stream after the set's other stages, with the band schedule in a two-lane context
+// (the other schedules share per-MB progress words with the intra stage, and a one-lane context
+// is the strictly sequential shape: there deblocking stays on the lane).  Inter / intra / bS:
+//  - on the lane, after the newest deblocking launch in flight that writes a slot these
+//    pictures write or read (deblocking launches on one stream complete in order, so that one
+//    covers the older ones) and after the previous set's;
+//  - on the deblocking stream when that launch is the last one there, as in a chain of P
+//    pictures: what they wait for is then the launch before them on the same stream, and no
+//    picture crosses between streams (the two crossings took 13 of 88 us per CIF P picture).
+int enqueue(h264g_ctx *c, const StageSet &q, int lane, const std::vector<SlotUse> &uses, bool events = true) {
     hipStream_t s = lane_stream(c, lane), ds = c->dstream[lane];
-    for (int k = 1; k <= kDbkHist; k++) {
-        const DbkRec &r = c->hist[lane][(c->hist_next[lane] - k + kDbkHist) % kDbkHist];
-        if (r.live && conflicts(r, uses)) {
-            HIPCHK(hipStreamWaitEvent(s, r.ev, 0));
-            break;
-        }
-    }
     // one-lane contexts (lane_split_mbs < 0) keep the strictly sequential shape
     const bool split = c->dbk_schedule == H264G_DEBLOCK_BANDS && !q.dbk_off && c->split_mbs > 0;
     hipEvent_t *ev = events ? profile_events(c) : nullptr;
-    const bool graphs = sb && !c->profile && !c->no_graphs;
-    // capture of the launches `parts` on stream st into *g (kernel nodes only; every launch
-    // argument, including the wavefront epochs, which live in device memory, is the same
-    // on each replay)
-    auto capture = [&](int parts, hipStream_t st, hipGraphExec_t *g) -> int {
-        HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        int rc = launch_stages(c, q, lane, parts, st, nullptr);
-        hipGraph_t gr = nullptr;
-        hipError_t e = hipStreamEndCapture(st, &gr);
-        if (rc) { if (gr) (void)hipGraphDestroy(gr); return rc; }
-        if (e != hipSuccess) return h264g_set_error(H264G_E_DEVICE, "stream capture: %s", hipGetErrorString(e));
-        e = hipGraphInstantiate(g, gr, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(gr);
-        if (e != hipSuccess) { *g = nullptr; return h264g_set_error(H264G_E_DEVICE, "graph instantiate: %s", hipGetErrorString(e)); }
-        return 0;
-    };
+    const DbkRec &last = c->hist[lane][(c->hist_next[lane] - 1 + kDbkHist) % kDbkHist];
+    const bool chain = split && c->joined[lane] && last.live && conflicts(last, uses);
+    if (!chain) {
+        if (c->front_on_ds[lane]) HIPCHK(hipStreamWaitEvent(s, c->front[lane], 0));
+        for (int k = 1; k <= kDbkHist; k++) {
+            const DbkRec &r = c->hist[lane][(c->hist_next[lane] - k + kDbkHist) % kDbkHist];
+            if (r.live && conflicts(r, uses)) {
+                HIPCHK(hipStreamWaitEvent(s, r.ev, 0));
+                break;
+            }
+        }
+    }
+    hipStream_t fs = chain ? ds : s;
     const int first = split ? kFront : (kFront | kBack);
-    if (graphs) {
-        if (!sb->graph) { int rc = capture(first, s, &sb->graph); if (rc) return rc; }
-        HIPCHK(hipGraphLaunch(sb->graph, s));
-    } else {
-        int rc = launch_stages(c, q, lane, first, s, ev);
-        if (rc) return rc;
-    }
+    c->joined[lane] = false;
+    c->front_on_ds[lane] = false;
+    if (int rc = launch_stages(c, q, lane, first, fs, ev)) return rc;
     if (!split) return 0;
-    HIPCHK(hipEventRecord(c->front[lane], s));
-    HIPCHK(hipStreamWaitEvent(ds, c->front[lane], 0));
-    if (graphs) {
-        if (!sb->graph_dbk) { int rc = capture(kBack, ds, &sb->graph_dbk); if (rc) return rc; }
-        HIPCHK(hipGraphLaunch(sb->graph_dbk, ds));
-    } else {
-        int rc = launch_stages(c, q, lane, kBack, ds, ev);
-        if (rc) return rc;
-    }
+    HIPCHK(hipEventRecord(c->front[lane], fs));
+    c->front_on_ds[lane] = chain;
+    if (!chain) HIPCHK(hipStreamWaitEvent(ds, c->front[lane], 0));
+    c->joined[lane] = true;
+    if (int rc = launch_stages(c, q, lane, kBack, ds, ev)) return rc;
     DbkRec &r = c->hist[lane][c->hist_next[lane]];
-    if (r.live) HIPCHK(hipStreamWaitEvent(s, r.ev, 0));  // leaves the history: order the lane after it
+    // r leaves the history: order the lane after it (as its next wait for a front on ds does)
+    if (r.live && !chain) HIPCHK(hipStreamWaitEvent(s, r.ev, 0));
     if (!r.ev) HIPCHK(hipEventCreateWithFlags(&r.ev, hipEventDisableTiming));
     HIPCHK(hipEventRecord(r.ev, ds));
     r.dst.clear();
@@ -1137,15 +1122,10 @@ int enqueue(h264g_ctx *c, const StageSet &q, int lane, const std::vector<SlotUse
     return 0;
 }
 
-// Caller holds ctx->mu.  A batch with a graph is destroyed only when idle.
+// Caller holds ctx->mu.
 int free_batch(h264g_ctx *c, h264g_batch *b) {
     if (!b) return 0;
-    if (b->sub[0].graph || b->sub[1].graph || b->sub[0].graph_dbk || b->sub[1].graph_dbk) (void)sync_lanes(c);
-    for (Batch &sb : b->sub) {
-        if (sb.graph) (void)hipGraphExecDestroy(sb.graph);
-        if (sb.graph_dbk) (void)hipGraphExecDestroy(sb.graph_dbk);
-        pool_put(c, sb.dmem, sb.dbytes);
-    }
+    for (Batch &sb : b->sub) pool_put(c, sb.dmem, sb.dbytes);  // reused only after the launches enqueued so far
     delete b;
     return 0;
 }
@@ -1190,7 +1170,6 @@ int32_t h264g_create(const h264g_config *cfg, h264g_ctx **out) {
     c->device = dev;
     c->budget = cfg ? cfg->dpb_budget_bytes : 0;
     c->profile = cfg && cfg->profile;
-    c->no_graphs = cfg && cfg->no_graphs;
     c->dbk_schedule = cfg ? cfg->deblock_schedule : H264G_DEBLOCK_BANDS;
     c->dbk_waves = (cfg && cfg->deblock_waves > 0) ? cfg->deblock_waves : 8;
     c->intra_schedule = cfg ? cfg->intra_schedule : H264G_INTRA_BANDS;
@@ -1320,6 +1299,7 @@ int32_t h264g_stream_open(h264g_ctx *c, const h264g_stream_desc *d, uint32_t *id
         return h264g_set_error(H264G_E_NOMEM, "stream device memory");
     }
     hipStream_t ls = lane_stream(c, s.lane);
+    c->joined[s.lane] = false;
     HIPCHK(hipMemsetAsync(s.prog, 0, prog_bytes, ls));  // epoch 0 never matches a launch
     HIPCHK(hipMemsetAsync(s.dpb, 0, dpb_bytes, ls));
     s.strip_dbk_rows = c->dbk_waves;
@@ -1423,7 +1403,7 @@ int enqueue_picture(h264g_ctx *c, const h264g_pic *p, bool events = true) {
         q.n_ibands = (uint32_t)((p->H + intra_rows(c) - 1) / intra_rows(c));
         q.n_dbands = (uint32_t)((p->H + dbk_rows(c) - 1) / dbk_rows(c));
     }
-    return enqueue(c, q, c->streams[p->stream].lane, {slot_use(p->stream, p->desc)}, nullptr, events);
+    return enqueue(c, q, c->streams[p->stream].lane, {slot_use(p->stream, p->desc)}, events);
 }
 
 // State of the allocation-free entry point per device: the lock that serialises its calls
@@ -1685,7 +1665,7 @@ int32_t h264g_batch_run(h264g_ctx *c, h264g_batch *b) {
     for (int l = 0; l < 2; l++) {
         Batch &sb = b->sub[l];
         if (!sb.n_pics) continue;
-        int rc = enqueue(c, batch_stages(&sb), l, sb.uses, &sb);
+        int rc = enqueue(c, batch_stages(&sb), l, sb.uses);
         if (rc) return rc;
     }
     return H264G_OK;
@@ -1705,8 +1685,8 @@ int32_t h264g_batch_submit(h264g_ctx *c, h264g_pic *const *pics, uint32_t n) {
     if (rc) return rc;
     std::lock_guard<std::mutex> lk(c->mu);
     HIPCHK(hipSetDevice(c->device));
-    for (int l = 0; l < 2 && !rc; l++)  // used once: launched directly, not captured
-        if (b->sub[l].n_pics) rc = enqueue(c, batch_stages(&b->sub[l]), l, b->sub[l].uses, nullptr);
+    for (int l = 0; l < 2 && !rc; l++)
+        if (b->sub[l].n_pics) rc = enqueue(c, batch_stages(&b->sub[l]), l, b->sub[l].uses);
     free_batch(c, b);                   // its blocks are reused after these launches
     return rc;
 }

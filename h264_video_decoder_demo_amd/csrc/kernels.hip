@@ -809,7 +809,7 @@ __device__ __forceinline__ uint32_t launch_epoch(const uint32_t *epoch) {
 // The last wave of a launch resets the control block for the next launch on the stream
 // and advances the shared epoch, so the next wavefront launch (of either kind) uses a
 // value no progress word holds yet.  Launch arguments therefore stay identical from one
-// launch to the next, which lets a captured graph replay them.
+// launch to the next (a caller may capture them).
 __device__ void retire(DevCtl *ctl, uint32_t total_waves, uint32_t *epoch, uint32_t cur) {
     const uint32_t d = uniform(atomicAdd(&ctl->done, wave_lane() == 0 ? 1u : 0u));
     if (d == total_waves - 1) {

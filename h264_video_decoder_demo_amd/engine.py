@@ -193,9 +193,10 @@ class Engine:
                  intra_schedule: int = 0, intra_waves: int = 0, lane_split_mbs: int = 0):
         """deblock_schedule: _lib.DEBLOCK_BANDS (default), DEBLOCK_MB_WAVEFRONT or DEBLOCK_MB_ROWS;
         intra_schedule: _lib.INTRA_BANDS (default) or INTRA_MB_WAVEFRONT.  deblock_waves /
-        intra_waves: MB rows per band of the band schedules (0 = 8 / 8).  lane_split_mbs:
-        streams with pictures of at least this many MBs run on the context's second HIP
-        stream (0 = 16384, negative = one stream)."""
+        intra_waves: MB rows per band of the band schedules (0 = 8 / 8; bands run with at most
+        4 of them).  lane_split_mbs: streams with pictures of at least this many MBs run on the
+        context's second HIP stream (0 = 16384, negative = one stream).  graphs: no effect, a
+        batch's stages are launched directly."""
         cfg = Config(device=device, dpb_budget_bytes=dpb_budget_bytes, max_batch_pictures=max_batch_pictures,
                      profile=1 if profile else 0, waves=waves, no_graphs=0 if graphs else 1,
                      deblock_schedule=deblock_schedule, deblock_waves=deblock_waves,

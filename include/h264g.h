@@ -170,9 +170,8 @@ typedef struct h264g_config {
     int32_t  max_batch_pictures;  /* pictures per batched launch (0 = default 4096)   */
     int32_t  profile;             /* 1 = record per-stage HIP events                  */
     int32_t  waves;               /* persistent waves per wavefront launch (0 = auto) */
-    int32_t  no_graphs;           /* 1 = launch batch stages directly; 0 = replay each
-                                     batch's stage sequence as a captured hipGraph
-                                     (profiled contexts always launch directly)       */
+    int32_t  no_graphs;           /* no effect: a batch's stages are launched directly,
+                                     which costs less than replaying a graph of them  */
     int32_t  deblock_schedule;    /* H264G_DEBLOCK_*                                  */
     int32_t  deblock_waves;       /* MB rows per band of H264G_DEBLOCK_BANDS, 1..24
                                      (0 = 8); bands run with at most 4 of them       */
@@ -364,8 +363,7 @@ int32_t h264g_fence_wait(h264g_ctx *ctx, h264g_fence *fence);
 int32_t h264g_fence_destroy(h264g_ctx *ctx, h264g_fence *fence);
 
 /* Turn per-stage event recording on or off for later launches (as
- * h264g_config.profile).  While it is on, batches launch their stages directly
- * instead of replaying their captured graphs. */
+ * h264g_config.profile). */
 int32_t h264g_set_profile(h264g_ctx *ctx, int32_t on);
 
 /* Wait for all enqueued work; returns the first device error word if any. */
