@@ -143,6 +143,11 @@ struct DevCtl {
 };
 
 // Device error bits (ORed into the context's error word).
+// The error word of a context, in device memory; kernels take its address as that of `word`.
+struct DevErr {
+    uint32_t word, pad;
+    uint32_t *host;           // its copy in pinned memory
+};
 #define DEVERR_TIMEOUT  0x1u
 
 extern "C" {

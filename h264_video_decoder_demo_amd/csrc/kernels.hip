@@ -764,6 +764,13 @@ constexpr uint32_t SPIN_LIMIT = 1u << 20;
 // their own, which never terminates.
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// Sets the device error word (polled by the other waits, so it is device memory) and its copy in
+// pinned memory that the host reads.
+__device__ __forceinline__ void report_timeout(uint32_t *err) {
+    atomicOr(err, DEVERR_TIMEOUT);
+    __hip_atomic_store(G(G((const DevErr *)err)->host), DEVERR_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Waits until flags[i] == epoch for each listed neighbour.  Bounded: after SPIN_LIMIT
 // polls, or once another wave has raised the error word, the wave stops waiting (its
 // output is then wrong, and h264g_sync reports the error).
@@ -774,7 +781,7 @@ __device__ __forceinline__ void wait_dep(const uint32_t *flags, int dep, uint32_
     for (uint32_t it = 0;; ++it) {
         if (uniform(ld_acquire(&flags[d])) == epoch) break;
         if (it >= SPIN_LIMIT) {
-            atomicOr(err, DEVERR_TIMEOUT);
+            report_timeout(err);
             break;
         }
         if ((it & 255u) == 255u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) break;
@@ -1642,7 +1649,7 @@ __device__ void wait_row(const uint64_t *w, uint64_t want, uint32_t *err) {
         const uint32_t lo = uniform((uint32_t)v), hi = uniform((uint32_t)(v >> 32));
         if ((((uint64_t)hi << 32) | lo) >= want) break;
         if (it >= SPIN_LIMIT) {
-            atomicOr(err, DEVERR_TIMEOUT);
+            report_timeout(err);
             break;
         }
         if ((it & 255u) == 255u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) break;
@@ -1840,7 +1847,7 @@ __device__ __forceinline__ void lds_wait(const uint32_t *w, uint32_t seen, uint3
 #pragma unroll 1
     for (uint32_t it = 0; v < need; ++it) {
         if (it >= LDS_SPIN_LIMIT) {
-            atomicOr(err, DEVERR_TIMEOUT);
+            report_timeout(err);
             break;
         }
         if ((it & 1023u) == 1023u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) break;
@@ -2014,7 +2021,7 @@ __device__ __forceinline__ void istrip_reader(const GAS uint64_t *sw, const GAS 
                 continue;
             }
             if (it >= SPIN_LIMIT) {
-                atomicOr(err, DEVERR_TIMEOUT);
+                report_timeout(err);
                 return;
             }
             if ((it & 255u) == 255u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) return;
@@ -3058,7 +3065,7 @@ __device__ __forceinline__ void strip_reader(const GAS StripWords *sw, int W, Db
                 continue;
             }
             if (it >= SPIN_LIMIT) {
-                atomicOr(err, DEVERR_TIMEOUT);
+                report_timeout(err);
                 return;
             }
             if ((it & 255u) == 255u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) return;

@@ -341,7 +341,7 @@ class Engine:
         """BGR24 image of a DPB slot, rows padded to 4 bytes (the reference's BMP layout)."""
         W, H, _ = self.streams[sid]
         stride = (W * 16 * 3 + 3) // 4 * 4
-        out = np.zeros((H * 16, stride), np.uint8)
+        out = np.empty((H * 16, stride), np.uint8)
         check(lib().h264g_slot_to_bgr24(self._h, sid, slot, _ptr(out), stride, 1 if flip else 0))
         return out
 
