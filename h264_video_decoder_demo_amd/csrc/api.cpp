@@ -1065,9 +1065,11 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
     int e = 0;
     if (parts & kFront) {
         if (ev) HIPCHK(hipEventRecord(ev[0], s));
-        e = h264g_launch_inter(q.pics, q.chunks, q.n_chunks, 0, q.scaled ? 1 : 0, s);
+        // boundary strengths ride in the inter launches, unless the stages' times are taken
+        const int what = q.dbk_off || ev ? INTER_MBS : INTER_MBS | INTER_BS;
+        e = h264g_launch_inter(q.pics, q.chunks, q.n_chunks, 0, q.scaled ? 1 : 0, what, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "inter launch: %s", hipGetErrorString((hipError_t)e));
-        e = h264g_launch_inter(q.pics, q.mchunks, q.n_mchunks, 1, 0, s);
+        e = h264g_launch_inter(q.pics, q.mchunks, q.n_mchunks, 1, 0, what, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "inter launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         if (ev) HIPCHK(hipEventRecord(ev[1], s));
         if (q.n_intra)
@@ -1079,9 +1081,9 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
         if (q.n_mintra) e = h264g_launch_intra_mbaff(q.pics, q.n_pics, ctx->d_err, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "intra launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         if (ev) HIPCHK(hipEventRecord(ev[2], s));
-        if (!q.dbk_off) {
-            e = h264g_launch_bs(q.pics, q.chunks, q.n_chunks, 0, s);
-            if (!e) e = h264g_launch_bs(q.pics, q.mchunks, q.n_mchunks, 1, s);
+        if (!q.dbk_off && ev) {
+            e = h264g_launch_inter(q.pics, q.chunks, q.n_chunks, 0, 0, INTER_BS, s);
+            if (!e) e = h264g_launch_inter(q.pics, q.mchunks, q.n_mchunks, 1, 0, INTER_BS, s);
             if (e) return h264g_set_error(H264G_E_DEVICE, "bS launch: %s", hipGetErrorString((hipError_t)e));
         }
         if (ev) HIPCHK(hipEventRecord(ev[3], s));

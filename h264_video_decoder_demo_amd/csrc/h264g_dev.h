@@ -67,7 +67,7 @@ struct DevPic {
     uint64_t *rowprog;        // per-MB-row progress of row-pipelined deblocking:
                               // epoch << 32 | MBs of the row finished
     uint8_t  *bs;             // boundary strengths, 32 bytes per MB: [dir][4-line segment][edge]
-                              // (MBAFF frames: nibbles, see k_bs_mbaff)
+                              // (MBAFF frames: nibbles, see bs_mbaff_mb)
     const uint32_t *irow;     // intra MBs per row: H + 1 offsets, then one ICOL entry per intra MB
     uint32_t n_intra;         // intra-predicted MBs of the picture
     int32_t  dst;             // destination slot
@@ -89,7 +89,7 @@ struct DevPic {
     uint32_t dbk_stop;        // MBs from this address on filter none of their edges (the
                               // first MB of no slice; W * H when every MB has one)
     int32_t  multi_slice;     // the MBs carry more than one slice number (MBs of no slice
-                              // aside): k_bs reads them
+                              // aside): bs_pair_of_mbs reads them
     const uint16_t *ls;       // scaling matrices: LevelScale4x4 [intra, inter luma list][qP % 6]
                               // [raster 16] at 0, LevelScale8x8 [list][qP % 6][raster 64] at
                               // LS8_AT; null with flat lists
@@ -159,9 +159,11 @@ int h264g_launch_stage(const StageIn *in, void *stream);
 #define MB_CHUNK 64u
 // mbaff: every picture of the launch is an MBAFF frame (else none is).
 // scaled: some picture of the launch has scaling matrices (DevPic::ls).
-int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, void *stream);
-// Boundary strengths, of pictures that are deblocked.
-int h264g_launch_bs(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, void *stream);
+// what: INTER_MBS, the inter stage; INTER_BS, the boundary strengths of pictures that are
+// deblocked; or both in one launch.
+#define INTER_MBS 1
+#define INTER_BS  2
+int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, int what, void *stream);
 // `epoch` points at the device word shared by all wavefront launches of a context
 // (initially 1; each launch's last wave advances it).
 int h264g_launch_intra(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,

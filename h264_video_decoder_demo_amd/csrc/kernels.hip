@@ -1309,7 +1309,7 @@ __device__ __forceinline__ int view_ref(const MbView &v, int l, int q) { return 
 __device__ __forceinline__ int dbq_qp(uint32_t q, int plane) { return (q >> (8 * plane)) & 255; }
 __device__ __forceinline__ bool dbq_t8(uint32_t q) { return (q >> 24) & 1u; }
 // the MB's left / top MB edge lies between slices under disable_deblocking_filter_idc 0:
-// its p side takes the MB's own qP (see k_bs)
+// its p side takes the MB's own qP (see bs_pair_of_mbs)
 constexpr uint32_t DBQ_OWN_LEFT = 1u << 25, DBQ_OWN_TOP = 1u << 26;
 
 __device__ __forceinline__ void load_view(const DevPic &P, int addr, MbView &v) {
@@ -1324,7 +1324,7 @@ __device__ __forceinline__ void load_view(const DevPic &P, int addr, MbView &v) 
     v.ref1 = (uint32_t)(uint8_t)ax.refid[1][0] | ((uint32_t)(uint8_t)ax.refid[1][1] << 8) |
              ((uint32_t)(uint8_t)ax.refid[1][2] << 16) | ((uint32_t)(uint8_t)ax.refid[1][3] << 24);
 }
-// Deblocking word of an MB (G(P.dbq), written by k_bs): qP of luma, Cb edges, Cr edges in
+// Deblocking word of an MB (G(P.dbq), written by bs_pair_of_mbs): qP of luma, Cb edges, Cr edges in
 // bytes 0..2, transform_size_8x8_flag in bit 24, DBQ_OWN_LEFT / DBQ_OWN_TOP in bits 25, 26.
 
 __device__ __forceinline__ bool mv_far(int ax, int ay, int bx, int by) { return iabs(ax - bx) >= 4 || iabs(ay - by) >= 4; }
@@ -1507,7 +1507,7 @@ __device__ __forceinline__ void dbk_line_edge(uint32_t (&w)[5], bool act, bool l
 // it, keeps the line in registers and runs its edges in order: left / top MB edge (when
 // `edge`), then the internal ones (luma 4 / 12 skipped with the 8x8 transform, chroma
 // only 4).  Lines of one direction touch disjoint samples, so this gives the reference's
-// edge-by-edge order (8.7, Deblock.cpp:76-635).  qq / eq: deblocking words (see k_bs) of
+// edge-by-edge order (8.7, Deblock.cpp:76-635).  qq / eq: deblocking words (see bs_pair_of_mbs) of
 // the MB and of the left / top MB.
 // cur: tile column of the MB's luma column 0 (16 or 0; chroma cur / 2); the left MB sits
 // in the other half of the tile, so a row's columns -4..-1 are at (16 - cur) + 12.
@@ -1546,7 +1546,7 @@ __device__ __forceinline__ void dbk_lines(const DevPic &P, uint32_t eq, bool edg
     const int iAi = clip3(0, 51, qpq + P.offA), iBi = clip3(0, 51, qpq + P.offB);
     const bool t8 = dbq_t8(qq), on = P.dbk_idc != 1;
     const int seg = luma ? (k >> 2) : (k >> 1);  // 4-line luma segment of the line
-    // bS of this segment's edges 0..3 (k_bs stores them [direction][segment][edge]); chroma
+    // bS of this segment's edges 0..3 (stored [direction][segment][edge]); chroma
     // edge j lies on luma edge 2j.  All table lookups are issued before the filtering.
     const uint32_t bsv = *(const uint32_t *)&bsrec[DIR * 16 + seg * 4];
     const int bs0 = bsv & 255u, bs1 = luma ? (bsv >> 8) & 255u : (bsv >> 16) & 255u, bs2 = (bsv >> 16) & 255u,
@@ -1730,10 +1730,19 @@ __device__ __forceinline__ MbSlot mb_slot(const uint32_t *chunks, uint32_t s) {
 // their entry built for the intra stage.
 // MBAFF: the instance for MBAFF frames (field MBs: geometry, field scans, field references);
 // frame pictures run the instance without any of it.
+// Blocks from n on derive boundary strengths, which depend on the records alone: in a launch of
+// their own they cost a chain of CIF P pictures 3 of 59 us each, one of 1280x720 4 of 164.
+__device__ void bs_pair_of_mbs(const DevPic *pics, const uint32_t *chunks, uint32_t b, uint32_t n);
+__device__ void bs_mbaff_mb(const DevPic *pics, const uint32_t *chunks, uint32_t b, uint32_t n);
 template <bool MBAFF, bool SCALED>
-__global__ __launch_bounds__(WAVE) void k_inter(const DevPic *__restrict__ pics, const uint32_t *__restrict__ chunks) {
+__global__ __launch_bounds__(WAVE) void k_inter(const DevPic *__restrict__ pics, const uint32_t *__restrict__ chunks, uint32_t n) {
     __shared__ WaveRes lds;
-    const MbSlot m = mb_slot(chunks, xcd_item(blockIdx.x, gridDim.x));
+    if (blockIdx.x >= n) {
+        if (MBAFF) bs_mbaff_mb(pics, chunks, blockIdx.x - n, gridDim.x - n);
+        else bs_pair_of_mbs(pics, chunks, blockIdx.x - n, gridDim.x - n);
+        return;
+    }
+    const MbSlot m = mb_slot(chunks, xcd_item(blockIdx.x, n));
     const DevPic &P = pics[m.pic];
     if (m.addr >= P.W * P.H) return;
     if (!(uniform(G(P.aux)[m.addr].kind) & AUX_INTRA)) inter_mb<MBAFF, SCALED>(P, m.addr, &lds);
@@ -2563,11 +2572,11 @@ __device__ __forceinline__ MbaffNb mbaff_nb(int W, int addr, bool field, bool lf
 //   52  horizontal edges 4, 8, 12
 // (chroma edge 4 lies on luma edge 8), 0 where an edge is not filtered.  Fully parallel: they
 // depend on syntax only.  A lane per nibble, a MB per wave.  The MB's deblocking word as in
-// k_bs, with its field flag.
+// bs_pair_of_mbs, with its field flag.
 constexpr int MBS_LEFT = 0, MBS_LEFT_C = 16, MBS_V = 24, MBS_TOP = 36, MBS_TOP_C = 40, MBS_TOP2 = 44, MBS_TOP2_C = 48, MBS_H = 52;
 constexpr uint32_t DBQ_FIELD = 1u << 27;
-__global__ __launch_bounds__(WAVE) void k_bs_mbaff(const DevPic *__restrict__ pics, const uint32_t *__restrict__ chunks) {
-    const MbSlot m = mb_slot(chunks, xcd_item(blockIdx.x, gridDim.x));
+__device__ __forceinline__ void bs_mbaff_mb(const DevPic *pics, const uint32_t *chunks, uint32_t b, uint32_t n) {
+    const MbSlot m = mb_slot(chunks, xcd_item(b, n));
     const DevPic &P = pics[m.pic];
     const int addr = m.addr, pair = addr >> 1, W = P.W, px = pair % W, py = pair / W;
     if (addr >= W * P.H || P.dbk_idc == 1) return;
@@ -3358,9 +3367,9 @@ __global__ __launch_bounds__(WAVE *(DBK_MAX_ROWS + 1)) void k_deblock_band(const
 // 25 / 26); fully parallel: they depend on syntax
 // only, not on samples.  Half a wave per MB (neighbouring MBs, so that an XCD's L2 serves the
 // records two MBs share); lane j = 16 * dir + 4 * edge + segment.
-__global__ __launch_bounds__(WAVE) void k_bs(const DevPic *__restrict__ pics, const uint32_t *__restrict__ chunks) {
+__device__ __forceinline__ void bs_pair_of_mbs(const DevPic *pics, const uint32_t *chunks, uint32_t b, uint32_t n) {
     const int lane = wave_lane();
-    const MbSlot m = mb_slot(chunks, 2 * xcd_item(blockIdx.x, gridDim.x));
+    const MbSlot m = mb_slot(chunks, 2 * xcd_item(b, n));
     const DevPic &P = pics[m.pic];
     const int addr = m.addr + (lane >> 5), W = P.W, mbx = addr % W, mby = addr / W;
     if (addr >= W * P.H || P.dbk_idc == 1) return;
@@ -3686,15 +3695,18 @@ int h264g_launch_stage(const StageIn *in, void *stream) {
     return (int)hipGetLastError();
 }
 
-int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, void *stream) {
+int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, int what, void *stream) {
     if (n == 0) return 0;
-    const dim3 grid(n * MB_CHUNK), block(WAVE);
+    const uint32_t n_mb = (what & INTER_MBS) ? n * MB_CHUNK : 0u;
+    const uint32_t n_bs = !(what & INTER_BS) ? 0u : mbaff ? n * MB_CHUNK : n * (MB_CHUNK / 2);
+    if (n_mb + n_bs == 0) return 0;
+    const dim3 grid(n_mb + n_bs), block(WAVE);
     if (mbaff)  // (scaling matrices are refused in MBAFF frames)
-        hipLaunchKernelGGL((k_inter<true, false>), grid, block, 0, (hipStream_t)stream, pics, chunks);
+        hipLaunchKernelGGL((k_inter<true, false>), grid, block, 0, (hipStream_t)stream, pics, chunks, n_mb);
     else if (scaled)
-        hipLaunchKernelGGL((k_inter<false, true>), grid, block, 0, (hipStream_t)stream, pics, chunks);
+        hipLaunchKernelGGL((k_inter<false, true>), grid, block, 0, (hipStream_t)stream, pics, chunks, n_mb);
     else
-        hipLaunchKernelGGL((k_inter<false, false>), grid, block, 0, (hipStream_t)stream, pics, chunks);
+        hipLaunchKernelGGL((k_inter<false, false>), grid, block, 0, (hipStream_t)stream, pics, chunks, n_mb);
     return (int)hipGetLastError();
 }
 
@@ -3749,13 +3761,6 @@ int h264g_launch_deblock_band(const DevPic *pics, const uint32_t *bands, uint32_
 int h264g_launch_deblock_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *err, void *stream) {
     if (n_pics == 0) return 0;
     hipLaunchKernelGGL(k_deblock_mbaff, dim3(n_pics), dim3(WAVE * MBAFF_WAVES), 0, (hipStream_t)stream, pics, n_pics, err);
-    return (int)hipGetLastError();
-}
-
-int h264g_launch_bs(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, void *stream) {
-    if (n == 0) return 0;
-    if (mbaff) hipLaunchKernelGGL(k_bs_mbaff, dim3(n * MB_CHUNK), dim3(WAVE), 0, (hipStream_t)stream, pics, chunks);
-    else hipLaunchKernelGGL(k_bs, dim3(n * (MB_CHUNK / 2)), dim3(WAVE), 0, (hipStream_t)stream, pics, chunks);
     return (int)hipGetLastError();
 }
 
