@@ -143,6 +143,7 @@ struct Batch {
     uint32_t *d_ibands = nullptr, *d_dbands = nullptr;   // (picture, band) items, band-major
     uint32_t n_chunks = 0, n_mchunks = 0, n_all = 0, n_rows = 0, n_ibands = 0, n_dbands = 0;
     uint32_t n_intra = 0, n_mintra = 0;  // intra MBs of the frame pictures / MBAFF frames
+    uint32_t mpair_rows = 0;         // MB pair rows of the tallest MBAFF frame
     bool dbk_off = false;            // no picture of the batch is deblocked
     bool scaled = false;             // a picture of the batch has scaling matrices
     std::vector<SlotUse> uses;       // DPB slots the pictures write and read
@@ -1051,6 +1052,7 @@ struct StageSet {
     const uint32_t *chunks = nullptr, *mchunks = nullptr, *intra = nullptr, *all = nullptr, *rows = nullptr,
                    *ibands = nullptr, *dbands = nullptr;
     uint32_t n_chunks = 0, n_mchunks = 0, n_intra = 0, n_mintra = 0, n_all = 0, n_rows = 0, n_ibands = 0, n_dbands = 0;
+    uint32_t mpair_rows = 0;  // MB pair rows of the tallest MBAFF frame
     bool dbk_off = false;
     bool scaled = false;  // a picture has scaling matrices: the inter stage takes the kernel that reads them
 };
@@ -1104,7 +1106,7 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
                 e = h264g_launch_deblock_rows(q.pics, q.rows, q.n_rows, &ctl[1], epoch, ctx->d_err, ctx->waves, s);
             }
             if (e) return h264g_set_error(H264G_E_DEVICE, "deblock launch: %s", hipGetErrorString((hipError_t)e));
-            if (q.n_mchunks) e = h264g_launch_deblock_mbaff(q.pics, q.n_pics, ctx->d_err, s);
+            if (q.n_mchunks) e = h264g_launch_deblock_mbaff(q.pics, q.n_pics, q.mpair_rows, &ctl[1], epoch, ctx->d_err, s);
             if (e) return h264g_set_error(H264G_E_DEVICE, "deblock launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         }
         if (ev) HIPCHK(hipEventRecord(ev[5], s));
@@ -1459,6 +1461,7 @@ int enqueue_picture(h264g_ctx *c, const h264g_pic *p, bool events = true) {
     if (p->mbaff) {
         q.n_mchunks = n_chunks;
         q.n_mintra = p->n_intra;
+        q.mpair_rows = (uint32_t)p->H / 2;
     } else {
         q.n_chunks = n_chunks;
         q.n_intra = p->n_intra;
@@ -1569,6 +1572,7 @@ int build_sub(h264g_ctx *c, const std::vector<const h264g_pic *> &pics, Batch *b
         std::vector<uint32_t> &ch = p->mbaff ? mchunks : chunks;
         for (uint32_t a = 0; a < (uint32_t)(p->W * p->H); a += MB_CHUNK) ch.push_back((i << WI_PIC_SHIFT) | a);
         (p->mbaff ? b->n_mintra : b->n_intra) += p->n_intra;
+        if (p->mbaff) b->mpair_rows = std::max(b->mpair_rows, (uint32_t)p->H / 2);
         (p->mbaff ? any_mdbk : any_dbk) |= p->desc.disable_deblocking_filter_idc != 1;
         maxt = std::max(maxt, (p->W - 1) + 2 * (p->H - 1));
     }
@@ -1705,6 +1709,7 @@ StageSet batch_stages(const Batch *b) {
     q.intra = b->d_intra;
     q.n_intra = b->n_intra;
     q.n_mintra = b->n_mintra;
+    q.mpair_rows = b->mpair_rows;
     q.all = b->d_all;
     q.n_all = b->n_all;
     q.rows = b->d_rows;

@@ -187,8 +187,12 @@ int h264g_launch_intra_band(const DevPic *pics, const uint32_t *bands, uint32_t 
 #define H264G_DBK_MAX_ROWS 4
 int h264g_launch_deblock_band(const DevPic *pics, const uint32_t *bands, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                               int rows, uint32_t *err, void *stream);
-// Deblocking of the MBAFF frames among the launch's pictures, one workgroup per picture.
-int h264g_launch_deblock_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *err, void *stream);
+// Deblocking of the MBAFF frames among the launch's pictures, in bands of H264G_MBAFF_ROWS of
+// their at most pair_rows rows of MB pairs.  (A band of 4 pair rows hands down 512 B per pair
+// column, as much as the two bands of 4 MB rows that a stream's strips have in its place.)
+#define H264G_MBAFF_ROWS 4
+int h264g_launch_deblock_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t pair_rows, DevCtl *ctl, uint32_t *epoch, uint32_t *err,
+                               void *stream);
 int h264g_launch_bgr24(const uint8_t *yuv, int wl, int hl, uint8_t *bgr, uint32_t stride, int flip, void *stream);
 int h264g_launch_copy(const uint8_t *src, uint8_t *dst, uint64_t bytes, void *stream);
 }

@@ -2454,48 +2454,7 @@ __global__ __launch_bounds__(WAVE) void k_deblock(const DevPic *__restrict__ pic
     retire(ctl, gridDim.x, epoch_p, epoch);
 }
 
-// ---- deblocking of MBAFF frames, one MB pair per wave at a time
-// 8.7 in MB address order (Deblock.cpp:76-635): the pair's top MB, then its bottom MB.
-// Pair (x, y) follows pair (x - 1, y), whose right columns its left edges filter, and
-// pair (x + 1, y - 1), whose left edges filter the right columns of pair (x, y - 1) that
-// its top edges read (k_deblock_mbaff).  The wave works on an LDS copy of the samples its
-// edges touch: luma rows -8..31 (a field MB's top edge reads four rows of its parity above
-// the pair) by columns -4..15, chroma rows -8..15 by columns -4..7, written back afterwards.
-constexpr int MR_LROWS = 40, MR_LCOLS = 20, MR_CROWS = 24, MR_CCOLS = 12, MR_ROW0 = 8, MR_COL0 = 4;
-struct alignas(16) MbaffRegion {
-    uint8_t L[MR_LROWS][MR_LCOLS];
-    uint8_t C[2][MR_CROWS][MR_CCOLS];
-};
-
-// Copies the pair's region between the picture and LDS (to_lds: load, else store).
-// Columns left of the picture and rows above it are skipped.
-__device__ void mbaff_region(const DevPic &P, int px, int py, MbaffRegion *rg, bool to_lds) {
-    const int lane = wave_lane(), wl = P.W * 16, wc = P.W * 8;
-    uint8_t *y = slot_base(P, P.dst), *cb = y + (uint64_t)wl * (P.H * 16), *cr = cb + (uint64_t)wc * (P.H * 8);
-    // dwords: luma rows x 5, then chroma planes x rows x 3
-    constexpr int NL = MR_LROWS * 5, NC = MR_CROWS * 3;
-    for (int i = lane; i < NL + 2 * NC; i += WAVE) {
-        uint8_t *pic, *lds;
-        int r, d;
-        if (i < NL) {
-            r = i / 5 - MR_ROW0;
-            d = i % 5;
-            if ((py == 0 && r < 0) || (px == 0 && d == 0)) continue;
-            pic = y + (uint64_t)(py * 32 + r) * wl + px * 16 - 4 + 4 * d;
-            lds = &rg->L[r + MR_ROW0][4 * d];
-        } else {
-            const int k = i - NL, c = k / NC;
-            r = (k % NC) / 3 - MR_ROW0;
-            d = (k % NC) % 3;
-            if ((py == 0 && r < 0) || (px == 0 && d == 0)) continue;
-            pic = (c ? cr : cb) + (uint64_t)(py * 16 + r) * wc + px * 8 - 4 + 4 * d;
-            lds = &rg->C[c][r + MR_ROW0][4 * d];
-        }
-        if (to_lds) *(uint32_t *)lds = *(const uint32_t *)pic;
-        else *(uint32_t *)pic = *(const uint32_t *)lds;
-    }
-}
-
+// ---- deblocking of MBAFF frames
 // 8.7.2.1 (Deblock.cpp:994-1310) in an MBAFF frame, for the luma positions (xp, yp) of p0
 // in MB ap and (xq, yq) of q0 in MB aq: mixedModeEdgeFlag between a frame and a field MB;
 // bS 4 at MB edges between frame MBs and at vertical MB edges, 3 at the other intra edges;
@@ -2636,148 +2595,324 @@ __device__ __forceinline__ void bs_mbaff_mb(const DevPic *pics, const uint32_t *
                          (nb.field ? DBQ_FIELD : 0u);
 }
 
-// One edge pass of a MB (8.7.1, Deblock.cpp:639-990) on the pair's LDS region: lane k of a
-// plane (luma lanes 0-15, Cb 16-23, Cr 24-31; act: the lane's plane takes part) owns line k.
-// e: the edge's x (vertical) or y (horizontal) inside the MB; lines of a field-mode pass are
-// two rows apart (dy = 1 + fieldMode), and yE % 2 picks the bottom-field lines of a frame MB's
-// top edge over a field pair.  bS: the lane's strength; qp: the deblocking word of the MB
-// holding p0, qq: of the MB.
-__device__ __forceinline__ void mbaff_edge(const DevPic &P, MbaffRegion *rg, const DbkTables *tb, int lrow0, int crow0, bool act,
-                                           bool vertical, int e, int fieldMode, int bS, uint32_t qp, uint32_t qq) {
-    const int lane = wave_lane();
-    const int plane = lane < 16 ? 0 : (lane < 24 ? 1 : 2), chroma = plane != 0;
-    const int k = chroma ? (lane & 7) : (lane & 15), dy = 1 + fieldMode;
-    act = act && lane < 32;
-    uint8_t *base = chroma ? &rg->C[plane - 1][0][0] : &rg->L[0][0];
-    const int pitch = chroma ? MR_CCOLS : MR_LCOLS, row0 = MR_ROW0 + (chroma ? crow0 : lrow0);
-    const int xE = vertical ? e : k, yE = vertical ? k : e;
-    int qi[4], pi[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (vertical) {
-            qi[i] = (row0 + dy * yE) * pitch + MR_COL0 + xE + i;
-            pi[i] = (row0 + dy * yE) * pitch + MR_COL0 + xE - i - 1;
-        } else {
-            qi[i] = (row0 + dy * (yE + i) - (yE & 1)) * pitch + MR_COL0 + xE;
-            pi[i] = (row0 + dy * (yE - i - 1) - (yE & 1)) * pitch + MR_COL0 + xE;
-        }
-    }
-    uint32_t w[5] = {0, 0, 0, 0, 0};
-    int alpha = 0, beta = 0, tc0 = 0;
-    act = act && bS != 0;
-    if (act) {
-        w[0] = pack4(base[pi[3]], base[pi[2]], base[pi[1]], base[pi[0]]);
-        w[1] = pack4(base[qi[0]], base[qi[1]], base[qi[2]], base[qi[3]]);
-        const int qav = (dbq_qp(qp, plane) + dbq_qp(qq, plane) + 1) >> 1;
-        const int ia = clip3(0, 51, qav + P.offA), ib = clip3(0, 51, qav + P.offB);
-        alpha = tb->alpha[ia];
-        beta = tb->beta[ib];
-        tc0 = bS >= 1 && bS <= 3 ? tb->tc0[bS - 1][ia] : 0;
-    }
-    dbk_line_edge<0>(w, act, !chroma, bS, alpha, beta, tc0);
-    if (act) {
-        base[pi[0]] = (uint8_t)(w[0] >> 24);
-        base[pi[1]] = (uint8_t)(w[0] >> 16);
-        base[pi[2]] = (uint8_t)(w[0] >> 8);
-        base[qi[0]] = (uint8_t)w[1];
-        base[qi[1]] = (uint8_t)(w[1] >> 8);
-        base[qi[2]] = (uint8_t)(w[1] >> 16);
-    }
-    wave_sync();
+// ds_read_b64_tr_b8: in each group of 16 lanes, lanes 2j and 2j + 1 name the two 8-byte
+// halves of row j (j < 8) of an 8 x 16 byte matrix and lane i gets its column i, byte j
+// from row j.  Every lane of the wave takes part.
+__device__ __forceinline__ uint2 lds_tr(const uint8_t *p) {
+    typedef int v2i __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) v2i lds_v2i;
+    const v2i r = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)p);
+    return make_uint2((uint32_t)r.x, (uint32_t)r.y);
 }
 
-// The edges of one MB of the pair in the reference's order (Deblock.cpp:76-635): luma
-// left, internal vertical, top (twice, in field mode, for a frame MB under a field pair:
-// its top field lines against the pair's top MB, its bottom field lines against the bottom
-// MB; chroma against the bottom MB both times, quirk Q5), internal horizontal; chroma in
-// the same order, each chroma pass beside a luma pass (different planes).  bs: the MB's 32 bytes of
-// strengths in LDS; q: deblocking words of the pair, of the left pair, of the pair above (top
-// MB, bottom MB each).
-__device__ __forceinline__ void deblock_mb_mbaff(const DevPic &P, int addr, MbaffRegion *rg, const DbkTables *tb, const uint8_t *bs,
-                                                 const uint32_t (&q)[6]) {
-    const int lane = wave_lane(), W = P.W, pair = addr >> 1, bot = addr & 1;
-    const uint32_t own = q[bot];
-    const MbaffNb nb = mbaff_nb(W, addr, (own & DBQ_FIELD) != 0, (q[2] & DBQ_FIELD) != 0, (q[4] & DBQ_FIELD) != 0, dbq_t8(own));
-    const int fm = nb.field ? 1 : 0, lrow0 = nb.field ? bot : 16 * bot, crow0 = nb.field ? bot : 8 * bot;
-    const bool luma = lane < 16, chroma = lane >= 16;
-    const int k = luma ? lane : lane & 7;
+// ---- deblocking of MBAFF frames over bands of pair rows
+// 8.7 (Deblock.cpp:76-635) takes the MBs in address order: a pair's top MB, then its bottom MB,
+// each with its vertical edges, left to right, then its horizontal ones, top to bottom.  A band
+// is MBAFF_ROWS rows of MB pairs on one workgroup, a wave per row and one more that brings in
+// what the band above hands down.
+//
+// Of one pair, the vertical edges of both MBs go together, half a wave each (luma lines in lanes
+// 0-15, Cb 16-23, Cr 24-31): the top MB's horizontal edges touch no row of a bottom frame MB, and
+// no line of the other field.  So do the horizontal edges of a field pair; a frame pair's eight
+// follow one another on lanes 0-31, and the two passes over the top edge of a frame MB under a
+// field pair, each on the lines of one field, go half a wave each before them.  A line is held in
+// registers for all its edges.
+//
+// Pair (x, y) takes the bottom 8 rows of pair (x, y - 1) over from that pair's wave, which has
+// left them to it (a field MB's top edge reads four and filters three rows of its parity), once
+// pair (x + 1, y - 1) has filtered its right columns; from then on they are its own to store.
+// They travel through a ring in LDS, between bands as epoch-tagged words in device memory.
+//
+// Bound: the chain of W + 2 HP steps of about 3 us, what the lines of one pair take one wave.
+// Measured (1920x1088, one launch): 560 us; with one workgroup of 16 waves for the picture, an edge of one MB
+// at a time and the samples in device memory between pairs 3300; before that, with a persistent
+// wave and a progress word in device memory per pair, 112000.
+constexpr int MBAFF_ROWS = H264G_MBAFF_ROWS, MRING_SLOTS = 8, MRING_WORDS = 64;
+// One pair's samples: luma rows -8..31 by columns -4..15, chroma rows -8..15 by columns -4..7;
+// column -4 at byte 4 of a row, so that column 0 is aligned for ds_read_b64_tr_b8.
+constexpr int MR_ROW0 = 8, MR_LP = 24, MR_CP = 16;
+struct alignas(16) MbaffRegion {
+    uint8_t L[40][MR_LP];
+    uint8_t C[2][24][MR_CP];
+    uint8_t pad[16];           // (a chroma line is read as if it were as long as a luma line)
+};
+struct MbaffDbkShared {
+    MbaffRegion rg[MBAFF_ROWS];
+    uint32_t bs[MBAFF_ROWS][16];                       // the pair's strengths (MBS_*)
+    uint32_t ring[MBAFF_ROWS][MRING_SLOTS][MRING_WORDS];  // [w]: what row w takes over
+    uint32_t prog[MBAFF_ROWS + 1], cons[MBAFF_ROWS + 1];  // pairs in ring[w], pairs read from it
+    DbkTables tb;
+};
+
+// Edges of a line: the MB edge with deblocking word qe beyond it, then the internal ones (luma 4,
+// 8, 12, chroma 4).  bs: strength nibbles of the MB; be, bi: nibble of the MB edge / of the first
+// internal one.
+__device__ __forceinline__ void mbaff_line(uint32_t (&w)[5], const DevPic &P, const DbkTables *tb, const uint8_t *bs, int be, int bi,
+                                           uint32_t qe, uint32_t qq, int plane, bool act) {
+    const bool luma = plane == 0;
     auto bs_at = [&](int n) -> int { return (bs[n >> 1] >> (4 * (n & 1))) & 15; };
-    const int seg = luma ? k >> 2 : k >> 1;
-    // left MB edge: a frame MB beside a field pair alternates between its MBs (quirk Q6 is in bS)
-    const uint32_t ql = nb.leftMix ? ((k & 1) ? q[3] : q[2]) : ((nb.mbA & 1) ? q[3] : q[2]);
-    const uint32_t qt = nb.mbB == addr - 1 && bot ? q[0] : ((nb.mbB & 1) ? q[5] : q[4]);
-    const int vi = luma ? 0 : 4;  // chroma edge 4 takes the strengths of luma edge 8
-    mbaff_edge(P, rg, tb, lrow0, crow0, nb.left, true, 0, fm, bs_at(luma ? MBS_LEFT + k : MBS_LEFT_C + k), ql, own);
-    mbaff_edge(P, rg, tb, lrow0, crow0, true, true, 4, fm, bs_at(MBS_V + vi + seg), own, own);
-    mbaff_edge(P, rg, tb, lrow0, crow0, luma, true, 8, fm, bs_at(MBS_V + 4 + seg), own, own);
-    mbaff_edge(P, rg, tb, lrow0, crow0, luma, true, 12, fm, bs_at(MBS_V + 8 + seg), own, own);
-    if (nb.topMix) {
-        mbaff_edge(P, rg, tb, lrow0, crow0, true, false, 0, 1, bs_at((luma ? MBS_TOP : MBS_TOP_C) + seg), luma ? q[4] : q[5], own);
-        mbaff_edge(P, rg, tb, lrow0, crow0, true, false, 1, 1, bs_at((luma ? MBS_TOP2 : MBS_TOP2_C) + seg), q[5], own);
-    } else {
-        mbaff_edge(P, rg, tb, lrow0, crow0, nb.upper, false, 0, fm, bs_at((luma ? MBS_TOP : MBS_TOP_C) + seg), qt, own);
-    }
-    mbaff_edge(P, rg, tb, lrow0, crow0, true, false, 4, fm, bs_at(MBS_H + vi + seg), own, own);
-    mbaff_edge(P, rg, tb, lrow0, crow0, luma, false, 8, fm, bs_at(MBS_H + 4 + seg), own, own);
-    mbaff_edge(P, rg, tb, lrow0, crow0, luma, false, 12, fm, bs_at(MBS_H + 8 + seg), own, own);
-    (void)chroma;
-    (void)pair;
+    const int b0 = be < 0 ? 0 : bs_at(max(be, 0)), b1 = bs_at(luma ? bi : bi + 4), b2 = bs_at(bi + 4), b3 = bs_at(bi + 8);
+    const int q = dbq_qp(qq, plane), qa = (dbq_qp(qe, plane) + q + 1) >> 1;
+    const int ia = clip3(0, 51, qa + P.offA), ib = clip3(0, 51, qa + P.offB), ja = clip3(0, 51, q + P.offA), jb = clip3(0, 51, q + P.offB);
+    auto tc = [&](int b, int i) -> int { return tb->tc0[clip3(0, 2, b - 1)][i]; };  // (used for bS 1..3)
+    const int a0 = tb->alpha[ia], e0 = tb->beta[ib], ai = tb->alpha[ja], ei = tb->beta[jb];
+    const int t0 = tc(b0, ia), t1 = tc(b1, ja), t2 = tc(b2, ja), t3 = tc(b3, ja);
+    dbk_line_edge<0>(w, act, luma, b0, a0, e0, t0);
+    dbk_line_edge<1>(w, act, luma, b1, ai, ei, t1);
+    dbk_line_edge<2>(w, act && luma, luma, b2, ai, ei, t2);
+    dbk_line_edge<3>(w, act && luma, luma, b3, ai, ei, t3);
 }
 
-// One workgroup per picture (which an MBAFF frame uses), a wave per row of MB pairs: wave w takes pair rows w, w + nw, ...
-// and walks each from left to right.  The picture's samples travel between the rows through
-// the CU's caches (workgroup scope: no L2 write-back or invalidation), their order through
-// LDS counters: pair (x, y) follows pair (x + 1, y - 1).  The strengths of the next pair are
-// loaded while this one is filtered.
-// Bound: the chain of W pairs per row and ceil(HP / 16) rows per wave, 20 edges a pair.  One
-// persistent wave per pair and a progress word per pair in device memory, with the strengths
-// derived inside the chain, took 112 ms per 1920x1088 launch, this 3.3 ms: every poll and
-// publication was an agent-scope acquire or release, an invalidation or write-back of the
-// XCD's whole L2.
-constexpr int MBAFF_WAVES = 16;
-__global__ __launch_bounds__(WAVE *MBAFF_WAVES) void k_deblock_mbaff(const DevPic *__restrict__ pics, uint32_t n, uint32_t *err) {
-    __shared__ MbaffRegion rgs[MBAFF_WAVES];
-    __shared__ alignas(16) uint8_t bss[MBAFF_WAVES][64];
-    __shared__ DbkTables tb;
-    __shared__ uint32_t prog[512];  // pairs of each pair row finished
-    dbk_tables_init(&tb);
-    for (int i = threadIdx.x; i < 512; i += blockDim.x) prog[i] = 0;
-    __syncthreads();
-    if (blockIdx.x >= n) return;
-    const DevPic &P = pics[blockIdx.x];
-    if (!P.mbaff || P.dbk_idc == 1) return;
-    const int W = P.W, HP = P.H >> 1, w = (int)uniform(threadIdx.x / WAVE), nw = blockDim.x / WAVE, lane = wave_lane();
-    MbaffRegion *const rg = &rgs[w];
+// One row of pairs, on wave w of the workgroup: rows y0 .. y1 - 1 are the band's.  out: the
+// strips to the next band (its last row writes them), W x MRING_WORDS words.
+__device__ __forceinline__ void mbaff_dbk_row(const DevPic &P, int w, int y, int y1, GAS uint64_t *out, MbaffDbkShared &sh,
+                                              uint32_t epoch, uint32_t *err) {
+    const int lane = wave_lane(), W = P.W, HP = P.H >> 1;
+    const int h = lane >> 5, l32 = lane & 31, plane = l32 < 16 ? 0 : (l32 < 24 ? 1 : 2), k = plane == 0 ? l32 : l32 & 7;
+    const bool luma = plane == 0, last_row = y == HP - 1, ring_out = y + 1 < y1;
+    const int seg = luma ? k >> 2 : k >> 1, hs = luma ? 16 : 8;
+    const DbkPlanes d = dbk_planes(P);
+    MbaffRegion *const rg = &sh.rg[w];
+    const uint8_t *const bsb = (const uint8_t *)sh.bs[w];
     const GAS uint32_t *const dq = G(P.dbq);
-    for (int y = w; y < HP; y += nw) {
-        uint32_t bsw = ((const GAS uint32_t *)(G(P.bs) + (size_t)(y * W) * 64))[lane & 15];
-        uint32_t q0 = dq[2 * (y * W)], q1 = dq[2 * (y * W) + 1], l0 = 0u, l1 = 0u;
-        for (int x = 0; x < W; x++) {
-            const int pair = y * W + x;
-            if (lane < 16) *(uint32_t *)&bss[w][4 * lane] = bsw;
-            const uint32_t q[6] = {uniform(q0), uniform(q1), l0, l1, y > 0 ? uniform(dq[2 * (pair - W)]) : 0u,
-                                   y > 0 ? uniform(dq[2 * (pair - W) + 1]) : 0u};
-            if (x + 1 < W) {
-                bsw = ((const GAS uint32_t *)(G(P.bs) + (size_t)(pair + 1) * 64))[lane & 15];
-                q0 = dq[2 * pair + 2];
-                q1 = dq[2 * pair + 3];
+    // the lane's line as a row / as a column of the region
+    uint8_t *const rows = luma ? &rg->L[MR_ROW0][4] : &rg->C[plane - 1][MR_ROW0][4];
+    const int pitch = luma ? MR_LP : MR_CP, rmax = luma ? 31 : 15;
+    uint8_t *const col = rows + 4 + k;
+    // ds_read_b64_tr_b8: the lane's 8-byte half of row tj of its group's 8 x 16 block (chroma: Cb | Cr)
+    const int tj = (lane & 15) >> 1;
+    const uint8_t *const tr = luma ? &rg->L[MR_ROW0][8 + 8 * (lane & 1)] : &rg->C[lane & 1][MR_ROW0][8];
+    // samples of the pair, one pair ahead: luma rows 0..31, chroma rows 0..15 twice, on lanes 0-31
+    const int r32 = lane & 31, cp = r32 >> 4, cr = r32 & 15;
+    const GAS uint8_t *const gl = G(d.y) + (uint64_t)(y * 32 + r32) * d.wl;
+    const GAS uint8_t *const gc = G(cp ? d.cr : d.cb) + (uint64_t)(y * 16 + cr) * d.wc;
+    // where it is stored: luma rows -8..31 on lanes 0-39, chroma rows -8..15 twice on lanes 0-47
+    const int slr = lane - MR_ROW0, sp = lane >= 24 ? 1 : 0, scr = lane - 24 * sp - MR_ROW0;
+    const bool sl = lane < 40 && (slr >= 0 || y > 0) && (slr < 24 || last_row);
+    const bool sc = lane < 48 && (scr >= 0 || y > 0) && (scr < 8 || last_row);
+    GAS uint8_t *const ol = G(d.y) + (int64_t)(y * 32 + (sl ? slr : 0)) * d.wl;
+    GAS uint8_t *const oc = G(sp ? d.cr : d.cb) + (int64_t)(y * 16 + (sc ? scr : 0)) * d.wc;
+    // the dword this lane hands down: (luma) row 24 + hr, (chroma) row 8 + hr of the pair
+    const int hp = h ? 1 + (l32 >> 4) : 0, hr = h ? (l32 >> 1) & 7 : l32 >> 2, hd = h ? l32 & 1 : l32 & 3;
+    const uint8_t *const hrow = h ? &rg->C[hp - 1][16 + hr][4] : &rg->L[32 + hr][4];
+    const int hw = h ? 32 + (hp - 1) * 16 + hr * 2 : hr * 4, hn = h ? 2 : 4;  // its row's words in a strip, their number
+    uint4 lrow = *(const GAS uint4 *)gl;
+    uint2 crow = *(const GAS uint2 *)gc;
+    uint32_t bsw = ((const GAS uint32_t *)(G(P.bs) + (size_t)(y * W) * 64))[lane & 15];
+    uint32_t n0 = dq[2 * (y * W)], n1 = dq[2 * (y * W) + 1], u0 = y > 0 ? dq[2 * (y * W - W)] : 0u, u1 = y > 0 ? dq[2 * (y * W - W) + 1] : 0u;
+    uint32_t left0 = 0u, left1 = 0u;
+    uint2 s0, s1, s2;          // the last pair's samples, stored after this pair's have arrived
+    uint32_t s3 = 0u, s4 = 0u;
+    s0 = s1 = s2 = make_uint2(0u, 0u);
+    auto store = [&](int x) {
+        if (sl) {
+            *(GAS uint4 *)(ol + x * 16) = make_uint4(s0.x, s0.y, s1.x, s1.y);
+            if (x > 0 && slr >= 0) *(GAS uint32_t *)(ol + x * 16 - 4) = s3;
+        }
+        if (sc) {
+            *(GAS uint2 *)(oc + x * 8) = s2;
+            if (x > 0 && scr >= 0) *(GAS uint32_t *)(oc + x * 8 - 4) = s4;
+        }
+    };
+    for (int x = 0; x < W; x++) {
+        const int pair = y * W + x;
+        // ---- the pair into the region; the last pair's right columns become the left ones
+        {
+            uint8_t *const lr = lane < 32 ? &rg->L[MR_ROW0 + r32][4] : &rg->C[cp][MR_ROW0 + cr][4];
+            const uint32_t c = *(const uint32_t *)(lr + (lane < 32 ? 16 : 8));
+            wave_sync();
+            *(uint32_t *)lr = c;
+            if (lane < 32) {
+                *(uint2 *)&rg->L[MR_ROW0 + r32][8] = make_uint2(lrow.x, lrow.y);
+                *(uint2 *)&rg->L[MR_ROW0 + r32][16] = make_uint2(lrow.z, lrow.w);
             }
+            wave_sync();
+            if (lane < 32) *(uint2 *)&rg->C[cp][MR_ROW0 + cr][8] = crow;
+            if (lane < 16) sh.bs[w][lane] = bsw;
+        }
+        const uint32_t q0 = uniform(n0), q1 = uniform(n1), a0 = uniform(u0), a1 = uniform(u1);
+        if (x > 0) store(x - 1);
+        if (x + 1 < W) {
+            lrow = *(const GAS uint4 *)(gl + (x + 1) * 16);
+            crow = *(const GAS uint2 *)(gc + (x + 1) * 8);
+            bsw = ((const GAS uint32_t *)(G(P.bs) + (size_t)(pair + 1) * 64))[lane & 15];
+            n0 = dq[2 * pair + 2];
+            n1 = dq[2 * pair + 3];
             if (y > 0) {
-                lds_wait(&prog[y - 1], 0u, (uint32_t)min(x + 2, W), err);
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                u0 = dq[2 * (pair - W) + 2];
+                u1 = dq[2 * (pair - W) + 3];
             }
-            mbaff_region(P, x, y, rg, true);
+        }
+        wave_sync();
+        const bool field = (q0 & DBQ_FIELD) != 0, lfield = (left0 & DBQ_FIELD) != 0, afield = (a0 & DBQ_FIELD) != 0;
+        const uint32_t own = h ? q1 : q0;
+        const uint8_t *const bs = bsb + 32 * h;
+        uint32_t wv[5];
+        // ---- vertical edges.  A frame MB beside a field pair alternates between its MBs, a field
+        // MB beside a frame pair takes its top one
+        {
+            const uint32_t qe = field == lfield ? (h ? left1 : left0) : !field && (k & 1) ? left1 : left0;
+            uint8_t *const r = rows + pitch * (field ? h + 2 * k : hs * h + k);
+            wv[0] = *(const uint32_t *)r;
+            const uint2 m0 = *(const uint2 *)(r + 4), m1 = *(const uint2 *)(r + 12);
+            wv[1] = m0.x; wv[2] = m0.y; wv[3] = m1.x; wv[4] = m1.y;
+            mbaff_line(wv, P, &sh.tb, bs, luma ? MBS_LEFT + k : MBS_LEFT_C + k, MBS_V + seg, qe, own, plane, true);
+            *(uint32_t *)r = wv[0];
+            *(uint2 *)(r + 4) = make_uint2(wv[1], wv[2]);
+            if (luma) *(uint2 *)(r + 12) = make_uint2(wv[3], wv[4]);
+        }
+        // ---- the rows above
+        if (y > 0) {
+            lds_wait(&sh.prog[w], 0u, (uint32_t)x + 1u, err);
+            const uint32_t v = sh.ring[w][x % MRING_SLOTS][lane];
+            uint8_t *const to = h ? &rg->C[hp - 1][hr][8 + 4 * hd] : &rg->L[hr][8 + 4 * hd];
+            *(uint32_t *)to = v;
+            lds_post(&sh.cons[w], (uint32_t)x + 1u);
+        }
+        wave_sync();
+        // ---- horizontal edges
+        const int top = luma ? MBS_TOP : MBS_TOP_C, hin = MBS_H + seg;
+        auto blk = [&](int dy, int r0, int s) -> uint2 { return lds_tr(tr + pitch * min(r0 + dy * (s + tj), rmax)); };
+        auto put = [&](uint8_t *c, int dy, uint32_t v) {
+            c[0] = (uint8_t)v;
+            c[dy * pitch] = (uint8_t)(v >> 8);
+            c[2 * dy * pitch] = (uint8_t)(v >> 16);
+            c[3 * dy * pitch] = (uint8_t)(v >> 24);
+        };
+        if (field) {  // each MB on the lines of its field
+            const uint2 A = blk(2, h, -4), B = blk(2, h, 4), C = blk(2, h, 12);
+            wv[0] = A.x; wv[1] = A.y; wv[2] = B.x; wv[3] = B.y; wv[4] = C.x;
+            mbaff_line(wv, P, &sh.tb, bs, top + seg, hin, h || !afield ? a1 : a0, own, plane, true);
             wave_sync();
-            deblock_mb_mbaff(P, 2 * pair, rg, &tb, bss[w], q);
-            deblock_mb_mbaff(P, 2 * pair + 1, rg, &tb, bss[w] + 32, q);
-            mbaff_region(P, x, y, rg, false);
+            uint8_t *const c = col + pitch * h;
+            if (y > 0) put(c - 8 * pitch, 2, wv[0]);
+            put(c, 2, wv[1]);
+            put(c + 8 * pitch, 2, wv[2]);
+            if (luma) {
+                put(c + 16 * pitch, 2, wv[3]);
+                put(c + 24 * pitch, 2, wv[4]);
+            }
+        } else {
+            if (afield) {  // top edge under a field pair: the lines of each field
+                const uint2 A = blk(2, h, -4);
+                wv[0] = A.x; wv[1] = A.y;
+                const int n = (h ? (luma ? MBS_TOP2 : MBS_TOP2_C) : top) + seg;
+                const int b = (bsb[n >> 1] >> (4 * (n & 1))) & 15, qa = (dbq_qp(h || !luma ? a1 : a0, plane) + dbq_qp(q0, plane) + 1) >> 1;
+                const int ia = clip3(0, 51, qa + P.offA);
+                dbk_line_edge<0>(wv, true, luma, b, sh.tb.alpha[ia], sh.tb.beta[clip3(0, 51, qa + P.offB)], sh.tb.tc0[clip3(0, 2, b - 1)][ia]);
+                wave_sync();
+                put(col + pitch * (h - 8), 2, wv[0]);
+                put(col + pitch * h, 2, wv[1]);
+                wave_sync();
+            }
+            const uint2 A = blk(1, 0, -4), B = blk(1, 0, 4), C = blk(1, 0, 12), D = blk(1, 0, 20), E = blk(1, 0, 28);
+            wv[0] = A.x; wv[1] = A.y; wv[2] = B.x; wv[3] = B.y; wv[4] = C.x;
+            mbaff_line(wv, P, &sh.tb, bsb, afield ? -1 : top + seg, hin, a1, q0, plane, h == 0);
+            uint32_t wb[5] = {luma ? wv[4] : wv[2], luma ? C.y : B.y, luma ? D.x : C.x, D.y, E.x};
+            mbaff_line(wb, P, &sh.tb, bsb + 32, top + seg, hin, q0, q1, plane, h == 0);
             wave_sync();
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            __hip_atomic_store(&prog[y], (uint32_t)x + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            l0 = q[0];
-            l1 = q[1];
+            if (h == 0) {
+                if (y > 0) put(col - 4 * pitch, 1, wv[0]);
+                put(col, 1, wv[1]);
+                if (luma) {
+                    put(col + 4 * pitch, 1, wv[2]);
+                    put(col + 8 * pitch, 1, wv[3]);
+                    put(col + 12 * pitch, 1, wb[0]);
+                    put(col + 16 * pitch, 1, wb[1]);
+                    put(col + 20 * pitch, 1, wb[2]);
+                    put(col + 24 * pitch, 1, wb[3]);
+                    put(col + 28 * pitch, 1, wb[4]);
+                } else {
+                    put(col + 4 * pitch, 1, wb[0]);
+                    put(col + 8 * pitch, 1, wb[1]);
+                    put(col + 12 * pitch, 1, wb[2]);
+                }
+            }
+        }
+        wave_sync();
+        // ---- the bottom rows to the row below: columns -4..11, the last pair's to the end
+        if (!last_row) {
+            const uint32_t v = *(const uint32_t *)(hrow + 4 * hd), v2 = *(const uint32_t *)(hrow + 4 * hn);
+            const int hx = hd == 0 ? x - 1 : x, hi = hw + (hd == 0 ? hn - 1 : hd - 1);
+            if (ring_out) {
+                if (x >= MRING_SLOTS) lds_wait(&sh.cons[w + 1], 0u, (uint32_t)(x - MRING_SLOTS + 1), err);
+                if (hx >= 0) sh.ring[w + 1][hx % MRING_SLOTS][hi] = v;
+                if (x == W - 1 && hd == 0) {
+                    wave_sync();
+                    sh.ring[w + 1][x % MRING_SLOTS][hw + hn - 1] = v2;
+                }
+                lds_post(&sh.prog[w + 1], (uint32_t)(x == W - 1 ? W : x));
+            } else {
+                const uint64_t tag = (uint64_t)epoch << 32;
+                if (hx >= 0) __hip_atomic_store(&out[(size_t)hx * MRING_WORDS + hi], tag | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (x == W - 1 && hd == 0)
+                    __hip_atomic_store(&out[(size_t)x * MRING_WORDS + hw + hn - 1], tag | v2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        // ---- what goes to the picture
+        {
+            const uint8_t *const l = &rg->L[min(lane, 39)][4], *const c = &rg->C[sp][lane < 48 ? scr + MR_ROW0 : 0][4];
+            s3 = *(const uint32_t *)l;
+            s0 = *(const uint2 *)(l + 4);
+            s1 = *(const uint2 *)(l + 12);
+            s4 = *(const uint32_t *)c;
+            s2 = *(const uint2 *)(c + 4);
+        }
+        wave_sync();
+        left0 = q0;
+        left1 = q1;
+    }
+    store(W - 1);
+}
+
+// Brings the strips of the band above into ring 0, one pair after another.
+__device__ __forceinline__ void mbaff_strip_reader(const GAS uint64_t *sw, int W, MbaffDbkShared &sh, uint32_t epoch, uint32_t *err) {
+    const int lane = wave_lane();
+#pragma unroll 1
+    for (int x = 0; x < W; x++) {
+        if (x >= MRING_SLOTS) lds_wait(&sh.cons[0], 0u, (uint32_t)(x - MRING_SLOTS + 1), err);
+        uint64_t r;
+#pragma unroll 1
+        for (uint32_t it = 0;; ++it) {
+            r = __hip_atomic_load(&sw[(size_t)x * MRING_WORDS + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (__builtin_amdgcn_ballot_w64((uint32_t)(r >> 32) != epoch) == 0) break;
+            if (it >= SPIN_LIMIT) {
+                report_timeout(err);
+                return;
+            }
+            if ((it & 255u) == 255u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) return;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        sh.ring[0][x % MRING_SLOTS][lane] = (uint32_t)r;
+        lds_post(&sh.prog[0], (uint32_t)x + 1u);
+    }
+}
+
+// Workgroup t is band t / n of picture t mod n, n pictures; those that are no MBAFF frame or
+// have no such band have nothing to do.
+__global__ __launch_bounds__(WAVE *(MBAFF_ROWS + 1)) void k_deblock_mbaff(const DevPic *__restrict__ pics, uint32_t n, DevCtl *ctl,
+                                                                          uint32_t *epoch_p, uint32_t *err) {
+    __shared__ MbaffDbkShared sh;
+    __shared__ uint32_t s_ticket;
+    const uint32_t epoch = launch_epoch(epoch_p);
+    const int w = (int)uniform(threadIdx.x / WAVE);
+    if ((int)threadIdx.x <= MBAFF_ROWS) sh.cons[threadIdx.x] = 0;
+    dbk_tables_init(&sh.tb);
+    const uint32_t t = band_ticket(ctl, &s_ticket, sh.prog, MBAFF_ROWS + 1);
+    if (t < gridDim.x) {
+        const DevPic &P = pics[t % n];
+        const int b = (int)(t / n), HP = P.H >> 1, y0 = b * MBAFF_ROWS, y1 = min(HP, y0 + MBAFF_ROWS);
+        if (P.mbaff && P.dbk_idc != 1 && y0 < HP) {
+            GAS uint64_t *const strips = (GAS uint64_t *)G(P.gstrip);
+            const size_t strip = (size_t)P.W * MRING_WORDS;
+            if (w < MBAFF_ROWS) {
+                if (y0 + w < y1) mbaff_dbk_row(P, w, y0 + w, y1, strips + b * strip, sh, epoch, err);
+            } else if (b > 0) {
+                mbaff_strip_reader(strips + (b - 1) * strip, P.W, sh, epoch, err);
+            }
         }
     }
+    band_retire(ctl, epoch_p, epoch);
 }
 
 // Intra MBs of MBAFF frames: one workgroup per picture, waves over rows of MB pairs like
@@ -2911,16 +3046,6 @@ __device__ void dbk_lut_init(DbkLut *t) {
         t->at[a][bS] = bS < 1 || bS > 4 ? 0u : (uint32_t)c_alpha[a] | (bS < 4 ? (uint32_t)c_tc0[bS - 1][a] << 16 : 0u);
     }
     for (int i = threadIdx.x; i < 52; i += blockDim.x) t->beta[i] = (uint32_t)c_beta[i] * 0x10001u;
-}
-
-// ds_read_b64_tr_b8: in each group of 16 lanes, lanes 2j and 2j + 1 name the two 8-byte
-// halves of row j (j < 8) of an 8 x 16 byte matrix and lane i gets its column i, byte j
-// from row j.  Every lane of the wave takes part.
-__device__ __forceinline__ uint2 lds_tr(const uint8_t *p) {
-    typedef int v2i __attribute__((ext_vector_type(2)));
-    typedef __attribute__((address_space(3))) v2i lds_v2i;
-    const v2i r = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)p);
-    return make_uint2((uint32_t)r.x, (uint32_t)r.y);
 }
 
 // The value of the lane 16 below (row e of 16 lanes gets row e - 1; row 0 anything).
@@ -3758,9 +3883,12 @@ int h264g_launch_deblock_band(const DevPic *pics, const uint32_t *bands, uint32_
     return (int)hipGetLastError();
 }
 
-int h264g_launch_deblock_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *err, void *stream) {
-    if (n_pics == 0) return 0;
-    hipLaunchKernelGGL(k_deblock_mbaff, dim3(n_pics), dim3(WAVE * MBAFF_WAVES), 0, (hipStream_t)stream, pics, n_pics, err);
+int h264g_launch_deblock_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t pair_rows, DevCtl *ctl, uint32_t *epoch, uint32_t *err,
+                               void *stream) {
+    if (n_pics == 0 || pair_rows == 0) return 0;
+    const uint32_t bands = (pair_rows + MBAFF_ROWS - 1) / MBAFF_ROWS;
+    hipLaunchKernelGGL(k_deblock_mbaff, dim3(n_pics * bands), dim3(WAVE * (MBAFF_ROWS + 1)), 0, (hipStream_t)stream, pics, n_pics, ctl,
+                       epoch, err);
     return (int)hipGetLastError();
 }
 

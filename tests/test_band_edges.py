@@ -72,3 +72,23 @@ def test_mbaff_and_frame_pictures_in_one_batch():
             eng.batch_destroy(b)
             for p in pics:
                 eng.release(p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", [(1, 8), (2, 10), (7, 16), (8, 18), (9, 24), (17, 26)])
+def test_mbaff_band_cuts_match_oracle(size):
+    """MBAFF frames of whole bands of 4 pair rows, one row more and one less, narrower and wider
+    than what a row hands down at a time (8 pairs)."""
+    w, h = size
+    with Engine(device=0) as eng:
+        gen = Generator(3, width_mbs=w, height_mbs=h, n_frames=4, seed=0xBAA000 + w, qp_lo=26, qp_hi=51, intra_in_inter_permille=200)
+        assert gen.mbaff
+        sid = eng.open_stream_for(gen)
+        for i, desc, want in oracle_decode(gen):
+            p = eng.begin(sid, *gen.picture(i))
+            eng.submit(p)
+            eng.sync()
+            for got, ref, plane in zip(eng.readback(sid, desc.dst_slot), want[2], "YUV"):
+                assert np.array_equal(got, ref), (size, i, plane)
+            eng.release(p)
+        eng.close_stream(sid)
