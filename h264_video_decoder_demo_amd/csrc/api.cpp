@@ -1080,7 +1080,7 @@ int launch_stages(h264g_ctx *ctx, const StageSet &q, int lane, int parts, hipStr
                                               ctx->d_err, s)
                     : h264g_launch_intra(q.pics, q.intra, q.n_intra, &ctl[0], &ctl[2].ticket, ctx->d_err, ctx->waves, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "intra launch: %s", hipGetErrorString((hipError_t)e));
-        if (q.n_mintra) e = h264g_launch_intra_mbaff(q.pics, q.n_pics, ctx->d_err, s);
+        if (q.n_mintra) e = h264g_launch_intra_mbaff(q.pics, q.n_pics, q.mpair_rows, &ctl[0], &ctl[2].ticket, ctx->d_err, s);
         if (e) return h264g_set_error(H264G_E_DEVICE, "intra launch (MBAFF): %s", hipGetErrorString((hipError_t)e));
         if (ev) HIPCHK(hipEventRecord(ev[2], s));
         if (!q.dbk_off && ev) {

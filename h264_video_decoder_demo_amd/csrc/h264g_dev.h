@@ -168,8 +168,10 @@ int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, i
 // (initially 1; each launch's last wave advances it).
 int h264g_launch_intra(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                        uint32_t *err, int waves, void *stream);
-// Intra MBs of the MBAFF frames among the launch's pictures, one workgroup per picture.
-int h264g_launch_intra_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *err, void *stream);
+// Intra MBs of the MBAFF frames among the launch's pictures, in bands of H264G_MBAFF_ROWS of
+// their at most pair_rows rows of MB pairs (128 B handed down per pair column and band).
+int h264g_launch_intra_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t pair_rows, DevCtl *ctl, uint32_t *epoch, uint32_t *err,
+                             void *stream);
 int h264g_launch_deblock(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,
                          uint32_t *err, int waves, void *stream);
 int h264g_launch_deblock_rows(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch,

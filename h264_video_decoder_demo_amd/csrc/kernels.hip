@@ -942,7 +942,7 @@ __constant__ I4Taps c_i4taps = make_i4taps();
 // MB's first wave barrier in intra_mb.
 __device__ __forceinline__ void intra4_prep(const h264g_mb *mb, const Avail &av, WaveIntra *wi) {
     const int lane = wave_lane(), g = lane >> 4, j = lane & 15;
-#pragma unroll 1
+#pragma unroll  // (the loads of a step's modes and taps beside those of the others)
     for (int t = 0; t < 10; t++) {
         const int by = (t < 2 ? 0 : (t - 2) >> 1) + g, bx = t - 2 * by;
         const bool has = lane < 32 && bx >= 0 && by < 4;
@@ -1103,17 +1103,20 @@ __device__ __forceinline__ void intra_res_place(const IntraRes &r, WaveIntra *wi
 // Prediction and reconstruction of an intra MB whose residual intra_res_place left in
 // wi->res (res: the MB has levels); the neighbours it reads are final.  The LDS writes of
 // the residual are ordered before its first wave barrier.
-// An Intra_4x4 MB has run intra4_prep, an Intra_8x8 MB intra8_prep.
-template <bool MBAFF>
-__device__ __forceinline__ void intra_mb(const DevPic &P, int addr, WaveIntra *wi, const Avail &av, bool res) {
+// An Intra_4x4 MB has run intra4_prep, an Intra_8x8 MB intra8_prep.  PLANES: 1 luma, 2 chroma
+// (which share nothing that either writes), 3 both.
+struct IntraHdr {
+    int type, i16, chroma;     // mb_type, Intra16x16 and chroma prediction modes
+};
+template <int PLANES>
+__device__ __forceinline__ void intra_mb(const DevPic &P, const MbGeo &g, const IntraHdr &mb, WaveIntra *wi, const Avail &av, bool res) {
+    constexpr bool LUMA = PLANES & 1, CHROMA = PLANES & 2;
     const int lane = wave_lane();
-    const h264g_mb *mb = &G(P.mbs)[addr];
     const int W = P.W, H = P.H, wl = W * 16, hl = H * 16, wc = W * 8, hc = H * 8;
     // In an MBAFF frame every neighbouring sample that 6.4.12.2 (Table 6-4) gives an MB lies
     // in the MB's own view of the picture: frame rows for frame MBs, the rows of its parity
     // for field MBs (rows step apart from its first row), at the same columns; Table 6-4
     // only decides availability (the caller's av).
-    const MbGeo g = mb_geo<MBAFF>(P, addr);
     const int mbx = g.mbx, st = g.step;
     uint8_t *dst = slot_base(P, P.dst);
     uint8_t *dy = dst, *dcb = dst + (uint64_t)wl * hl, *dcr = dcb + (uint64_t)wc * hc;
@@ -1121,24 +1124,25 @@ __device__ __forceinline__ void intra_mb(const DevPic &P, int addr, WaveIntra *w
     if (lane < 25) {  // row -1, x = lane - 1
         int x = lane - 1;
         bool ok = x < 0 ? av.D() : (x < 16 ? av.B() : av.C());
-        if (ok) wi->T[0][lane] = dy[(uint64_t)(g.ly - st) * wl + mbx * 16 + x];
+        if (LUMA && ok) wi->T[0][lane] = dy[(uint64_t)(g.ly - st) * wl + mbx * 16 + x];
     } else if (lane < 41) {  // column -1
         int y = lane - 25;
-        if (av.A()) wi->T[y + 1][0] = dy[(uint64_t)(g.ly + y * st) * wl + mbx * 16 - 1];
+        if (LUMA && av.A()) wi->T[y + 1][0] = dy[(uint64_t)(g.ly + y * st) * wl + mbx * 16 - 1];
     } else if (lane < 59) {  // chroma row -1 (x = -1..7) for both planes
         int k = lane - 41, c = k / 9, x = k % 9 - 1;
         bool ok = x < 0 ? av.D() : av.B();
         const uint8_t *pl = c == 0 ? dcb : dcr;
-        if (ok) wi->C[c][0][x + 1] = pl[(uint64_t)(g.cy - st) * wc + mbx * 8 + x];
+        if (CHROMA && ok) wi->C[c][0][x + 1] = pl[(uint64_t)(g.cy - st) * wc + mbx * 8 + x];
     }
     if (lane < 16) {  // chroma column -1
         int c = lane >> 3, y = lane & 7;
         const uint8_t *pl = c == 0 ? dcb : dcr;
-        if (av.A()) wi->C[c][y + 1][0] = pl[(uint64_t)(g.cy + y * st) * wc + mbx * 8 - 1];
+        if (CHROMA && av.A()) wi->C[c][y + 1][0] = pl[(uint64_t)(g.cy + y * st) * wc + mbx * 8 - 1];
     }
     wave_sync();
     // ---- luma
-    if (mb->mb_type == H264G_MB_I4x4) {
+    if (!LUMA) {
+    } else if (mb.type == H264G_MB_I4x4) {
         // 4x4 blocks in wavefront order t = bx + 2 by, two blocks per step (lanes 0-15 and
         // 16-31): every neighbour a block reads has a smaller t, and a top-right block that
         // the reference's block order has not decoded yet (blocks 3, 11) counts as not
@@ -1170,7 +1174,7 @@ __device__ __forceinline__ void intra_mb(const DevPic &P, int addr, WaveIntra *w
             }
             wave_sync();
         }
-    } else if (mb->mb_type == H264G_MB_I8x8) {
+    } else if (mb.type == H264G_MB_I8x8) {
         // each block: gather its 25 reference samples at the indices intra8_prep found,
         // filter them, then one four-tap sum per pixel
         const uint8_t *Tf = &wi->T[0][0];
@@ -1229,7 +1233,7 @@ __device__ __forceinline__ void intra_mb(const DevPic &P, int addr, WaveIntra *w
             wave_sync();
         }
     } else {  // Intra_16x16, 8.3.3 (H264PictureBase.cpp:1847-2056)
-        int mode = mb->intra16x16_pred_mode;
+        int mode = mb.i16;
         int dc = 128, a = 0, bq = 0, cq = 0;
         if (mode == 2) {
             int st = 0, sl = 0;
@@ -1256,8 +1260,8 @@ __device__ __forceinline__ void intra_mb(const DevPic &P, int addr, WaveIntra *w
         wave_sync();
     }
     // ---- chroma, 8.3.4 (H264PictureBase.cpp:2076-2381); DC tests "> 0" (quirk Q1)
-    {
-        int mode = mb->intra_chroma_pred_mode;
+    if (CHROMA) {
+        int mode = mb.chroma;
         for (int k = 0; k < 2; k++) {
             int i = lane + k * WAVE, c = i >> 6, x = i & 7, y = (i >> 3) & 7;
             const uint8_t (*Cp)[9] = wi->C[c];
@@ -1290,7 +1294,7 @@ __device__ __forceinline__ void intra_mb(const DevPic &P, int addr, WaveIntra *w
         }
     }
     // ---- luma tile -> picture
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; LUMA && k < 4; k++) {
         int i = lane + k * WAVE, x = i & 15, y = i >> 4;
         dy[(uint64_t)(g.ly + y * st) * wl + mbx * 16 + x] = wi->T[y + 1][x + 1];
     }
@@ -1811,7 +1815,8 @@ __global__ __launch_bounds__(WAVE) void k_intra(const DevPic *__restrict__ pics,
         else if (G(P.mbs)[addr].mb_type == H264G_MB_I8x8) intra8_prep(&G(P.mbs)[addr], av, &lds);
         wait_deps(G(P.flags), deps, 4, epoch, err);
         intra_res_place(r, &lds);
-        intra_mb<false>(P, addr, &lds, av, r.res);
+        const GAS h264g_mb &m = G(P.mbs)[addr];
+        intra_mb<3>(P, mb_geo<false>(P, addr), {m.mb_type, m.intra16x16_pred_mode, m.intra_chroma_pred_mode}, &lds, av, r.res);
         publish(&G(P.flags)[addr], epoch);
     }
     retire(ctl, gridDim.x, epoch_p, epoch);
@@ -2915,47 +2920,181 @@ __global__ __launch_bounds__(WAVE *(MBAFF_ROWS + 1)) void k_deblock_mbaff(const 
     band_retire(ctl, epoch_p, epoch);
 }
 
-// Intra MBs of MBAFF frames: one workgroup per picture, waves over rows of MB pairs like
-// k_deblock_mbaff, the top MB of a pair before the bottom one.  An MB reads MBs of its own and
-// the left pair, earlier in its row, and of the pairs above up to x + 1; residual and tap
-// preparation go before the wait.  1920x1088: an I frame 40.0 to 5.6 ms, P and B frames (10 %
-// intra MBs) 10 to 0.6 ms, against persistent waves with progress words in device memory.
-constexpr int MBAFF_INTRA_WAVES = 16;
-__global__ __launch_bounds__(WAVE *MBAFF_INTRA_WAVES) void k_intra_mbaff(const DevPic *__restrict__ pics, uint32_t n, uint32_t *err) {
-    __shared__ WaveIntra tiles[MBAFF_INTRA_WAVES];
-    __shared__ uint32_t prog[512];
-    for (int i = threadIdx.x; i < 512; i += blockDim.x) prog[i] = 0;
-    __syncthreads();
-    if (blockIdx.x >= n) return;
-    const DevPic &P = pics[blockIdx.x];
-    if (!P.mbaff || P.n_intra == 0) return;
-    const int W = P.W, HP = P.H >> 1, w = (int)uniform(threadIdx.x / WAVE), nw = blockDim.x / WAVE;
-    for (int y = w; y < HP; y += nw)
-        for (int x = 0; x < W; x++) {
-            const int pair = y * W + x;
-            const uint32_t c0 = uniform(G(P.mbs)[2 * pair].mb_type), c1 = uniform(G(P.mbs)[2 * pair + 1].mb_type);
-            bool waited = y == 0;
+// Intra MBs of MBAFF frames over the same bands, the top MB of a pair before the bottom one.  An
+// MB reads MBs of its own and the left pair, earlier in its row, and of the pairs above up to
+// x + 1.  A row is three waves: one prepares the row's MBs up to two ahead (residual, tap
+// addresses, what the record says) in one of two tiles, one predicts luma and one chroma, whose
+// chains never meet.  Inside a band the samples travel through the CU's caches (workgroup scope).
+// A band's last row sends the two bottom rows of every pair with an intra MB to the next band as
+// epoch-tagged words, and that band's last wave writes them to where they stand already, so that
+// its workgroup's reads find them.
+// Bound: the chain of W + 2 HP pairs, with two trips through the caches per MB.  1920x1088: an I
+// frame 1.44 ms, P and B frames (10 % intra MBs) 0.15; with preparation, luma and chroma on one wave
+// 3.06 and 0.33; with one workgroup of 16 such waves per picture 5.4 and 0.6, with persistent
+// waves and progress words in device memory 40 and 10.
+constexpr int MISTRIP_WORDS = 16;  // luma rows 30, 31 in four dwords each, then two of Cb rows 14, 15 and of Cr
+constexpr int MBAFF_INTRA_WAVES = 3 * MBAFF_ROWS + 1;
+struct MbaffIntraRow {
+    WaveIntra tile[2];
+    uint32_t hdr[2][4];        // address, availability, residual flag and modes, field flag
+    uint32_t ready, done[2];   // MBs prepared, MBs whose luma / chroma is finished
+};
+struct MbaffIntraShared {
+    MbaffIntraRow row[MBAFF_ROWS];
+    uint32_t prog[2][MBAFF_ROWS + 1];  // [c][w]: pairs above row w whose luma / chroma is finished
+};
+// Whether the pairs x0 .. x0 + 63 of row y have an intra top (bottom) MB.
+struct PairMask {
+    uint64_t top, bot;
+};
+__device__ __forceinline__ PairMask mbaff_intra_pairs(const DevPic &P, int y, int x0) {
+    const int x = x0 + wave_lane();
+    const GAS h264g_mb *const m = G(P.mbs) + 2 * (y * P.W + min(x, P.W - 1));
+    return {__builtin_amdgcn_ballot_w64(x < P.W && cls_intra(m[0].mb_type)), __builtin_amdgcn_ballot_w64(x < P.W && cls_intra(m[1].mb_type))};
+}
+__device__ __forceinline__ void mbaff_intra_prep(const DevPic &P, int y, MbaffIntraRow &row, uint32_t *err) {
+    const int W = P.W, lane = wave_lane();
+    uint32_t n = 0;
+    for (int x0 = 0; x0 < W; x0 += WAVE) {
+        const PairMask pm = mbaff_intra_pairs(P, y, x0);
+        for (uint64_t todo = pm.top | pm.bot; todo; todo &= todo - 1) {
+            const int i = (int)__builtin_ctzll(todo);
             for (int h = 0; h < 2; h++) {
-                if (!cls_intra((int)(h ? c1 : c0))) continue;
-                const int addr = 2 * pair + h;
+                if (!(((h ? pm.bot : pm.top) >> i) & 1u)) continue;
+                const int addr = 2 * (y * W + x0 + i) + h;
+                const GAS h264g_mb *const m = &G(P.mbs)[addr];
+                WaveIntra *const tile = &row.tile[n & 1u];
                 const Avail av = intra_avail_mbaff(P, addr);
                 const IntraRes r = intra_res_fetch(P, addr);
-                if (G(P.mbs)[addr].mb_type == H264G_MB_I4x4) intra4_prep(&G(P.mbs)[addr], av, &tiles[w]);
-                else if (G(P.mbs)[addr].mb_type == H264G_MB_I8x8) intra8_prep(&G(P.mbs)[addr], av, &tiles[w]);
-                if (!waited) {
-                    lds_wait(&prog[y - 1], 0u, (uint32_t)min(x + 2, W), err);
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                    waited = true;
+                const uint32_t type = m->mb_type, modes = (uint32_t)m->intra16x16_pred_mode << 8 | (uint32_t)m->intra_chroma_pred_mode << 16;
+                const uint32_t field = m->flags & H264G_MBF_FIELD ? 1u : 0u;
+                if (n >= 2) {  // the tile's last MB is finished
+                    lds_wait(&row.done[0], 0u, n - 1, err);
+                    lds_wait(&row.done[1], 0u, n - 1, err);
                 }
-                intra_res_place(r, &tiles[w]);
-                intra_mb<true>(P, addr, &tiles[w], av, r.res);
+                if (type == H264G_MB_I4x4) intra4_prep((const h264g_mb *)m, av, tile);
+                else if (type == H264G_MB_I8x8) intra8_prep((const h264g_mb *)m, av, tile);
+                intra_res_place(r, tile);
+                if (lane < 4) row.hdr[n & 1u][lane] = lane == 0 ? (uint32_t)addr : lane == 1 ? av.m : lane == 2 ? type | modes | (r.res ? 1u << 31 : 0u) : field;
+                lds_post(&row.ready, ++n);
+            }
+        }
+    }
+}
+// Address of dword i of the two bottom rows of pair (px, py).
+__device__ __forceinline__ GAS uint32_t *mbaff_bottom(const DbkPlanes &d, int px, int py, int i) {
+    const int j = i & 7;
+    GAS uint8_t *const p = i < 8 ? G(d.y) + (uint64_t)(py * 32 + 30 + (j >> 2)) * d.wl + px * 16 + 4 * (j & 3)
+                                 : G(j < 4 ? d.cb : d.cr) + (uint64_t)(py * 16 + 14 + ((j >> 1) & 1)) * d.wc + px * 8 + 4 * (j & 1);
+    return (GAS uint32_t *)p;
+}
+// Luma (c = 0) or chroma (1) of the row's MBs.
+template <int C>
+__device__ __forceinline__ void mbaff_intra_row(const DevPic &P, int w, int y, bool send, GAS uint64_t *out, MbaffIntraShared &sh,
+                                                uint32_t epoch, uint32_t *err) {
+    const int W = P.W, lane = wave_lane();
+    const DbkPlanes d = dbk_planes(P);
+    MbaffIntraRow &row = sh.row[w];
+    uint32_t n = 0;
+    for (int x0 = 0; x0 < W; x0 += WAVE) {
+        const PairMask pm = mbaff_intra_pairs(P, y, x0);
+        for (uint64_t todo = pm.top | pm.bot; todo; todo &= todo - 1) {
+            const int i = (int)__builtin_ctzll(todo), x = x0 + i;
+            if (!send) lds_post(&sh.prog[C][w + 1], (uint32_t)x);
+            if (y > 0) {
+                lds_wait(&sh.prog[C][w], 0u, (uint32_t)min(x + 2, W), err);
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            }
+            for (uint32_t k = (uint32_t)((pm.top >> i) & 1u) + (uint32_t)((pm.bot >> i) & 1u); k; k--) {
+                lds_wait(&row.ready, 0u, n + 1, err);
+                const uint32_t *const hdr = row.hdr[n & 1u];
+                const uint32_t addr = uniform(hdr[0]), m = uniform(hdr[2]), bot = addr & 1u;
+                const bool field = uniform(hdr[3]) != 0u;
+                const Avail av{uniform(hdr[1])};
+                MbGeo g;
+                g.mbx = x;
+                g.bot = (int)bot;
+                g.field = field;
+                g.step = field ? 2 : 1;
+                g.ly = y * 32 + (int)(field ? bot : 16 * bot);
+                g.cy = y * 16 + (int)(field ? bot : 8 * bot);
+                g.mcy = 0;
+                intra_mb<1 << C>(P, g, {(int)(m & 255u), (int)(m >> 8 & 255u), (int)(m >> 16 & 255u)}, &row.tile[n & 1u], av, (m >> 31) != 0u);
                 wave_sync();
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // its samples before the next MB reads them
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                lds_post(&row.done[C], ++n);
             }
-            wave_sync();
-            __hip_atomic_store(&prog[y], (uint32_t)x + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (send && lane < MISTRIP_WORDS / 2) {
+                const uint32_t v = *mbaff_bottom(d, x, y, 8 * C + lane);
+                __hip_atomic_store(&out[(size_t)x * MISTRIP_WORDS + 8 * C + lane], (uint64_t)epoch << 32 | v, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
         }
+        if (!send) lds_post(&sh.prog[C][w + 1], (uint32_t)min(x0 + WAVE, W));
+    }
+}
+// What pair row y, of the band above, hands down.
+__device__ __forceinline__ void mbaff_istrip_reader(const DevPic &P, int y, const GAS uint64_t *sw, MbaffIntraShared &sh, uint32_t epoch,
+                                                    uint32_t *err) {
+    const int W = P.W, lane = wave_lane();
+    const DbkPlanes d = dbk_planes(P);
+    auto post = [&](int x) {
+        lds_post(&sh.prog[0][0], (uint32_t)x);
+        lds_post(&sh.prog[1][0], (uint32_t)x);
+    };
+    for (int x0 = 0; x0 < W; x0 += WAVE) {
+        const PairMask pm = mbaff_intra_pairs(P, y, x0);
+        for (uint64_t todo = pm.top | pm.bot; todo; todo &= todo - 1) {
+            const int x = x0 + (int)__builtin_ctzll(todo);
+            post(x);
+            uint64_t r;
+#pragma unroll 1
+            for (uint32_t it = 0;; ++it) {
+                r = __hip_atomic_load(&sw[(size_t)x * MISTRIP_WORDS + (lane & (MISTRIP_WORDS - 1))], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (__builtin_amdgcn_ballot_w64((uint32_t)(r >> 32) != epoch) == 0) break;
+                if (it >= SPIN_LIMIT) {
+                    report_timeout(err);
+                    return;
+                }
+                if ((it & 255u) == 255u && uniform(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) return;
+                __builtin_amdgcn_s_sleep(1);
+            }
+            if (lane < MISTRIP_WORDS) *mbaff_bottom(d, x, y, lane) = (uint32_t)r;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        }
+        post(min(x0 + WAVE, W));
+    }
+}
+__global__ __launch_bounds__(WAVE *MBAFF_INTRA_WAVES) void k_intra_mbaff(const DevPic *__restrict__ pics, uint32_t n, DevCtl *ctl,
+                                                                         uint32_t *epoch_p, uint32_t *err) {
+    __shared__ MbaffIntraShared sh;
+    __shared__ uint32_t s_ticket;
+    const uint32_t epoch = launch_epoch(epoch_p);
+    const int wave = (int)uniform(threadIdx.x / WAVE), w = wave / 3, part = wave % 3;
+    if ((int)threadIdx.x < MBAFF_ROWS) sh.row[threadIdx.x].ready = sh.row[threadIdx.x].done[0] = sh.row[threadIdx.x].done[1] = 0;
+    const uint32_t t = band_ticket(ctl, &s_ticket, &sh.prog[0][0], 2 * (MBAFF_ROWS + 1));
+    if (t < gridDim.x) {
+        const DevPic &P = pics[t % n];
+        const int b = (int)(t / n), HP = P.H >> 1, y0 = b * MBAFF_ROWS, y1 = min(HP, y0 + MBAFF_ROWS), y = y0 + w;
+        if (P.mbaff && P.n_intra != 0 && y0 < HP) {
+            GAS uint64_t *const strips = G(P.istrip), *const out = strips + (size_t)b * P.W * MISTRIP_WORDS;
+            const bool send = y + 1 == y1 && y1 < HP;
+            if (w < MBAFF_ROWS) {
+                if (y >= y1) {
+                } else if (part == 0) {
+                    mbaff_intra_prep(P, y, sh.row[w], err);
+                } else if (part == 1) {
+                    mbaff_intra_row<0>(P, w, y, send, out, sh, epoch, err);
+                } else {
+                    mbaff_intra_row<1>(P, w, y, send, out, sh, epoch, err);
+                }
+            } else if (b > 0) {
+                mbaff_istrip_reader(P, y0 - 1, strips + (size_t)(b - 1) * P.W * MISTRIP_WORDS, sh, epoch, err);
+            }
+        }
+    }
+    band_retire(ctl, epoch_p, epoch);
 }
 
 // Row-pipelined deblocking: a ticket is one MB row of one picture (queue ordered by
@@ -3843,9 +3982,12 @@ int h264g_launch_intra(const DevPic *pics, const uint32_t *items, uint32_t n, De
     return (int)hipGetLastError();
 }
 
-int h264g_launch_intra_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t *err, void *stream) {
-    if (n_pics == 0) return 0;
-    hipLaunchKernelGGL(k_intra_mbaff, dim3(n_pics), dim3(WAVE * MBAFF_INTRA_WAVES), 0, (hipStream_t)stream, pics, n_pics, err);
+int h264g_launch_intra_mbaff(const DevPic *pics, uint32_t n_pics, uint32_t pair_rows, DevCtl *ctl, uint32_t *epoch, uint32_t *err,
+                             void *stream) {
+    if (n_pics == 0 || pair_rows == 0) return 0;
+    const uint32_t bands = (pair_rows + MBAFF_ROWS - 1) / MBAFF_ROWS;
+    hipLaunchKernelGGL(k_intra_mbaff, dim3(n_pics * bands), dim3(WAVE * MBAFF_INTRA_WAVES), 0, (hipStream_t)stream, pics, n_pics, ctl,
+                       epoch, err);
     return (int)hipGetLastError();
 }
 
