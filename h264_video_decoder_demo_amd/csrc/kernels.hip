@@ -3675,9 +3675,10 @@ __device__ __forceinline__ void bs_pair_of_mbs(const DevPic *pics, const uint32_
 // Validation of a frame picture's syntax records and the per-MB values the other kernels read
 // (DevAux, ICOL), a lane per MB, 64 MBs of a row per wave.  The rules are those of the host's
 // staging (stage_picture in api.cpp), which decides what an error is called: this kernel only
-// names the first MB that breaks one.  Bound: one pass over the records and masks, latency of
-// a few dependent loads (record, masks, neighbours' records); the host's pass took 1.6 ms for
-// a 1920x1088 B picture.
+// names the first MB that breaks one.  Bound: the latency of three dependent rounds of loads
+// (record and neighbours, masks, motion), so each round is issued whole: 11 us for a CIF picture,
+// 15 for 1920x1088, 29 for 3840x2160, where loads at the checks that use them took 17, 23 and 35.
+// The host's pass took 1.6 ms for a 1920x1088 B picture.
 __constant__ uint8_t c_cqp[22] = {29, 30, 31, 32, 32, 33, 34, 34, 35, 35, 36, 36, 37, 37, 37, 38, 38, 38, 39, 39, 39, 39};
 __device__ __forceinline__ uint32_t stage_chroma_qp(int qp, int off) {  // 8.5.8, Table 8-15
     const int q = clip3(0, 51, qp + off);
@@ -3693,22 +3694,66 @@ __device__ __forceinline__ bool stage_mode_ok(int mode, bool left, bool top, boo
 struct StageSums {
     uint32_t inter, intra, lists;
 };
-// One MB; false when it breaks a rule.  ax is complete but for the residual index of an intra MB.
-__device__ __forceinline__ bool stage_mb(const StageIn &S, int x, int y, DevAux &ax, StageSums &sum) {
-    const int W = S.W, a = y * W + x;
+// What an MB's record says beside its motion, and the class, shape and slice of its neighbours A,
+// B, C and D (of the MB itself where there is none): loaded together, ahead of the checks, whose
+// branches would each wait for what they look at.
+struct StageRec {
+    uint32_t w[9];             // mb_type .. ref_idx
+    uint32_t off, sn;
+    uint32_t nw[4], nshape[4], nsn[4];
+    __device__ __forceinline__ uint32_t byte(int k) const { return (w[k >> 2] >> (8 * (k & 3))) & 255u; }
+};
+__device__ __forceinline__ StageRec stage_load(const StageIn &S, int a, const int (&nb)[4]) {
+    StageRec r;
     const GAS h264g_mb *const mbs = G(S.mbs);
-    const GAS h264g_mb &m = mbs[a];
-    const int cls = m.mb_type, cbp = m.cbp, qp = m.qp_y;
-    const bool i16 = cls == H264G_MB_I16x16, t8 = m.flags & H264G_MBF_T8x8;
-    const uint64_t off = m.level_offset;
+    const GAS uint32_t *const p = (const GAS uint32_t *)&mbs[a];
+#pragma unroll
+    for (int k = 0; k < 9; k++) r.w[k] = p[k];
+    r.off = mbs[a].level_offset;
+    r.sn = mbs[a].slice_num;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const GAS h264g_mb &n = mbs[nb[k]];
+        r.nw[k] = n.mb_type;
+        r.nshape[k] = n.part_shape;
+        r.nsn[k] = n.slice_num;
+    }
+    return r;
+}
+static_assert(offsetof(h264g_mb, mb_type) == 0 && offsetof(h264g_mb, flags) == 1 && offsetof(h264g_mb, qp_y) == 2 &&
+              offsetof(h264g_mb, cbp) == 3 && offsetof(h264g_mb, intra16x16_pred_mode) == 4 && offsetof(h264g_mb, intra_chroma_pred_mode) == 5 &&
+              offsetof(h264g_mb, part_shape) == 6 && offsetof(h264g_mb, sub_part_shape) == 8 && offsetof(h264g_mb, intra_pred_modes) == 12 &&
+              offsetof(h264g_mb, ref_idx) == 28 && offsetof(h264g_mb, mv) == 36, "StageRec::w");
+// A neighbour that constrained intra prediction hides (cip_hides).
+__device__ __forceinline__ bool stage_hides(const StageRec &R, int k) {
+    return R.nw[k] == H264G_MB_P_SKIP || ((R.nw[k] == H264G_MB_P || R.nw[k] == H264G_MB_B) && R.nshape[k] != H264G_PART_8x8);
+}
+// One MB; false when it breaks a rule.  ax is complete but for the residual index of an intra MB.
+// there: which neighbours are in the picture.
+__device__ __forceinline__ bool stage_mb(const StageIn &S, const StageRec &R, int a, uint32_t there, DevAux &ax, StageSums &sum) {
+    const GAS h264g_mb &m = G(S.mbs)[a];
+    const int cls = (int)R.byte(0), cbp = (int)R.byte(3), qp = (int)R.byte(2), shape = (int)R.byte(6);
+    const uint32_t flags = R.byte(1);
+    const bool i16 = cls == H264G_MB_I16x16, t8 = flags & H264G_MBF_T8x8;
+    const uint64_t off = R.off;
+    // the masks: DC of an Intra16x16 MB | luma, four for each 8x8 block of cbp | chroma.  Taken
+    // whole (what lies behind the levels is in the picture's block), in pairs.
+    const int lm = cbp & 15, cc = cbp >> 4, nl = 4 * __popc((uint32_t)lm), first = i16 ? 1 : 0;
+    const GAS uint16_t *const lv = (const GAS uint16_t *)G(S.levels) + min(off, S.n_levels);
+    typedef uint32_t __attribute__((aligned(2), may_alias)) u32_a2;
+    uint32_t dcm = lv[0], lw[8], cw[5];
+#pragma unroll
+    for (int k = 0; k < 8; k++) lw[k] = *(const GAS u32_a2 *)(lv + first + 2 * k);
+#pragma unroll
+    for (int k = 0; k < 5; k++) cw[k] = *(const GAS u32_a2 *)(lv + first + nl + 2 * k);
     if (cls > H264G_MB_B || qp > 51 || off > S.n_levels || (cbp >> 4) > 2) return false;
     if (i16 && (cbp & 15) != 0 && (cbp & 15) != 15) return false;
     if (cls == H264G_MB_P_SKIP && cbp) return false;
     if (cls == H264G_MB_I8x8 && !t8) return false;
     if ((cls == H264G_MB_I4x4 || i16) && t8) return false;
-    const uint32_t sub = *(const GAS uint32_t *)m.sub_part_shape;
-    if (cls_inter(cls) && t8 && ((cbp & 15) == 0 || (m.part_shape == H264G_PART_8x8 && sub != 0u))) return false;
-    if (m.flags & H264G_MBF_FIELD) return false;
+    const uint32_t sub = R.w[2];
+    if (cls_inter(cls) && t8 && ((cbp & 15) == 0 || (shape == H264G_PART_8x8 && sub != 0u))) return false;
+    if (flags & H264G_MBF_FIELD) return false;
     if (S.slice_type == H264G_SLICE_I && cls_inter(cls)) return false;
     if (S.slice_type != H264G_SLICE_B && cls == H264G_MB_B) return false;
     if (S.slice_type != H264G_SLICE_P && (cls == H264G_MB_P || cls == H264G_MB_P_SKIP)) return false;
@@ -3731,39 +3776,33 @@ __device__ __forceinline__ bool stage_mb(const StageIn &S, int x, int y, DevAux 
     const bool intra = cls_intra(cls);
     uint32_t kind = (intra ? AUX_INTRA : AUX_INTER) | (t8 ? AUX_T8 : 0u);
     // ---- levels: masks -> non-zero bits
-    const int lm = cbp & 15, cc = cbp >> 4, nl = 4 * __popc((uint32_t)lm);
-    const int nmask = (i16 ? 1 : 0) + nl + (cc >= 1 ? 2 : 0) + (cc == 2 ? 8 : 0);
+    const int nmask = first + nl + (cc >= 1 ? 2 : 0) + (cc == 2 ? 8 : 0);
     if (off + (uint64_t)nmask > S.n_levels) return false;
-    const GAS uint16_t *const lv = (const GAS uint16_t *)G(S.levels) + off;
-    uint32_t nvals = 0, nz4 = 0, nz8 = 0, stray = 0;
-    int i = 0;
-    if (i16) nvals += __popc((uint32_t)lv[i++]);
-    const uint32_t lbits = i16 ? 0xFFFEu : 0xFFFFu;
-    for (int q = 0; q < 4; q++)
-        if ((lm >> q) & 1)
+    uint32_t nvals = i16 ? (uint32_t)__popc(dcm) : 0u, nz4 = 0, nz8 = 0, stray = 0;
+    const uint32_t lbits = i16 ? 0xFFFEFFFEu : 0xFFFFFFFFu;
+    uint32_t left = (uint32_t)lm;
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const uint32_t mk = lv[i++];
-                nvals += __popc(mk);
-                stray |= mk & ~lbits;
-                if (mk && t8) nz8 |= 1u << q;
-                if (mk && !t8) nz4 |= 1u << (4 * q + b);
-            }
-    if (cc >= 1)
+    for (int g = 0; g < 4; g++) {  // the masks of the g-th 8x8 block that has any
+        const bool on = left != 0u;
+        const uint32_t q = on ? (uint32_t)__builtin_ctz(left) : 0u, w0 = on ? lw[2 * g] : 0u, w1 = on ? lw[2 * g + 1] : 0u;
+        left &= left - 1u;
+        nvals += (uint32_t)__popc(w0) + (uint32_t)__popc(w1);
+        stray |= (w0 | w1) & ~lbits;
+        const uint32_t nz = ((w0 & 0xFFFFu) ? 1u : 0u) | ((w0 >> 16) ? 2u : 0u) | ((w1 & 0xFFFFu) ? 4u : 0u) | ((w1 >> 16) ? 8u : 0u);
+        if (t8) nz8 |= (nz ? 1u : 0u) << q;
+        else nz4 |= nz << (4u * q);
+    }
+    if (cc >= 1) {
+        nvals += (uint32_t)__popc(cw[0]);
+        stray |= cw[0] & ~0x000F000Fu;
+    }
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const uint32_t mk = lv[i++];
-            nvals += __popc(mk);
-            stray |= mk & ~0x000Fu;
-        }
-    if (cc == 2)
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const uint32_t mk = lv[i++];
-            nvals += __popc(mk);
-            stray |= mk & ~0xFFFEu;
-        }
-    if (stray & 0xFFFFu) return false;
+    for (int k = 1; k < 5; k++) {
+        const uint32_t w = cc == 2 ? cw[k] : 0u;
+        nvals += (uint32_t)__popc(w);
+        stray |= w & ~0xFFFEFFFEu;
+    }
+    if (stray) return false;
     if (off + (uint64_t)nmask + nvals > S.n_levels) return false;
     if (nmask) kind |= AUX_RESID;
     ax.kind = (uint8_t)kind;
@@ -3773,60 +3812,63 @@ __device__ __forceinline__ bool stage_mb(const StageIn &S, int x, int y, DevAux 
     ax.ires = nvals << AUX_NVALS_SHIFT;
     // ---- intra modes vs neighbour availability
     if (intra) {
-        auto avail = [&](int dx, int dy) -> bool {
-            const int nx = x + dx, ny = y + dy;
-            if (nx < 0 || ny < 0 || nx >= W) return false;
-            const GAS h264g_mb &n = mbs[ny * W + nx];
-            if (n.slice_num != m.slice_num) return false;
-            return !(S.cip && (n.mb_type == H264G_MB_P_SKIP || ((n.mb_type == H264G_MB_P || n.mb_type == H264G_MB_B) &&
-                                                               n.part_shape != H264G_PART_8x8)));
-        };
-        const bool A = avail(-1, 0), B = avail(0, -1), D = avail(-1, -1);
+        auto avail = [&](int k) -> bool { return ((there >> k) & 1u) && R.nsn[k] == R.sn && !(S.cip && stage_hides(R, k)); };
+        const bool A = avail(0), B = avail(1), D = avail(3);
         if (!i16) {
             const int n = cls == H264G_MB_I4x4 ? 4 : 2;
+            auto mode = [&](int blk) -> uint32_t {  // byte blk of the modes
+                const uint32_t w = blk < 8 ? (blk < 4 ? R.w[3] : R.w[4]) : blk < 12 ? R.w[5] : R.w[6];
+                return (w >> (8 * (blk & 3))) & 255u;
+            };
             for (int by = 0; by < n; by++)
                 for (int bx = 0; bx < n; bx++) {
                     const bool left = bx > 0 || A, top = by > 0 || B;
                     const bool tl = bx > 0 ? (by > 0 || B) : (by > 0 ? A : D);
                     const int blk = n == 4 ? 8 * (by >> 1) + 4 * (bx >> 1) + 2 * (by & 1) + (bx & 1) : by * 2 + bx;
-                    if (!stage_mode_ok(m.intra_pred_modes[blk], left, top, tl)) return false;
+                    if (!stage_mode_ok((int)mode(blk), left, top, tl)) return false;
                 }
         } else {
-            const int md = m.intra16x16_pred_mode;
+            const int md = (int)R.byte(4);
             if (md > 3 || (md == 0 && !B) || (md == 1 && !A) || (md == 3 && !(A && B && D))) return false;
         }
-        const int cm = m.intra_chroma_pred_mode;
+        const int cm = (int)R.byte(5);
         if (cm > 3 || (cm == 1 && !A) || (cm == 2 && !B) || (cm == 3 && !(A && B && D))) return false;
         sum.intra += 384 + 2 * ((uint32_t)nmask + nvals) + 16 * 2 + 48;
         return true;
     }
     // ---- inter: reference slots, prediction flags, weight entries
-    const int shape = m.part_shape;
     if (shape > 3) return false;
     if (shape == H264G_PART_8x8 && (sub & 0xFCFCFCFCu)) return false;
-    uint32_t pf = 0;
+    uint32_t pf = 0, e[4], rejected = 0;
+    bool bad = false;
+    int8_t slot[2][4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        const int r0 = m.ref_idx[0][q], r1 = m.ref_idx[1][q];
-        if (r0 < 0 && r1 < 0) return false;
-        if (cls != H264G_MB_B && r1 >= 0) return false;
-        if (r0 < -1 || r0 >= S.nref[0] || r1 < -1 || r1 >= S.nref[1]) return false;
-        if (r0 >= 0) {
-            ax.refid[0][q] = S.ref_slot[0][r0];
-            pf |= 1u << q;
-        }
-        if (r1 >= 0) {
-            ax.refid[1][q] = S.ref_slot[1][r1];
-            pf |= 16u << q;
-        }
-        const uint32_t e = (uint32_t)((r0 + 1) * S.n1 + r1 + 1);
-        if ((S.bad_weight[e >> 5] >> (e & 31u)) & 1u) return false;
-        ax.wp[q] = (uint8_t)e;
+        const int r0 = (int8_t)(R.w[7] >> (8 * q)), r1 = (int8_t)(R.w[8] >> (8 * q));
+        bad |= (r0 < 0 && r1 < 0) || (cls != H264G_MB_B && r1 >= 0) || r0 < -1 || r0 >= S.nref[0] || r1 < -1 || r1 >= S.nref[1];
+        pf |= (r0 >= 0 ? 1u : 0u) << q | (r1 >= 0 ? 16u : 0u) << q;
+        e[q] = (uint32_t)((r0 + 1) * S.n1 + r1 + 1) & 255u;
+        rejected |= S.bad_weight[e[q] >> 5] >> (e[q] & 31u);
+        slot[0][q] = S.ref_slot[0][clip3(0, 31, r0)];
+        slot[1][q] = S.ref_slot[1][clip3(0, 31, r1)];
+    }
+    if (bad || (rejected & 1u)) return false;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        ax.refid[0][q] = (pf >> q) & 1u ? slot[0][q] : (int8_t)-1;
+        ax.refid[1][q] = (pf >> (4 + q)) & 1u ? slot[1][q] : (int8_t)-1;
+        ax.wp[q] = (uint8_t)e[q];
     }
     ax.pf = (uint8_t)pf;
     // ---- algorithmic bytes: per partition and list used (stage_picture)
     const int ps = cls == H264G_MB_P_SKIP ? H264G_PART_16x16 : shape;
     uint32_t bytes = 0, lists = 0;
+    uint32_t mv[2][16];
+#pragma unroll
+    for (int l = 0; l < 2; l++)
+#pragma unroll
+        for (int b = 0; b < 16; b++) mv[l][b] = ((const GAS uint32_t *)m.mv)[16 * l + b];
+#pragma unroll
     for (int b = 0; b < 16; b++) {
         const int bx = b & 3, by = b >> 2, q = (by >> 1) * 2 + (bx >> 1);
         int w, h;
@@ -3842,7 +3884,7 @@ __device__ __forceinline__ bool stage_mb(const StageIn &S, int x, int y, DevAux 
 #pragma unroll
         for (int l = 0; l < 2; l++) {
             if (!((pf >> (4 * l + q)) & 1u)) continue;
-            const int mx = m.mv[l][b][0], my = m.mv[l][b][1];
+            const int mx = (int16_t)mv[l][b], my = (int16_t)(mv[l][b] >> 16);
             bytes += (uint32_t)((4 * w + 5 * ((mx & 3) != 0)) * (4 * h + 5 * ((my & 3) != 0)) +
                                 2 * (2 * w + ((mx & 7) != 0)) * (2 * h + ((my & 7) != 0)) + 5);
             lists++;
@@ -3857,7 +3899,11 @@ __global__ __launch_bounds__(WAVE) void k_stage(StageIn S) {
     const int y = (int)(blockIdx.x / (uint32_t)per), x0 = (int)(blockIdx.x % (uint32_t)per) * WAVE, x = x0 + lane;
     const GAS h264g_mb *const mbs = G(S.mbs);
     const bool in = x < W;
-    const int a = y * W + (in ? x : W - 1);
+    const int xc = in ? x : W - 1, a = y * W + xc;
+    const uint32_t there = (xc > 0 ? 1u : 0u) | (y > 0 ? 2u : 0u) | (y > 0 && xc < W - 1 ? 4u : 0u) | (xc > 0 && y > 0 ? 8u : 0u);
+    const int nb[4] = {(there & 1u) ? a - 1 : a, (there & 2u) ? a - W : a, (there & 4u) ? a - W + 1 : a, (there & 8u) ? a - W - 1 : a};
+    const StageRec R = stage_load(S, a, nb);
+    uint32_t before = G(S.irow)[y];
     DevAux ax;
     {
         uint32_t *const w = (uint32_t *)&ax;
@@ -3865,33 +3911,28 @@ __global__ __launch_bounds__(WAVE) void k_stage(StageIn S) {
         for (int k = 0; k < (int)(sizeof(DevAux) / 4); k++) w[k] = k < 2 ? 0xFFFFFFFFu : 0u;  // refid -1, the rest 0
     }
     StageSums sum{0u, 0u, 0u};
-    const bool ok = !in || stage_mb(S, x, y, ax, sum);
-    const GAS h264g_mb &m = mbs[a];
-    const uint32_t sn = m.slice_num;
-    const bool intra = in && cls_intra(m.mb_type);
+    const bool ok = !in || stage_mb(S, R, a, there, ax, sum);
+    const uint32_t sn = R.sn, cls = R.byte(0);
+    const bool intra = in && cls_intra((int)cls);
     // residual index: the row's intra MBs before this one
-    uint32_t before = G(S.irow)[y];
     for (int c = 0; c < x0; c += WAVE) before += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(cls_intra(mbs[y * W + c + lane].mb_type)));
     const uint64_t im = __builtin_amdgcn_ballot_w64(intra);
     const uint32_t idx = before + __builtin_amdgcn_mbcnt_hi((uint32_t)(im >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)im, 0u));
     if (intra) {
         ax.ires |= idx;
-        uint32_t av = (x > 0 ? 1u : 0u) | (y > 0 ? 2u : 0u) | (y > 0 && x < W - 1 ? 4u : 0u) | (x > 0 && y > 0 ? 8u : 0u), dep = 0;
-        const int nb[4] = {a - 1, a - W, a - W + 1, a - W - 1};
+        uint32_t av = there, dep = 0;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             if (!(av & (1u << k))) continue;
-            const GAS h264g_mb &n = mbs[nb[k]];
-            if (n.slice_num != sn) {
+            if (R.nsn[k] != sn) {
                 av &= ~(1u << k);
                 continue;
             }
-            const int c = n.mb_type;
-            if (S.cip && (c == H264G_MB_P_SKIP || ((c == H264G_MB_P || c == H264G_MB_B) && n.part_shape != H264G_PART_8x8))) av &= ~(1u << k);
-            if (cls_intra(c)) dep |= 1u << k;
+            if (S.cip && stage_hides(R, k)) av &= ~(1u << k);
+            if (cls_intra((int)R.nw[k])) dep |= 1u << k;
         }
-        if (!(m.mb_type == H264G_MB_I8x8 || (m.mb_type == H264G_MB_I4x4 && (m.intra_pred_modes[5] == 3 || m.intra_pred_modes[5] == 7))))
-            dep &= ~4u;
+        const uint32_t m5 = (R.w[4] >> 8) & 255u;  // mode of block 5
+        if (!(cls == H264G_MB_I8x8 || (cls == H264G_MB_I4x4 && (m5 == 3u || m5 == 7u)))) dep &= ~4u;
         G(S.icol)[idx] = (uint32_t)x | av << ICOL_AV_SHIFT | dep << ICOL_DEP_SHIFT | ((ax.kind & AUX_RESID) ? ICOL_RES : 0u);
     }
     if (in) {
