@@ -3961,6 +3961,13 @@ __global__ __launch_bounds__(WAVE) void k_stage(StageIn S) {
     }
 }
 
+// Strengths by themselves, for runs that time the stages apart.
+template <bool MBAFF>
+__global__ __launch_bounds__(WAVE) void k_bs(const DevPic *__restrict__ pics, const uint32_t *__restrict__ chunks) {
+    if (MBAFF) bs_mbaff_mb(pics, chunks, blockIdx.x, gridDim.x);
+    else bs_pair_of_mbs(pics, chunks, blockIdx.x, gridDim.x);
+}
+
 // YUV420P -> BGR24 of one DPB slot (CH264PictureBase::convertYuv420pToBgr24,
 // H264PictureBase.cpp:440-495): one thread per 2x2 luma block (one chroma sample);
 // BT.601 integer coefficients over 1000 with C division (toward zero), clipped.
@@ -4004,8 +4011,12 @@ int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, i
     if (n == 0) return 0;
     const uint32_t n_mb = (what & INTER_MBS) ? n * MB_CHUNK : 0u;
     const uint32_t n_bs = !(what & INTER_BS) ? 0u : mbaff ? n * MB_CHUNK : n * (MB_CHUNK / 2);
-    if (n_mb + n_bs == 0) return 0;
     const dim3 grid(n_mb + n_bs), block(WAVE);
+    if (n_mb == 0) {
+        if (mbaff) hipLaunchKernelGGL((k_bs<true>), grid, block, 0, (hipStream_t)stream, pics, chunks);
+        else hipLaunchKernelGGL((k_bs<false>), grid, block, 0, (hipStream_t)stream, pics, chunks);
+        return (int)hipGetLastError();
+    }
     if (mbaff)  // (scaling matrices are refused in MBAFF frames)
         hipLaunchKernelGGL((k_inter<true, false>), grid, block, 0, (hipStream_t)stream, pics, chunks, n_mb);
     else if (scaled)
