@@ -115,7 +115,7 @@ struct alignas(16) WaveRes {
         struct {
             uint32_t sm[28];          // slot: mask (bits 0..15) | index of its first value << 16
             int16_t vals[7 * WAVE];   // level values in stream order (at most 27 * 16)
-            int32_t dense[4][64];     // levels: the 8x8 blocks in raster order, or [0] = the
+            int32_t dense[4][64];     // the 8x8 blocks dequantised, raster order, or [0] = the
                                       // Intra16x16 DC block in scan order
             int32_t cdc[2][4];        // scan-order levels: chroma DC
             int32_t t8[4][64];        // 8x8 transform: rows after the horizontal pass
@@ -166,18 +166,9 @@ constexpr uint64_t iscan4_table(const uint8_t (&scan)[16]) {
 constexpr uint64_t IZZ4 = iscan4_table(c_zz4);
 constexpr uint64_t IFLD4 = iscan4_table(c_fld4);
 
-// 4x4 transpose over the four lanes of a quad (lane r holds row r in m[0..3], afterwards
-// column r): two exchange stages with DPP quad permutations.
+// The value of the lane's neighbour in its quad, lane ^ 1 / lane ^ 2.
 __device__ __forceinline__ int dpp_xor1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true); }  // [1,0,3,2]
 __device__ __forceinline__ int dpp_xor2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true); }  // [2,3,0,1]
-__device__ __forceinline__ void quad_transpose(int32_t (&m)[4], int r) {
-    const bool odd = r & 1, hi = r & 2;
-    int a = dpp_xor1(odd ? m[0] : m[1]), b = dpp_xor1(odd ? m[2] : m[3]);
-    if (odd) { m[0] = a; m[2] = b; } else { m[1] = a; m[3] = b; }
-    a = dpp_xor2(hi ? m[0] : m[2]);
-    b = dpp_xor2(hi ? m[1] : m[3]);
-    if (hi) { m[0] = a; m[1] = b; } else { m[2] = a; m[3] = b; }
-}
 
 // 4x4 byte transpose over the four lanes of a quad: lane j holds row j of a block of bytes
 // (byte c = column c) and gets column j (byte r = row r).  Two exchange stages, each a DPP
@@ -200,13 +191,14 @@ __device__ __forceinline__ int32_t level_at(uint32_t e, const int16_t *vals, int
 }
 
 // 8.5.12 for row r of a 4x4 block on the quad that holds the block (lane r of the quad):
-// dequantise the row's levels (slot entry e), horizontal pass, transpose, vertical pass;
-// returns column r of the residual in out[0..3] (rows 0..3).  dc_pass: sample (0, 0) is
+// dequantise the row's levels (slot entry e), horizontal pass, vertical pass; returns row
+// quad_row(r) of the residual, four 16-bit values.  dc_pass: sample (0, 0) is
 // `dc` as it stands (Intra16x16 and chroma DC).  field: the levels follow the field scan
 // (field MBs, H264PictureBase.cpp:3419).
+__device__ __forceinline__ int quad_row(int r) { return (0x2130 >> (4 * r)) & 3; }
 template <bool SCALED = false>
-__device__ __forceinline__ void residual4x4_quad(uint32_t se, const int16_t *vals, int qp, bool dc_pass, int dc, int r,
-                                                 bool field, int32_t (&out)[4], const GAS uint16_t *lsm = nullptr) {
+__device__ __forceinline__ uint2 residual4x4_quad(uint32_t se, const int16_t *vals, int qp, bool dc_pass, int dc, int r,
+                                                 bool field, const GAS uint16_t *lsm = nullptr) {
     const int m = qp % 6, e = qp / 6;
     // LevelScale4x4 of row r: with flat lists 16 v0 at (even, even), 16 v1 at (odd, odd),
     // 16 v2 elsewhere; with scaling matrices (SCALED) lsm holds LevelScale4x4(qP % 6, i, j),
@@ -235,10 +227,18 @@ __device__ __forceinline__ void residual4x4_quad(uint32_t se, const int16_t *val
         const int32_t e0 = d[0] + d[2], e1 = d[0] - d[2], e2 = (d[1] >> 1) - d[3], e3 = d[1] + (d[3] >> 1);
         f[0] = e0 + e3; f[1] = e1 + e2; f[2] = e1 - e2; f[3] = e0 - e3;
     }
-    quad_transpose(f, r);
-    const int32_t g0 = f[0] + f[2], g1 = f[0] - f[2], g2 = (f[1] >> 1) - f[3], g3 = f[1] + (f[3] >> 1);
-    out[0] = (g0 + g3 + 32) >> 6; out[1] = (g1 + g2 + 32) >> 6;
-    out[2] = (g1 - g2 + 32) >> 6; out[3] = (g0 - g3 + 32) >> 6;
+    // Vertical pass across the quad, for every column: with f_r lane r's value, lanes 0..3 first
+    // hold f0 + f2, f1 + (f3 >> 1), f0 - f2 - 1, (f1 >> 1) - f3 - 1 (x ^ -1 is -x - 1), then, from
+    // their neighbours', rows 0, 3, 1 and 2 but for constants that join the rounding's 32.  Half the
+    // instructions of a 4x4 transpose and a pass in each lane, and a lane's results lie together.
+    const uint32_t neg1 = (r & 1) ? ~0u : 0u, neg2 = (r & 2) ? ~0u : 0u, add = r == 0 ? 32u : r == 2 ? 34u : 33u;
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t t = ((uint32_t)f[j] ^ neg2) + (uint32_t)(dpp_xor2(f[j]) >> (r & 1));
+        o[j] = (uint32_t)((int32_t)((t ^ neg1) + (uint32_t)dpp_xor1((int)t) + add) >> 6);
+    }
+    return make_uint2(__builtin_amdgcn_perm(o[1], o[0], 0x05040100u), __builtin_amdgcn_perm(o[3], o[2], 0x05040100u));
 }
 
 __device__ __forceinline__ void idct8(int32_t *v, int s) {  // 8.5.13.2, in place, stride s
@@ -252,6 +252,10 @@ __device__ __forceinline__ void idct8(int32_t *v, int s) {  // 8.5.13.2, in plac
 }
 
 // Places the MB's levels in LDS and computes all residual blocks into ws->rl / ws->rc.  Must be called by the whole wave.  Returns false when the MB has no levels.
+// Bound: vector instructions (the kernel's time follows their number).  The vertical pass of a 4x4
+// block across its quad, 8x8 blocks dequantised where a lane has one scale, values two per lane
+// and residuals added in pairs: three 1920x1088 B pictures 58.6 to 56.1 us, the 64-stream pass
+// 24.0 to 23.3 ms.
 // Field MBs of MBAFF frames take the field scans.  lstab: the picture's LevelScale tables
 // when it has scaling matrices (DevPic::ls), else null (flat lists).
 template <bool MBAFF, bool SCALED>
@@ -263,21 +267,23 @@ __device__ __forceinline__ bool build_residual(const h264g_mb *mb, const DevAux 
     const int cbp = mb->cbp;
     const int i16 = mb->mb_type == H264G_MB_I16x16;
     const int t8 = (ax.kind & AUX_T8) ? 1 : 0;
-    const int qp = mb->qp_y;
+    const int qp = (int)__builtin_amdgcn_readfirstlane((uint32_t)mb->qp_y);
     // the MB's luma lists (intra or inter), which serve its chroma blocks too (quirk Q13)
     const bool inter = !(ax.kind & AUX_INTRA);
     const GAS uint16_t *ls4t = SCALED ? lstab + (inter ? LS4_LIST : 0) : nullptr;
     const GAS uint16_t *ls8t = SCALED ? lstab + LS8_AT + (inter ? LS8_LIST : 0) : nullptr;
     const int16_t *lv = levels + mb->level_offset;
     // <= 27 masks of 16 bits, so at most 432 values; the host counted them, so the masks
-    // and the values load together (coalesced, all in flight at once)
-    const int nmask = ax.nmask, total = (int)(ax.ires >> AUX_NVALS_SHIFT);
+    // and the values load together (coalesced, all in flight at once), two values per lane and
+    // only as many rounds as the MB has values for (mostly two of the four)
+    const int nmask = ax.nmask, total = (int)__builtin_amdgcn_readfirstlane(ax.ires >> AUX_NVALS_SHIFT);
     const int mask = lane < nmask ? (uint16_t)lv[lane] : 0;
-    int16_t v[7];
+    typedef uint32_t __attribute__((aligned(2), may_alias)) u32_a2;
+    uint32_t v[4];
 #pragma unroll
-    for (int t = 0; t < 7; t++) {
-        const int k = lane + t * WAVE;
-        v[t] = k < total ? lv[nmask + k] : (int16_t)0;
+    for (int t = 0; t < 4; t++) {
+        const int k = 2 * (lane + t * WAVE);
+        if (2 * t * WAVE < total) v[t] = *(const GAS u32_a2 *)(lv + nmask + min(k, total - 1));
     }
     const int cnt = __popc(mask);
     // exclusive prefix sum of cnt (0..16) over the lanes, bit plane by bit plane (ballot +
@@ -292,46 +298,44 @@ __device__ __forceinline__ bool build_residual(const h264g_mb *mb, const DevAux 
     if (lane < 28) ws->sm[lane] = 0u;
     if (lane < nmask) ws->sm[level_slot(lane, i16, cbp)] = (uint32_t)mask | (uint32_t)pre << 16;
 #pragma unroll
-    for (int t = 0; t < 7; t++)
-        if (lane + t * WAVE < total) ws->vals[lane + t * WAVE] = v[t];
+    for (int t = 0; t < 4; t++)
+        if (2 * t * WAVE < total && lane + t * WAVE < 7 * WAVE / 2) ((uint32_t *)ws->vals)[lane + t * WAVE] = v[t];
     wave_sync();
     // dense levels where a pass reads positions of other rows: the 8x8 blocks, the
     // Intra16x16 DC block (lanes 0..15) and the chroma DC blocks (lanes 56..63)
     if (t8) {  // lane = raster position in the 8x8 blocks, p its scan position
         const int p = field ? c_ifld8[lane] : c_izz8[lane];
+        // 8.5.13.1: dequantised here, where every lane has one position and so one LevelScale8x8:
+        // that of its class among the six of 8-318, by row and column mod 4, or the matrix's
+        const int m = qp % 6, e = qp / 6;
+        int ls;
+        if (SCALED) {
+            ls = ls8t[64 * m + lane];
+        } else {
+            const uint32_t cls = (uint32_t)(0x1513525415133430ull >> (16 * ((lane >> 3) & 3) + 4 * (lane & 3))) & 15u;
+            const uint32_t lo = (uint32_t)c_v8[m][0] | (uint32_t)c_v8[m][1] << 8 | (uint32_t)c_v8[m][2] << 16 | (uint32_t)c_v8[m][3] << 24,
+                           hi = (uint32_t)c_v8[m][4] | (uint32_t)c_v8[m][5] << 8;
+            ls = (int)__builtin_amdgcn_perm(hi, lo, cls | 0x0c0c0c00u) << 4;
+        }
+        // 8-338 / 8-339 as one expression (qP / 6 >= 6 shifts left)
+        const int lsh = e >= 6 ? e - 6 : 0, rsh = e >= 6 ? 0 : 6 - e, rnd = e >= 6 ? 0 : 1 << (5 - e);
 #pragma unroll
-        for (int q = 0; q < 4; q++) ws->dense[q][lane] = level_at(ws->sm[1 + 4 * q + (p >> 4)], ws->vals, p & 15);
+        for (int q = 0; q < 4; q++) {
+            const int v = level_at(ws->sm[1 + 4 * q + (p >> 4)], ws->vals, p & 15);
+            ws->dense[q][lane] = (int32_t)(((uint32_t)(v * ls) << lsh) + (uint32_t)rnd) >> rsh;
+        }
     } else if (i16 && lane < 16) {
         ws->dense[0][lane] = level_at(ws->sm[0], ws->vals, lane);
     }
     if ((cbp >> 4) && lane >= 56) ws->cdc[(lane - 56) >> 2][lane & 3] = level_at(ws->sm[17 + ((lane - 56) >> 2)], ws->vals, lane & 3);
     if (t8 || i16 || (cbp >> 4)) wave_sync();
     if (t8) {
-        // 8.5.13: lanes 0-31 = (8x8 block q, row i): dequantise + horizontal pass ...
+        // 8.5.13: lanes 0-31 = (8x8 block q, row i): horizontal pass ...
         if (lane < 32) {
-            const int q = lane >> 3, i = lane & 7, m = qp % 6, e = qp / 6;
-            const int32_t *src = &ws->dense[q][i * 8];
-            // LevelScale8x8 of row i by column class (j % 4 == 0, j odd, j % 4 == 2): the
-            // six normAdjust8x8 classes of 8-318
-            const int v0 = 16 * c_v8[m][0], v1 = 16 * c_v8[m][1], v2 = 16 * c_v8[m][2], v3 = 16 * c_v8[m][3],
-                      v4 = 16 * c_v8[m][4], v5 = 16 * c_v8[m][5];
-            const int ls_0 = (i & 1) ? v3 : (i & 2) ? v4 : v0;
-            const int ls_1 = (i & 1) ? v1 : (i & 2) ? v5 : v3;
-            const int ls_2 = (i & 1) ? v5 : (i & 2) ? v2 : v4;
-            int lsr[8];  // LevelScale8x8 of row i: the classes above, or the matrix row
-#pragma unroll
-            for (int j = 0; j < 8; j++) lsr[j] = (j & 1) ? ls_1 : (j & 2) ? ls_2 : ls_0;
-            if (SCALED) {
-                const uint4 t = *(const GAS uint4 *)(ls8t + 64 * m + 8 * i);
-                const uint32_t w[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-                for (int j = 0; j < 8; j++) lsr[j] = (int)((w[j >> 1] >> (16 * (j & 1))) & 0xFFFFu);
-            }
-            // 8-338 / 8-339 as one expression (qP / 6 >= 6 shifts left)
-            const int lsh = e >= 6 ? e - 6 : 0, rsh = e >= 6 ? 0 : 6 - e, rnd = e >= 6 ? 0 : 1 << (5 - e);
+            const int q = lane >> 3, i = lane & 7;
             int32_t d[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) d[j] = (int32_t)(((uint32_t)(src[j] * lsr[j]) << lsh) + (uint32_t)rnd) >> rsh;
+            for (int j = 0; j < 8; j++) d[j] = ws->dense[q][i * 8 + j];
             idct8(d, 1);
 #pragma unroll
             for (int j = 0; j < 8; j++) ws->t8[q][i * 8 + j] = d[j];
@@ -365,11 +369,8 @@ __device__ __forceinline__ bool build_residual(const h264g_mb *mb, const DevAux 
             const int sc = SCALED ? ls4t[16 * (qp % 6)] : ls4(qp % 6, 0, 0);
             dc = qp >= 36 ? (f * sc) << (qp / 6 - 6) : (f * sc + (1 << (5 - qp / 6))) >> (6 - qp / 6);
         }
-        int32_t o[4];
-        residual4x4_quad<SCALED>(ws->sm[1 + b], ws->vals, qp, i16, dc, r, field, o, ls4t + 16 * (qp % 6));
-        const int x0 = blk_x(b), y0 = blk_y(b);
-#pragma unroll
-        for (int i = 0; i < 4; i++) ws->rl[(y0 + i) * 16 + x0 + r] = (int16_t)o[i];
+        const uint2 o = residual4x4_quad<SCALED>(ws->sm[1 + b], ws->vals, qp, i16, dc, r, field, ls4t + 16 * (qp % 6));
+        *(uint2 *)&ws->rl[(blk_y(b) + quad_row(r)) * 16 + blk_x(b)] = o;
     } else {  // no luma levels
         ((uint2 *)ws->rl)[lane] = make_uint2(0u, 0u);
     }
@@ -382,11 +383,8 @@ __device__ __forceinline__ bool build_residual(const h264g_mb *mb, const DevAux 
         const int32_t e00 = dcv[0] + dcv[2], e01 = dcv[1] + dcv[3], e10 = dcv[0] - dcv[2], e11 = dcv[1] - dcv[3];
         const int32_t f = b == 0 ? e00 + e01 : b == 1 ? e00 - e01 : b == 2 ? e10 + e11 : e10 - e11;
         const int dc = ((f * (SCALED ? ls4t[16 * (qpc % 6)] : ls4(qpc % 6, 0, 0))) << (qpc / 6)) >> 5;
-        int32_t o[4];
-        residual4x4_quad<SCALED>(ws->sm[19 + 4 * c + b], ws->vals, qpc, true, dc, r, field, o, ls4t + 16 * (qpc % 6));
-        const int x0 = (b & 1) * 4, y0 = (b >> 1) * 4;
-#pragma unroll
-        for (int i = 0; i < 4; i++) ws->rc[c][(y0 + i) * 8 + x0 + r] = (int16_t)o[i];
+        const uint2 o = residual4x4_quad<SCALED>(ws->sm[19 + 4 * c + b], ws->vals, qpc, true, dc, r, field, ls4t + 16 * (qpc % 6));
+        *(uint2 *)&ws->rc[c][((b >> 1) * 4 + quad_row(r)) * 8 + (b & 1) * 4] = o;
     }
     if (t8) {
         wave_sync();
@@ -652,6 +650,13 @@ __device__ __forceinline__ int wp_apply(const WpTerms &t, uint32_t pair) {
     return clip1((v >> t.sh) + t.off);
 }
 
+// Clip1 of the sums of two samples and two residual values, 16 bits each (the sums saturate).
+__device__ __forceinline__ uint32_t add_clip1(uint32_t samples, uint32_t res) {
+    typedef short short2_t __attribute__((ext_vector_type(2)));
+    const short2_t v = __builtin_elementwise_add_sat(__builtin_bit_cast(short2_t, samples), __builtin_bit_cast(short2_t, res));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_elementwise_max(v, (short2_t){0, 0}), (short2_t){255, 255}));
+}
+
 // Inter MB (or I_PCM copy): prediction + residual, written to the destination slot.
 // SCALED: the launch holds pictures with scaling matrices (their residual code reads the
 // LevelScale tables; the other pictures' the flat one).
@@ -697,9 +702,9 @@ __device__ void inter_mb(const DevPic &P, int addr, WaveRes *ws) {
                            wp_apply(t, __builtin_amdgcn_perm(p1, p0, 0x0c070c03u)));
         }
         if (res) {
-            const int16_t *rl = &ws->rl[(by * 4 + r) * 16 + bx * 4];
-            packed = pack4(clip1((int)(packed & 255) + rl[0]), clip1((int)((packed >> 8) & 255) + rl[1]),
-                           clip1((int)((packed >> 16) & 255) + rl[2]), clip1((int)(packed >> 24) + rl[3]));
+            const uint2 rl = *(const uint2 *)&ws->rl[(by * 4 + r) * 16 + bx * 4];
+            packed = __builtin_amdgcn_perm(add_clip1(__builtin_amdgcn_perm(0u, packed, 0x0c030c02u), rl.y),
+                                           add_clip1(__builtin_amdgcn_perm(0u, packed, 0x0c010c00u), rl.x), 0x06040200u);
         }
         *(uint32_t *)&dy[(uint64_t)(g.ly + (by * 4 + r) * g.step) * wl + mbx * 16 + bx * 4] = packed;
     }
@@ -736,11 +741,9 @@ __device__ void inter_mb(const DevPic &P, int addr, WaveRes *ws) {
             v0 = wp_apply(t, (uint32_t)c00 | (uint32_t)c10 << 16);
             v1 = wp_apply(t, (uint32_t)c01 | (uint32_t)c11 << 16);
         }
-        if (res) {
-            v0 = clip1(v0 + ws->rc[c][(by * 2 + r) * 8 + bx * 2]);
-            v1 = clip1(v1 + ws->rc[c][(by * 2 + r) * 8 + bx * 2 + 1]);
-        }
-        *(uint16_t *)&plane[(uint64_t)(g.cy + (by * 2 + r) * g.step) * wc + xC] = (uint16_t)(v0 | (v1 << 8));
+        uint32_t v = (uint32_t)v0 | (uint32_t)v1 << 16;
+        if (res) v = add_clip1(v, *(const uint32_t *)&ws->rc[c][(by * 2 + r) * 8 + bx * 2]);
+        *(uint16_t *)&plane[(uint64_t)(g.cy + (by * 2 + r) * g.step) * wc + xC] = (uint16_t)(v | v >> 8);
     }
     (void)H;
 }
