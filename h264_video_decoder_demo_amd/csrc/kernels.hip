@@ -3819,10 +3819,10 @@ __device__ __forceinline__ bool stage_mb(const StageIn &S, const StageRec &R, in
         const bool A = avail(0), B = avail(1), D = avail(3);
         if (!i16) {
             const int n = cls == H264G_MB_I4x4 ? 4 : 2;
-            auto mode = [&](int blk) -> uint32_t {  // byte blk of the modes
-                const uint32_t w = blk < 8 ? (blk < 4 ? R.w[3] : R.w[4]) : blk < 12 ? R.w[5] : R.w[6];
-                return (w >> (8 * (blk & 3))) & 255u;
-            };
+            // byte blk of the modes (shifted out of two registers: words picked from R by a
+            // condition would make it an array in scratch memory)
+            const uint64_t lo = (uint64_t)R.w[4] << 32 | R.w[3], hi = (uint64_t)R.w[6] << 32 | R.w[5];
+            auto mode = [&](int blk) -> uint32_t { return (uint32_t)((blk < 8 ? lo : hi) >> (8 * (blk & 7))) & 255u; };
             for (int by = 0; by < n; by++)
                 for (int bx = 0; bx < n; bx++) {
                     const bool left = bx > 0 || A, top = by > 0 || B;
