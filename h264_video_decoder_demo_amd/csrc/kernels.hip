@@ -6,11 +6,13 @@
 // H264PictureBase.cpp:707):
 //   inter   -- fully parallel over inter (and I_PCM) MBs: fractional-sample MC from
 //              the device-resident DPB + weighted prediction + residual.
-//   intra   -- persistent wavefront over intra MBs: each wave takes the next ticket of a
-//              queue ordered by t = x + 2y, waits on its A/B/C/D neighbours' progress
-//              words, reconstructs, publishes its own word.
-//   deblock -- the same wavefront scheme over all MBs with the raster-order edge filter.
-// The queues hold MBs of any number of pictures (batching across streams).
+//              The same launch derives the boundary strengths of deblocking.
+//   intra   -- bands of MB rows, a wave per row and plane type, walking its intra MBs
+//              behind the row above.
+//   deblock -- bands likewise, over all MBs, with the raster-order edge filter.
+// Before them a staging kernel, a lane per MB, checks a picture's records and expands them.
+// The per-MB wavefront and row schedules (queues ordered by t = x + 2y, progress words in
+// device memory) are alternatives.  A launch holds the pictures of any number of streams.
 #include <hip/hip_runtime.h>
 
 #include <mutex>

@@ -53,7 +53,7 @@ def test_sparse_and_dense_intra_rows_match_oracle(permille):
 
 @pytest.mark.gpu
 def test_mbaff_and_frame_pictures_in_one_batch():
-    """MBAFF frames of 1 to 20 pair rows (one workgroup walks them in rounds of 16) beside
+    """MBAFF frames of 1 to 20 pair rows (bands of 4 on workgroups of their own) beside
     frame pictures and a picture without deblocking in the same batches."""
     with Engine(device=0) as eng:
         gens = [Generator(3, width_mbs=w, height_mbs=h, n_frames=3, seed=0xBA9F00 + h, intra_in_inter_permille=200,
