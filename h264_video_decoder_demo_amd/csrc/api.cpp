@@ -172,6 +172,7 @@ struct h264g_ctx {
     hipEvent_t front[2] = {nullptr, nullptr};  // end of a lane's last pre-deblocking stages
     bool front_on_ds[2] = {false, false};      // those ran on its deblocking stream
     bool joined[2] = {true, true};             // the deblocking stream is ordered after all of the lane's work
+    bool used_since[4] = {false, false, false, false};  // any_stream(i) got launches since it was last seen idle
     DbkRec hist[2][kDbkHist];
     int hist_next[2] = {0, 0};
     int split_mbs = 16384;         // 0: one lane
@@ -197,13 +198,16 @@ struct h264g_ctx {
     int intra_schedule = H264G_INTRA_BANDS;
     int intra_waves = 8;           // rows per band (waves per workgroup) of the intra band schedule
     int dbk_waves = 8;             // configured MB rows per band of the deblocking band schedule (run: dbk_rows)
-    // One staging call at a time uses a slot: a stream and pinned memory for its small uploads
-    // and its result.  Slots are made when all are in use (one with the context) and kept.
+    // One staging call at a time uses a slot: a stream, pinned memory for its small uploads and
+    // its result, and the event it waits for.  Slots are made when all are in use (one with the
+    // context) and kept.
     struct StageSlot {
         hipStream_t s = nullptr;
         uint8_t *pin = nullptr;
+        hipEvent_t done = nullptr;
     };
     std::vector<StageSlot> slots;  // free ones
+    uint32_t stage_turn = 0;       // staging_stream's turn among the idle streams
     std::vector<hipEvent_t> ev;    // 6 events per profiled run: inter | intra | bS | end (lane), deblock | end
     size_t ev_used = 0;            // events recorded since the last h264g_stage_times
     std::mutex mu;
@@ -234,11 +238,13 @@ hipError_t sync_lanes(h264g_ctx *c) {
     for (int i = 0; i < 4; i++) {
         const hipError_t e = hipStreamSynchronize(any_stream(c, i));
         if (r == hipSuccess) r = e;
+        c->used_since[i] = false;
     }
     return r;
 }
 // A lane and its deblocking stream.
 hipError_t sync_lane(h264g_ctx *c, int lane) {
+    c->used_since[lane] = c->used_since[2 + lane] = false;
     const hipError_t e = hipStreamSynchronize(lane_stream(c, lane));
     const hipError_t e2 = hipStreamSynchronize(c->dstream[lane]);
     return e != hipSuccess ? e : e2;
@@ -526,6 +532,7 @@ constexpr size_t kSlotResult = kSlotPin - 256;  // where the result comes back
 
 bool make_slot(h264g_ctx::StageSlot &sl) {
     return hipStreamCreateWithFlags(&sl.s, hipStreamNonBlocking) == hipSuccess &&
+           hipEventCreateWithFlags(&sl.done, hipEventDisableTiming) == hipSuccess &&
            hipHostMalloc((void **)&sl.pin, kSlotPin, hipHostMallocDefault) == hipSuccess;
 }
 void free_slot(h264g_ctx::StageSlot &sl) {
@@ -533,8 +540,24 @@ void free_slot(h264g_ctx::StageSlot &sl) {
         (void)hipStreamSynchronize(sl.s);
         (void)hipStreamDestroy(sl.s);
     }
+    if (sl.done) (void)hipEventDestroy(sl.done);
     if (sl.pin) (void)hipHostFree(sl.pin);
     sl = h264g_ctx::StageSlot();
+}
+
+// The stream a staging call's copies and kernel go to.  More streams than the process has
+// hardware queues (4) share them, and what shares a queue runs in the order it was enqueued: on
+// a stream of its own alone a picture staged beside a batch of lane 0 waited for the batch to
+// end (7.3 of its 7.9 ms).  So while the context's streams have work, staging goes to one of
+// them that has none (50 us beside that batch), in turns; else to the slot's.  Caller holds mu.
+hipStream_t staging_stream(h264g_ctx *c, const h264g_ctx::StageSlot &sl) {
+    hipStream_t idle[4];
+    uint32_t n = 0;
+    for (int i = 0; i < 4; i++) {
+        if (c->used_since[i]) c->used_since[i] = hipStreamQuery(any_stream(c, i)) == hipErrorNotReady;
+        if (!c->used_since[i]) idle[n++] = any_stream(c, i);
+    }
+    return n == 0 || n == 4 ? sl.s : idle[c->stage_turn++ % n];
 }
 
 // Staging of a frame picture on the device: records and levels go up as they are, k_stage
@@ -584,6 +607,7 @@ int stage_on_device(h264g_ctx *ctx, const Stream &st, const h264g_pic_desc &d, c
     if (tail > kSlotResult) return 1;
     char *base = (char *)fixed;
     h264g_ctx::StageSlot sl;
+    hipStream_t ss = nullptr;
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
         if (!fixed) {
@@ -600,11 +624,20 @@ int stage_on_device(h264g_ctx *ctx, const Stream &st, const h264g_pic_desc &d, c
         } else if (fixed) {
             return 1;  // a fixed block is staged without allocating
         }
+        ss = staging_stream(ctx, sl);
     }
-    if (!sl.s && !make_slot(sl)) {
-        free_slot(sl);
-        return h264g_set_error(H264G_E_DEVICE, "staging stream");
+    if (!sl.s) {
+        if (!make_slot(sl)) {
+            free_slot(sl);
+            return h264g_set_error(H264G_E_DEVICE, "staging stream");
+        }
+        if (!ss) ss = sl.s;
     }
+    const auto wait = [&]() -> hipError_t {  // until what this call enqueued is done
+        if (ss == sl.s) return hipStreamSynchronize(ss);
+        const hipError_t e = hipEventRecord(sl.done, ss);
+        return e == hipSuccess ? hipEventSynchronize(sl.done) : e;
+    };
     fill_devpic(st, d, base, l, n_intra, !lsv.empty(), pic);
     DevPic &P = pic->hpic;
     P.irow = pic->d_items;
@@ -642,29 +675,29 @@ int stage_on_device(h264g_ctx *ctx, const Stream &st, const h264g_pic_desc &d, c
             std::memcpy(sl.pin, mbs, n_mbs * sizeof(h264g_mb));
             if (n_levels) std::memcpy(sl.pin + l.o_lv, levels, n_levels * sizeof(int16_t));
             put_tail(sl.pin + l.o_wt);
-            HIPCHK(hipMemcpyAsync(base, sl.pin, l.o_wt + tail, hipMemcpyHostToDevice, sl.s));
+            HIPCHK(hipMemcpyAsync(base, sl.pin, l.o_wt + tail, hipMemcpyHostToDevice, ss));
         } else {
-            HIPCHK(hipMemcpyAsync(pic->d_mbs, mbs, n_mbs * sizeof(h264g_mb), hipMemcpyHostToDevice, sl.s));
-            if (n_levels) HIPCHK(hipMemcpyAsync(pic->d_levels, levels, n_levels * sizeof(int16_t), hipMemcpyHostToDevice, sl.s));
+            HIPCHK(hipMemcpyAsync(pic->d_mbs, mbs, n_mbs * sizeof(h264g_mb), hipMemcpyHostToDevice, ss));
+            if (n_levels) HIPCHK(hipMemcpyAsync(pic->d_levels, levels, n_levels * sizeof(int16_t), hipMemcpyHostToDevice, ss));
             put_tail(sl.pin);
-            HIPCHK(hipMemcpyAsync(base + l.o_wt, sl.pin, tail, hipMemcpyHostToDevice, sl.s));
+            HIPCHK(hipMemcpyAsync(base + l.o_wt, sl.pin, tail, hipMemcpyHostToDevice, ss));
         }
-        if (int e = h264g_launch_stage(&in, sl.s)) return h264g_set_error(H264G_E_DEVICE, "staging launch: %s", hipGetErrorString((hipError_t)e));
-        HIPCHK(hipMemcpyAsync(sl.pin + kSlotResult, in.res, sizeof(StageResult), hipMemcpyDeviceToHost, sl.s));
-        HIPCHK(hipStreamSynchronize(sl.s));
+        if (int e = h264g_launch_stage(&in, ss)) return h264g_set_error(H264G_E_DEVICE, "staging launch: %s", hipGetErrorString((hipError_t)e));
+        HIPCHK(hipMemcpyAsync(sl.pin + kSlotResult, in.res, sizeof(StageResult), hipMemcpyDeviceToHost, ss));
+        HIPCHK(wait());
         std::memcpy(&res, sl.pin + kSlotResult, sizeof(res));
         if (res.err_mb != ~0u) return 1;
         P.dbk_stop = res.dbk_stop;
         P.multi_slice = res.multi_slice ? 1 : 0;
         if (res.dbk_stop != n_mbs || res.multi_slice) {  // k_stage's findings into the descriptor
             std::memcpy(sl.pin, &P, sizeof(P));
-            HIPCHK(hipMemcpyAsync(pic->d_pic, sl.pin, sizeof(P), hipMemcpyHostToDevice, sl.s));
-            HIPCHK(hipStreamSynchronize(sl.s));
+            HIPCHK(hipMemcpyAsync(pic->d_pic, sl.pin, sizeof(P), hipMemcpyHostToDevice, ss));
+            HIPCHK(wait());
         }
         return 0;
     };
     const int rc = run();
-    if (rc) (void)hipStreamSynchronize(sl.s);  // nothing reads the caller's arrays or the block any more
+    if (rc) (void)hipStreamSynchronize(ss);  // nothing reads the caller's arrays or the block any more
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
         ctx->slots.push_back(sl);
@@ -1148,6 +1181,7 @@ bool conflicts(const DbkRec &r, const std::vector<SlotUse> &uses) {
 //    picture crosses between streams (the two crossings took 13 of 88 us per CIF P picture).
 int enqueue(h264g_ctx *c, const StageSet &q, int lane, const std::vector<SlotUse> &uses, bool events = true) {
     hipStream_t s = lane_stream(c, lane), ds = c->dstream[lane];
+    c->used_since[lane] = c->used_since[2 + lane] = true;
     // one-lane contexts (lane_split_mbs < 0) keep the strictly sequential shape
     const bool split = c->dbk_schedule == H264G_DEBLOCK_BANDS && !q.dbk_off && c->split_mbs > 0;
     hipEvent_t *ev = events ? profile_events(c) : nullptr;
