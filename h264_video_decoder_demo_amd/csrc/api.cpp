@@ -260,22 +260,34 @@ int check_stream(const h264g_ctx *c, uint32_t id, uint64_t gen) {
 }
 
 // ------------------------------------------------------------ reading back
-// Device memory to host memory that is not pinned, after what is enqueued on st: through the
-// halves of the pinned bounce buffer, the copy of one part out of it beside the transfer of the
-// next.  A copy straight to such memory costs 70 us for a few bytes and runs at 18 GB/s; this
-// way a CIF picture takes 20 us instead of 105, a 1920x1088 picture 165 instead of 190, one of
-// 3840x2160 520 instead of 735 (transfers at 55 GB/s beside copies at 30).  A part costs 18 us
-// beside its bytes, so parts are large.
+// Device memory to the caller's, after what is enqueued on st.  Ordinary memory is reached
+// through the halves of the pinned bounce buffer, where a result of more than one half has the
+// copy of one part out of it beside the transfer of the next.  A transfer straight to such memory
+// costs 70 us for a few bytes and runs at 18 GB/s; this way a CIF picture takes 20 us instead of
+// 105, a 1920x1088 picture 165 instead of 190, one of 3840x2160 520 instead of 735 (transfers at
+// 55 GB/s, copies at 30).  A part costs 18 us beside its bytes, so parts are large.
 constexpr size_t kBounceHalf = 4 << 20;
+// Pinned memory (the caller's own) is written by the transfer itself, from this size per plane on:
+// 1920x1088 in 83 us instead of 152, 3840x2160 246 instead of 504; but a transfer more costs 7 us,
+// so that CIF planes take 30 that way instead of 16.
+constexpr size_t kDirectPlane = 128 << 10;
 struct Plane {
     uint8_t *to;
     size_t n;
 };
-// Planes that lie one after the other from `from`.  Caller holds ctx->mu.
-int read_planes(h264g_ctx *c, hipStream_t st, const uint8_t *from, std::initializer_list<Plane> planes) {
+// Whether the plane is written by the transfer itself (mean: bytes per plane of the call).
+bool direct_plane(const Plane &p, size_t mean) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p.to) != hipSuccess) {  // memory that the runtime does not know
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered && (mean >= kDirectPlane || a.type != hipMemoryTypeHost);
+}
+// Planes p .. end - 1, which lie one after the other from `from`, through the bounce buffer.
+int bounce_planes(h264g_ctx *c, hipStream_t st, const uint8_t *from, const Plane *p, const Plane *end) {
     size_t total = 0;
-    for (const Plane &p : planes) total += p.n;
-    const Plane *p = planes.begin();
+    for (const Plane *q = p; q != end; q++) total += q->n;
     size_t done = 0;  // bytes of *p that are there
     auto part = [&](size_t k) { return std::min(kBounceHalf, total - k * kBounceHalf); };
     auto fetch = [&](size_t k) -> hipError_t {
@@ -300,6 +312,31 @@ int read_planes(h264g_ctx *c, hipStream_t st, const uint8_t *from, std::initiali
         }
         if (k + 2 < parts) HIPCHK(fetch(k + 2));
     }
+    return H264G_OK;
+}
+// Planes that lie one after the other from `from`.  Caller holds ctx->mu.
+int read_planes(h264g_ctx *c, hipStream_t st, const uint8_t *from, std::initializer_list<Plane> planes) {
+    size_t mean = 0;
+    for (const Plane &p : planes) mean += p.n / planes.size();
+    const Plane *const end = planes.end(), *first = planes.begin();  // first: of those to go through the buffer
+    bool direct = false;
+    size_t n = 0;  // bytes of planes first .. p - 1
+    for (const Plane *p = first; p != end; p++) {
+        if (!direct_plane(*p, mean)) {
+            n += p->n;
+            continue;
+        }
+        if (n)
+            if (int rc = bounce_planes(c, st, from, first, p)) return rc;
+        from += n;
+        HIPCHK(hipMemcpyAsync(p->to, from, p->n, hipMemcpyDeviceToHost, st));
+        from += p->n;
+        first = p + 1;
+        n = 0;
+        direct = true;
+    }
+    if (n) return bounce_planes(c, st, from, first, end);  // (waits for all that is on st)
+    if (direct) HIPCHK(hipStreamSynchronize(st));
     return H264G_OK;
 }
 
