@@ -20,6 +20,7 @@
 #include "h264g.h"
 #include "h264g_dev.h"
 #include "h264g_internal.h"
+#include "readback.h"
 
 namespace {
 
@@ -271,73 +272,40 @@ constexpr size_t kBounceHalf = 4 << 20;
 // 1920x1088 in 83 us instead of 152, 3840x2160 246 instead of 504; but a transfer more costs 7 us,
 // so that CIF planes take 30 that way instead of 16.
 constexpr size_t kDirectPlane = 128 << 10;
-struct Plane {
-    uint8_t *to;
-    size_t n;
-};
-// Whether the plane is written by the transfer itself (mean: bytes per plane of the call).
-bool direct_plane(const Plane &p, size_t mean) {
-    hipPointerAttribute_t a;
-    if (hipPointerGetAttributes(&a, p.to) != hipSuccess) {  // memory that the runtime does not know
-        (void)hipGetLastError();
-        return false;
-    }
-    return a.type != hipMemoryTypeUnregistered && (mean >= kDirectPlane || a.type != hipMemoryTypeHost);
-}
-// Planes p .. end - 1, which lie one after the other from `from`, through the bounce buffer.
-int bounce_planes(h264g_ctx *c, hipStream_t st, const uint8_t *from, const Plane *p, const Plane *end) {
-    size_t total = 0;
-    for (const Plane *q = p; q != end; q++) total += q->n;
-    size_t done = 0;  // bytes of *p that are there
-    auto part = [&](size_t k) { return std::min(kBounceHalf, total - k * kBounceHalf); };
-    auto fetch = [&](size_t k) -> hipError_t {
-        const hipError_t e = hipMemcpyAsync(c->bounce + (k & 1) * kBounceHalf, from + k * kBounceHalf, part(k), hipMemcpyDeviceToHost, st);
-        return e == hipSuccess && total > kBounceHalf ? hipEventRecord(c->bounced[k & 1], st) : e;
-    };
-    const size_t parts = (total + kBounceHalf - 1) / kBounceHalf;
-    for (size_t k = 0; k < parts && k < 2; k++) HIPCHK(fetch(k));
-    for (size_t k = 0; k < parts; k++) {
-        HIPCHK(parts > 1 ? hipEventSynchronize(c->bounced[k & 1]) : hipStreamSynchronize(st));
-        const uint8_t *src = c->bounce + (k & 1) * kBounceHalf;
-        for (size_t left = part(k); left;) {
-            const size_t n = std::min(left, p->n - done);
-            std::memcpy(p->to + done, src, n);
-            src += n;
-            left -= n;
-            done += n;
-            if (done == p->n) {
-                p++;
-                done = 0;
-            }
+// What read_planes reads with: transfers from `from` on stream st.
+struct SlotIo {
+    h264g_ctx *c;
+    hipStream_t st;
+    const uint8_t *from;
+    bool direct(const Plane &p, size_t mean) {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, p.to) != hipSuccess) {  // memory that the runtime does not know
+            (void)hipGetLastError();
+            return false;
         }
-        if (k + 2 < parts) HIPCHK(fetch(k + 2));
+        return a.type != hipMemoryTypeUnregistered && (mean >= kDirectPlane || a.type != hipMemoryTypeHost);
     }
-    return H264G_OK;
-}
+    int fetch(uint8_t *to, size_t at, size_t n) {
+        HIPCHK(hipMemcpyAsync(to, from + at, n, hipMemcpyDeviceToHost, st));
+        return H264G_OK;
+    }
+    int mark(int half) {
+        HIPCHK(hipEventRecord(c->bounced[half], st));
+        return H264G_OK;
+    }
+    int wait(int half) {
+        HIPCHK(hipEventSynchronize(c->bounced[half]));
+        return H264G_OK;
+    }
+    int wait_all() {
+        HIPCHK(hipStreamSynchronize(st));
+        return H264G_OK;
+    }
+};
 // Planes that lie one after the other from `from`.  Caller holds ctx->mu.
 int read_planes(h264g_ctx *c, hipStream_t st, const uint8_t *from, std::initializer_list<Plane> planes) {
-    size_t mean = 0;
-    for (const Plane &p : planes) mean += p.n / planes.size();
-    const Plane *const end = planes.end(), *first = planes.begin();  // first: of those to go through the buffer
-    bool direct = false;
-    size_t n = 0;  // bytes of planes first .. p - 1
-    for (const Plane *p = first; p != end; p++) {
-        if (!direct_plane(*p, mean)) {
-            n += p->n;
-            continue;
-        }
-        if (n)
-            if (int rc = bounce_planes(c, st, from, first, p)) return rc;
-        from += n;
-        HIPCHK(hipMemcpyAsync(p->to, from, p->n, hipMemcpyDeviceToHost, st));
-        from += p->n;
-        first = p + 1;
-        n = 0;
-        direct = true;
-    }
-    if (n) return bounce_planes(c, st, from, first, end);  // (waits for all that is on st)
-    if (direct) HIPCHK(hipStreamSynchronize(st));
-    return H264G_OK;
+    SlotIo io{c, st, from};
+    return read_planes(io, c->bounce, kBounceHalf, planes.begin(), planes.end());
 }
 
 bool init_err(h264g_ctx *c) {
