@@ -1377,21 +1377,15 @@ int32_t h264g_stream_open(h264g_ctx *c, const h264g_stream_desc *d, uint32_t *id
     s.lane = c->split_mbs > 0 && s.W * s.H >= c->split_mbs ? 1 : 0;
     // DPB slots, and the progress sets: per-MB progress words, per-row progress words,
     // the strips between row bands (deblocking: 256 B per MB column and band; intra: 64 B)
+    // for bands of the heights that they are run with.  All of it counts in the budget.
     auto al = [](uint64_t v) { return (v + 255) & ~(uint64_t)255; };
     auto bands_of = [&](int rows) { return (uint64_t)((s.H + rows - 1) / rows); };
-    auto set_layout = [&](int drows, int irows) {  // with strips for bands of these heights
-        s.o_rowprog = al((uint64_t)s.W * s.H * 4);
-        s.o_gstrip = al(s.o_rowprog + (uint64_t)s.H * 8);
-        s.o_istrip = s.o_gstrip + bands_of(drows) * s.W * 256;
-        return al(s.o_istrip + bands_of(irows) * s.W * 64);
-    };
-    // The budget is charged for the strips of bands of the configured heights, whatever heights
-    // the bands are run with, and for a word per MB pair of MBAFF streams, so that admission
-    // does not depend on the schedule.
-    const uint64_t charged_set = al(set_layout(c->dbk_waves, c->intra_waves) + (s.mbaff ? (uint64_t)s.W * s.H / 2 * 4 : 0));
-    s.set_bytes = set_layout(dbk_rows(c), intra_rows(c));
+    s.o_rowprog = al((uint64_t)s.W * s.H * 4);
+    s.o_gstrip = al(s.o_rowprog + (uint64_t)s.H * 8);
+    s.o_istrip = s.o_gstrip + bands_of(dbk_rows(c)) * s.W * 256;
+    s.set_bytes = al(s.o_istrip + bands_of(intra_rows(c)) * s.W * 64);
     const size_t dpb_bytes = s.slot_bytes * d->dpb_slots, prog_bytes = s.set_bytes * H264G_MAX_STREAM_PICS;
-    const uint64_t need = dpb_bytes + charged_set * H264G_MAX_STREAM_PICS;
+    const uint64_t need = dpb_bytes + prog_bytes;
     if (c->budget && c->used + need > c->budget)
         return h264g_set_error(H264G_E_BUDGET, "DPB budget: %llu + %llu > %llu", (unsigned long long)c->used,
                                (unsigned long long)need, (unsigned long long)c->budget);

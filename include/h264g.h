@@ -166,7 +166,10 @@ typedef struct h264g_mb {
 /* ---------------------------------------------------------- descriptors */
 typedef struct h264g_config {
     int32_t  device;              /* HIP device ordinal                               */
-    uint64_t dpb_budget_bytes;    /* HBM budget for all streams' DPB slots (0 = none) */
+    uint64_t dpb_budget_bytes;    /* HBM budget for all streams' DPB slots and progress
+                                     sets (words and strips for the band heights that
+                                     are run), as requested from the block pool, which
+                                     rounds a block up (0 = none)                     */
     int32_t  max_batch_pictures;  /* pictures per batched launch (0 = default 4096)   */
     int32_t  profile;             /* 1 = record per-stage HIP events                  */
     int32_t  waves;               /* persistent waves per wavefront launch (0 = auto) */
