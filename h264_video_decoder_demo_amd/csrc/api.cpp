@@ -380,12 +380,14 @@ void pool_put(h264g_ctx *c, void *p, size_t n) {
 // reference aliases the preceding slice-header member: luma_weight_lX[-1] is
 // luma_weight_lX_flag (the last one parsed) and luma_offset_lX[-1] is
 // luma_weight_lX[31] (H264SliceHeader.h:78-80).  L1-only luma uses that (w0, o0).
-int derive_weight(const h264g_pic_desc &d, int r0, int r1, DevWeight &w) {
+// Returns whether the reference takes the pair: explicit bi-prediction whose weights sum to more
+// than it allows is refused.
+bool derive_weight(const h264g_pic_desc &d, int r0, int r1, DevWeight &w) {
     std::memset(&w, 0, sizeof(w));
     int pf0 = r0 >= 0, pf1 = r1 >= 0;
     if (d.slice_type == H264G_SLICE_P) w.mode = d.weighted_pred_flag == 1;
     else if (d.slice_type == H264G_SLICE_B) w.mode = d.weighted_bipred_idc == 1 || (d.weighted_bipred_idc == 2 && pf0 && pf1);
-    if (!w.mode) return 0;
+    if (!w.mode) return true;
     if (d.slice_type == H264G_SLICE_B && d.weighted_bipred_idc == 2) {
         int poc0 = d.ref_poc[0][r0], poc1 = d.ref_poc[1][r1];
         int ww0 = 32, ww1 = 32;
@@ -398,7 +400,7 @@ int derive_weight(const h264g_pic_desc &d, int r0, int r1, DevWeight &w) {
             if (!((dsf >> 2) < -64 || (dsf >> 2) > 128)) { ww0 = 64 - (dsf >> 2); ww1 = dsf >> 2; }
         }
         for (int c = 0; c < 3; c++) { w.logWD[c] = 5; w.w0[c] = (int16_t)ww0; w.w1[c] = (int16_t)ww1; }
-        return 0;
+        return true;
     }
     w.logWD[0] = (int16_t)d.luma_log2_weight_denom;
     w.logWD[1] = w.logWD[2] = (int16_t)d.chroma_log2_weight_denom;
@@ -416,9 +418,9 @@ int derive_weight(const h264g_pic_desc &d, int r0, int r1, DevWeight &w) {
         auto bad = [](int s, int lw) { return !(-128 <= s && s <= (lw == 7 ? 127 : 128)); };
         if (bad(w.w0[0] + w.w1[0], w.logWD[0]) || bad(w.w0[1] + w.w1[1], w.logWD[1]) ||
             !(-128 <= w.w0[2] + w.w1[2] && w.w0[1] + w.w1[2] <= (w.logWD[2] == 7 ? 127 : 128)))
-            return h264g_set_error(H264G_E_SYNTAX, "explicit bi-prediction weight sum out of range");
+            return false;
     }
-    return 0;
+    return true;
 }
 
 // Mask index -> level slot, the order residual() parses the blocks (H264MacroBlock.cpp:1592-1856).
@@ -588,7 +590,7 @@ int stage_on_device(h264g_ctx *ctx, const Stream &st, const h264g_pic_desc &d, c
     for (int r0 = -1; r0 < n0; r0++)
         for (int r1 = -1; r1 < n1; r1++) {
             const size_t e = (size_t)(r0 + 1) * (n1 + 1) + (size_t)(r1 + 1);
-            if (e && derive_weight(d, r0, r1, wt[e])) in.bad_weight[e >> 5] |= 1u << (e & 31);
+            if (e && !derive_weight(d, r0, r1, wt[e])) in.bad_weight[e >> 5] |= 1u << (e & 31);
         }
     // ---- intra MBs before each row, slice of the first MB that has one
     std::vector<uint32_t> irow(H + 1);
@@ -949,8 +951,8 @@ int stage_picture(h264g_ctx *ctx, Stream &st, const h264g_pic_desc &d, const h26
             auto it = wmap.find(key);
             if (it == wmap.end()) {
                 DevWeight w;
-                int rc = derive_weight(d, wr0, wr1, w);
-                if (rc) return rc;
+                if (!derive_weight(d, wr0, wr1, w))
+                    return h264g_set_error(H264G_E_SYNTAX, "explicit bi-prediction weight sum out of range");
                 it = wmap.emplace(key, (int)wt.size()).first;
                 wt.push_back(w);
                 if (wt.size() > 255) return h264g_set_error(H264G_E_ARG, "too many weight entries");
