@@ -150,19 +150,28 @@ struct DevErr {
 };
 #define DEVERR_TIMEOUT  0x1u
 
+#define MB_CHUNK 64u
+// Runs of MBs (see h264g_launch_inter) that one launch takes: a grid holds fewer than 2^32 threads,
+// 64 of them to a block, and a run takes blocks_of_run blocks: one for each of its MBs, and for the
+// boundary strengths one for each two, or each of an MBAFF frame's.
+constexpr uint32_t blocks_of_run(bool mbs, bool bs, bool mbaff) {
+    return (mbs ? MB_CHUNK : 0u) + (bs ? (mbaff ? MB_CHUNK : MB_CHUNK / 2) : 0u);
+}
+constexpr uint32_t runs_per_launch(bool mbs, bool bs, bool mbaff) { return (0xFFFFFFFFu / 64u) / blocks_of_run(mbs, bs, mbaff); }
+
 extern "C" {
 // Kernel launchers (kernels.hip); all enqueue on `stream` and return a hipError_t.
 // Validates a frame picture's records and derives their DevAux and ICOL entries.
 int h264g_launch_stage(const StageIn *in, void *stream);
 // Launches over MBs take them in runs of MB_CHUNK of one picture: chunks[0 .. n) (picture index
 // << 20 | first MB), or null with n runs of picture 0.
-#define MB_CHUNK 64u
 // mbaff: every picture of the launch is an MBAFF frame (else none is).
 // scaled: some picture of the launch has scaling matrices (DevPic::ls).
 // what: INTER_MBS, the inter stage; INTER_BS, the boundary strengths of pictures that are
 // deblocked; or both in one launch.
 #define INTER_MBS 1
 #define INTER_BS  2
+// (more runs than a grid has room for take several launches, see runs_per_launch)
 int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, int what, void *stream);
 // `epoch` points at the device word shared by all wavefront launches of a context
 // (initially 1; each launch's last wave advances it).

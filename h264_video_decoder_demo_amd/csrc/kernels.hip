@@ -4013,22 +4013,26 @@ int h264g_launch_stage(const StageIn *in, void *stream) {
 }
 
 int h264g_launch_inter(const DevPic *pics, const uint32_t *chunks, uint32_t n, int mbaff, int scaled, int what, void *stream) {
-    if (n == 0) return 0;
-    const uint32_t n_mb = (what & INTER_MBS) ? n * MB_CHUNK : 0u;
-    const uint32_t n_bs = !(what & INTER_BS) ? 0u : mbaff ? n * MB_CHUNK : n * (MB_CHUNK / 2);
-    const dim3 grid(n_mb + n_bs), block(WAVE);
-    if (n_mb == 0) {
-        if (mbaff) hipLaunchKernelGGL((k_bs<true>), grid, block, 0, (hipStream_t)stream, pics, chunks);
-        else hipLaunchKernelGGL((k_bs<false>), grid, block, 0, (hipStream_t)stream, pics, chunks);
-        return (int)hipGetLastError();
+    const uint32_t most = runs_per_launch(what & INTER_MBS, what & INTER_BS, mbaff);
+    if (!chunks && n > most) return (int)hipErrorInvalidValue;  // (one picture never has as many)
+    for (uint32_t at = 0; at < n; at += most) {
+        const uint32_t runs = n - at < most ? n - at : most;
+        const uint32_t n_mb = (what & INTER_MBS) ? runs * MB_CHUNK : 0u;
+        const uint32_t *const list = chunks ? chunks + at : nullptr;
+        const dim3 grid(runs * blocks_of_run(what & INTER_MBS, what & INTER_BS, mbaff)), block(WAVE);
+        if (n_mb == 0 && mbaff)
+            hipLaunchKernelGGL((k_bs<true>), grid, block, 0, (hipStream_t)stream, pics, list);
+        else if (n_mb == 0)
+            hipLaunchKernelGGL((k_bs<false>), grid, block, 0, (hipStream_t)stream, pics, list);
+        else if (mbaff)  // (scaling matrices are refused in MBAFF frames)
+            hipLaunchKernelGGL((k_inter<true, false>), grid, block, 0, (hipStream_t)stream, pics, list, n_mb);
+        else if (scaled)
+            hipLaunchKernelGGL((k_inter<false, true>), grid, block, 0, (hipStream_t)stream, pics, list, n_mb);
+        else
+            hipLaunchKernelGGL((k_inter<false, false>), grid, block, 0, (hipStream_t)stream, pics, list, n_mb);
+        if (const hipError_t e = hipGetLastError()) return (int)e;
     }
-    if (mbaff)  // (scaling matrices are refused in MBAFF frames)
-        hipLaunchKernelGGL((k_inter<true, false>), grid, block, 0, (hipStream_t)stream, pics, chunks, n_mb);
-    else if (scaled)
-        hipLaunchKernelGGL((k_inter<false, true>), grid, block, 0, (hipStream_t)stream, pics, chunks, n_mb);
-    else
-        hipLaunchKernelGGL((k_inter<false, false>), grid, block, 0, (hipStream_t)stream, pics, chunks, n_mb);
-    return (int)hipGetLastError();
+    return 0;
 }
 
 int h264g_launch_intra(const DevPic *pics, const uint32_t *items, uint32_t n, DevCtl *ctl, uint32_t *epoch, uint32_t *err,
