@@ -1,10 +1,11 @@
 """Band-height autotuner for the two sequential stages.
 
-Intra prediction and deblocking run as bands of MB rows, one workgroup per band (one
-row per wave for intra, two for deblocking).  The band height sets the waves per
-workgroup and so the waves per CU, and trades dependency-chain steps inside a band
-against band crossings through device memory; the best heights depend on the device
-and on the mix of picture sizes that share a launch.  `autotune` measures candidate
+Intra prediction and deblocking run as bands of MB rows, a workgroup per band for luma
+and one for chroma, with a wave per luma row.  The band height, at most 4 rows, sets the
+waves per workgroup and trades hand-overs through LDS inside a band against band
+crossings through device memory; the best heights depend on the device and on the mix of
+picture sizes that share a launch.  Candidates above 4 rows run as 4 and share one
+measurement.  `autotune` measures candidate
 heights on the caller's own streams -- their pictures (all, or the first n_frames),
 staged once and batched by runs of independent frames (engine.independent_runs) -- and caches the
 winner per device (architecture, name, CU count, clock), library build, engine
@@ -20,9 +21,9 @@ import json
 import os
 import time
 
-DEBLOCK_ROWS = (4, 6, 8, 10, 12, 16)
+DEBLOCK_ROWS = (2, 3, 4, 6, 8, 10, 12, 16)
 _clock = time.perf_counter
-INTRA_ROWS = (4, 6, 8)
+INTRA_ROWS = (2, 3, 4, 6, 8)
 
 
 def cache_path() -> str:
@@ -94,8 +95,15 @@ def autotune(gens, n_frames: int = 0, reps: int = 2, deblock_rows=DEBLOCK_ROWS, 
             sid = eng.open_stream(g.width_mbs, g.height_mbs, g.dpb_slots)
             rows.append([eng.begin_raw(sid, *g.picture_raw(i)) for i in range(n)])
 
+        took = {}  # by the heights that are run
+
         def measure(d: int, i: int) -> float:
-            eng.set_bands(d, i)
+            ran = eng.set_bands(d, i) or (d, i)
+            if ran not in took:
+                took[ran] = time_passes()
+            return took[ran]
+
+        def time_passes() -> float:
             batches = [eng.batch_create([r[f] for f in run for r in rows]) for run in independent_runs(rows)]
             try:
                 for b in batches:  # first pass untimed

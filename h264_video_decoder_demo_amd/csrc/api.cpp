@@ -61,7 +61,7 @@ struct Stream {
     uint8_t *prog = nullptr;
     uint64_t set_bytes = 0, o_rowprog = 0, o_gstrip = 0, o_istrip = 0;
     bool mbaff = false;            // MBAFF frames (pairs of field / frame MBs)
-    int strip_dbk_rows = 0, strip_intra_rows = 0;  // strips sized for bands of at least these many rows
+    int strip_dbk_rows = 0, strip_intra_rows = 0;  // the configured heights when it was opened
     uint64_t bytes = 0;
     int lane = 0;                  // HIP stream (lane) of the context that runs its pictures
     uint64_t gen = 0;              // open count of the context when this stream was opened:
@@ -1428,11 +1428,19 @@ int32_t h264g_set_bands(h264g_ctx *c, int32_t deblock_rows, int32_t intra_rows) 
     for (uint32_t k = 0; k < c->streams.size(); k++) {
         const Stream &s = c->streams[k];
         if (s.open && (d < s.strip_dbk_rows || i < s.strip_intra_rows))
-            return h264g_set_error(H264G_E_STATE, "stream %u has strips for bands of at least %d / %d rows", k,
+            return h264g_set_error(H264G_E_STATE, "stream %u was opened for bands of at least %d / %d rows", k,
                                    s.strip_dbk_rows, s.strip_intra_rows);
     }
     c->dbk_waves = d;
     c->intra_waves = i;
+    return H264G_OK;
+}
+
+int32_t h264g_band_rows(h264g_ctx *c, int32_t *deblock_rows, int32_t *intra_rows_out) {
+    if (!c || !deblock_rows || !intra_rows_out) return h264g_set_error(H264G_E_ARG, "NULL argument");
+    std::lock_guard<std::mutex> lk(c->mu);
+    *deblock_rows = dbk_rows(c);
+    *intra_rows_out = intra_rows(c);
     return H264G_OK;
 }
 

@@ -7,7 +7,7 @@ itself runs in the gfx950 kernels of the library.
 from __future__ import annotations
 
 import ctypes
-from ctypes import byref, c_float, c_uint32, c_uint64, c_void_p
+from ctypes import byref, c_float, c_int32, c_uint32, c_uint64, c_void_p
 from dataclasses import dataclass
 
 import numpy as np
@@ -243,8 +243,15 @@ class Engine:
 
     def set_bands(self, deblock_rows: int = 0, intra_rows: int = 0):
         """MB rows per band of the band schedules from now on (0 keeps one); batches
-        created before must be created again."""
+        created before must be created again.  Returns the heights bands are then run with."""
         check(lib().h264g_set_bands(self._h, deblock_rows, intra_rows))
+        return self.band_rows()
+
+    def band_rows(self):
+        """(deblocking, intra) MB rows that bands are run with: the configured ones, at most 4."""
+        d, i = c_int32(), c_int32()
+        check(lib().h264g_band_rows(self._h, byref(d), byref(i)))
+        return d.value, i.value
 
     # ---- pictures
     def begin(self, sid: int, desc: PicDesc, mbs: np.ndarray, levels: np.ndarray) -> StagedPicture:
