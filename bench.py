@@ -291,9 +291,9 @@ def main():
     ap.add_argument("--no-graphs", action="store_true", help="no effect: batch stages are launched directly")
     ap.add_argument("--deblock", choices=["bands", "mb_wavefront", "mb_rows"], default="bands",
                     help="deblocking schedule")
-    ap.add_argument("--deblock-waves", type=int, default=0, help="MB rows per band of the bands schedule (0 = 8)")
+    ap.add_argument("--deblock-waves", type=int, default=0, help="MB rows per band of the bands schedule, run with at most 4")
     ap.add_argument("--intra", choices=["bands", "mb_wavefront"], default="bands", help="intra schedule")
-    ap.add_argument("--intra-waves", type=int, default=0, help="MB rows per band of the bands intra schedule (0 = 8)")
+    ap.add_argument("--intra-waves", type=int, default=0, help="MB rows per band of the bands intra schedule, run with at most 4")
     ap.add_argument("--no-autotune", action="store_true",
                     help="keep the default band heights instead of autotuning them on the workload's first pictures")
     ap.add_argument("--serve-seconds", type=float, default=3.0,
@@ -351,6 +351,7 @@ def main():
     eng = Engine(device=0, profile=False, waves=args.waves, graphs=not args.no_graphs, deblock_schedule=schedule,
                  deblock_waves=args.deblock_waves, intra_schedule={"bands": 0, "mb_wavefront": 1}[args.intra],
                  intra_waves=args.intra_waves, lane_split_mbs=-1 if args.one_lane else 0)
+    rows_run = eng.band_rows()
     sids, slots, pics = [], {}, []
     alg = [0, 0, 0, 0]
     for g in gens:
@@ -583,10 +584,10 @@ def main():
                    "streams": len(gens), "frames_per_stream": nframes, "pictures_per_step": len(gens) * nframes,
                    "batches_per_step": n_batches,
                    "mpix_per_step": round(mpix_step, 3)},
-        "graphs": not args.no_graphs,
+        "graphs": False,  # batch stages are launched directly
         "deblock_schedule": args.deblock,
         "intra_schedule": args.intra,
-        "band_rows": {"deblock": args.deblock_waves or 8, "intra": args.intra_waves or 8,
+        "band_rows": {"deblock": rows_run[0], "intra": rows_run[1],
                       "autotune": ({"ms_per_sample": tune["ms"], "seconds": round(tune["seconds"], 1),
                                     "cached": tune["cached"]} if tune and not tune["cached"] else
                                    ({"cached": True} if tune else None))},
