@@ -1,11 +1,12 @@
 // api.cpp -- host side of libh264g: the C ABI of include/h264g.h.
 //
 // Staging a picture (h264g_picture_begin) validates the host parser's syntax
-// records, derives the per-MB values the kernels need (DPB slots of the
+// records and derives the per-MB values the kernels need (DPB slots of the
 // reference indices, resolved weighted-prediction entries, non-zero masks for
-// the boundary strength, chroma / deblocking QPs) and builds the three device
-// work queues: inter MBs, intra MBs and all MBs, the latter two ordered by the
-// wavefront time t = x + 2y so that every dependency of a queue entry precedes it.
+// the boundary strength, chroma / deblocking QPs) and the intra MBs of each row: a frame
+// picture's in a kernel (stage_on_device), an MBAFF frame's, a refused picture's and one whose
+// schedules walk lists of MBs on the host, which builds those lists, ordered by the wavefront
+// time t = x + 2y so that every dependency of an entry precedes it.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -127,8 +128,8 @@ struct h264g_pic {
     DevPic hpic;                   // host copy (batches re-pack it)
     std::vector<uint32_t> intra_t, all_t;  // host copies of the t-ordered queues (MB addresses), for
                                            // the schedules that walk them
-    bool mbaff = false;            // an MBAFF frame: one workgroup walks its MB pairs (the band
-                                   // schedules take frame MBs only)
+    bool mbaff = false;            // an MBAFF frame: its bands are rows of MB pairs, whatever the
+                                   // schedules of frame pictures
     uint64_t alg[3] = {0, 0, 0};
 };
 

@@ -3,8 +3,8 @@
 #include <stdint.h>
 #include "h264g.h"
 
-// Per-MB values the host derives once while staging a picture (picture_begin):
-// everything the kernels would otherwise recompute per sample.
+// Per-MB values derived once while a picture is staged (picture_begin; by k_stage or the
+// host): everything the kernels would otherwise recompute per sample.
 struct DevAux {
     int8_t   refid[2][4];     // reference picture per list and 8x8 quadrant as a DPB slot,
                               // -1 = none: the MC source when the list is used, and (frame

@@ -275,7 +275,7 @@ __device__ __forceinline__ bool build_residual(const h264g_mb *mb, const DevAux 
     const GAS uint16_t *ls4t = SCALED ? lstab + (inter ? LS4_LIST : 0) : nullptr;
     const GAS uint16_t *ls8t = SCALED ? lstab + LS8_AT + (inter ? LS8_LIST : 0) : nullptr;
     const int16_t *lv = levels + mb->level_offset;
-    // <= 27 masks of 16 bits, so at most 432 values; the host counted them, so the masks
+    // <= 27 masks of 16 bits, so at most 432 values; staging counted them, so the masks
     // and the values load together (coalesced, all in flight at once), two values per lane and
     // only as many rounds as the MB has values for (mostly two of the four)
     const int nmask = ax.nmask, total = (int)__builtin_amdgcn_readfirstlane(ax.ires >> AUX_NVALS_SHIFT);

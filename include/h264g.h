@@ -292,7 +292,8 @@ int32_t h264g_stream_close(h264g_ctx *ctx, uint32_t stream_id);
  * autotuner; 0 keeps a height.  A stream's strips between bands are sized when it is
  * opened, so heights below those that the context had when any open stream was opened
  * fail with H264G_E_STATE, and a batch created before a call that changes one fails in
- * h264g_batch_run (H264G_E_STATE) until it is created again.  No counterpart in the reference (it has no GPU schedules). */
+ * h264g_batch_run (H264G_E_STATE) until it is created again.  No counterpart in the
+ * reference (it has no GPU schedules). */
 int32_t h264g_set_bands(h264g_ctx *ctx, int32_t deblock_rows, int32_t intra_rows);
 /* The heights that bands are run with now: those of the configuration or of
  * h264g_set_bands, at most 4 of either.  No counterpart in the reference. */
@@ -376,7 +377,8 @@ int32_t h264g_set_profile(h264g_ctx *ctx, int32_t on);
 int32_t h264g_sync(h264g_ctx *ctx);
 
 /* Copy a decoded DPB slot to host planes (stride = width).  Call before the
- * output callback fires, as do_callback does (H264VideoDecoder.cpp:383-435). */
+ * output callback fires, as do_callback does (H264VideoDecoder.cpp:383-435).  Planes
+ * in pinned memory (hipHostMalloc) are written without a copy in between. */
 int32_t h264g_slot_readback(h264g_ctx *ctx, uint32_t stream_id, int32_t slot,
                             uint8_t *y, uint8_t *cb, uint8_t *cr);
 /* Convert a decoded DPB slot to BGR24 on the device and copy it to host memory:
